@@ -199,27 +199,100 @@ __device__ __forceinline__ void block_merge(float& m, float& s, float* slots) {
     m = M;
 }
 
+// A row whose 16-byte window is not the row itself (D % 8 != 0, or a base
+// that is not 16-byte aligned): the aligned 16-byte vectors that cover it.
+// Element e of the row is at window position e + shift (shift < 8), so only
+// vector 0 and the last one hold elements of other rows.  Those share a
+// 16-byte granule with the row's own, so reading them never reaches another
+// page; they are masked to -inf after the load and never stored.  x and y
+// at the same offset from a 16-byte boundary (the caller checks) have the
+// same shift in every row, so a vector is stored where it was loaded.
+struct RowWindow {
+    int shift;   // elements of the window before the row
+    int nv;      // vectors of the window
+    int64_t end;  // shift + D
+    __device__ __forceinline__ RowWindow(const half_t* row, int64_t D)
+        : shift(static_cast<int>((reinterpret_cast<uintptr_t>(row) & 15) >> 1)),
+          nv(static_cast<int>((shift + D + 7) >> 3)),
+          end(shift + D) {}
+    // elements [lo, hi) of vector v belong to the row
+    __device__ __forceinline__ int lo(int v) const { return v == 0 ? shift : 0; }
+    __device__ __forceinline__ int hi(int v) const {
+        const int64_t left = end - static_cast<int64_t>(v) * 8;
+        return left < 8 ? static_cast<int>(left) : 8;
+    }
+    __device__ __forceinline__ bool partial(int v) const { return lo(v) != 0 || hi(v) != 8; }
+    __device__ __forceinline__ void mask(int v, h8& a) const {
+        const int l = lo(v), h = hi(v);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (k < l || k >= h) a[k] = -__builtin_huge_valf16();
+    }
+    // vector v of the row's window to p (16-byte aligned).  A vector that
+    // the row begins in is stored as a 2-, a 4- and an 8-byte piece up to the
+    // granule's end, one that it ends in as an 8-, a 4- and a 2-byte piece
+    // from its start; a row inside one granule element by element.
+    __device__ __forceinline__ void store(int v, half_t* p, h8 a) const {
+        const int l = lo(v), h = hi(v);
+        if (l == 0 && h == 8) {
+            st8_out<MI_WT_SM>(p, a);
+            return;
+        }
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        const u32x4 w = __builtin_bit_cast(u32x4, a);
+        auto* p2 = reinterpret_cast<uint16_t*>(p);
+        auto* p4 = reinterpret_cast<uint32_t*>(p);
+        if (h == 8) {  // elements l .. 7
+            if (l & 1)
+                p2[l] = static_cast<uint16_t>((l < 4 ? (l < 2 ? w[0] : w[1]) : (l < 6 ? w[2] : w[3])) >> 16);
+            const int d = (l + 1) >> 1;  // first whole dword
+            if (d & 1) p4[d] = d == 1 ? w[1] : w[3];
+            if (d <= 2) *reinterpret_cast<u32x2*>(p + 4) = u32x2{w[2], w[3]};
+            if (d == 0) *reinterpret_cast<u32x2*>(p) = u32x2{w[0], w[1]};
+        } else if (l == 0) {  // elements 0 .. h - 1
+            if (h & 4) *reinterpret_cast<u32x2*>(p) = u32x2{w[0], w[1]};
+            if (h & 2) p4[(h & 4) >> 1] = h & 4 ? w[2] : w[0];
+            if (h & 1)
+                p2[h - 1] = static_cast<uint16_t>(h & 4 ? (h & 2 ? w[3] : w[2]) : (h & 2 ? w[1] : w[0]));
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (k >= l && k < h) p[k] = a[k];
+        }
+    }
+};
+
 // Register-resident rows (16-byte vectors, D <= G * VPT * 8): G lanes per
 // row -- G <= 64: 256 / G rows per workgroup and DPP-only reductions;
-// G = 256 or 1024: one row per workgroup and one LDS exchange per
+// G = 128, 256 or 1024: one row per workgroup and one LDS exchange per
 // reduction -- with VPT vectors per lane.  x is read once: a packed fp16
 // lane maximum, the row maximum, one exp per element (kept in registers when
 // VPT <= 4, recomputed at the write otherwise), the row sum, then the scaled
 // write.  Lanes past the row hold -inf, whose exp is 0.  No lane returns
 // early, so every group reduction sees all of its lanes.
-template <int G, int VPT>
-__global__ __launch_bounds__(G > 256 ? G : 256) void softmax_reg_kernel(const half_t* x,
+// RAGGED: rows walked through their aligned windows (RowWindow), bound by HBM
+// like the aligned rows but for the two partial granules of each row.  Against
+// the 2-byte kernel that such rows took before (one element per lane, the row
+// read twice): [57344, 511] 137 -> 24.7 us (aligned 512: 20.6), [17108, 1203]
+// 90 -> 16.7, [28672, 2047] 173 -> 44.2, [14336, 1001] 79 -> 13.4.  Plain
+// instead of streaming stores here: 16.7 -> 19.4 us at 1203; the partial
+// vectors element by element: 16.8 -> 17.7.
+template <int G, int VPT, bool RAGGED>
+__global__ __launch_bounds__(G > 64 ? G : 256) void softmax_reg_kernel(const half_t* x,
                                                                         half_t* y, int64_t N,
                                                                         int64_t D) {
-    constexpr int kThreads = G > 256 ? G : 256;
+    constexpr int kThreads = G > 64 ? G : 256;
     constexpr int kRows = kThreads / G;
     constexpr bool kKeepExp = VPT <= 4;
     __shared__ float smax[kThreads / kWave], ssum[kThreads / kWave];
     const int gl = threadIdx.x & (G - 1);
     const int64_t row = static_cast<int64_t>(blockIdx.x) * kRows + threadIdx.x / G;
     const bool live = row < N;
-    const int64_t nv = D >> 3;
-    const half_t* xr = x + row * D;
+    const RowWindow win(x + row * D, D);  // RAGGED
+    const int64_t nv = RAGGED ? win.nv : D >> 3;
+    const int64_t off = row * D - (RAGGED ? win.shift : 0);
+    const half_t* xr = x + off;
     h8 a[VPT];
     // vector j of this lane: a uniform base per j (xr + j * G * 8) plus the
     // lane's 32-bit byte offset (with the forced recompute below, 8-vector
@@ -229,8 +302,15 @@ __global__ __launch_bounds__(G > 256 ? G : 256) void softmax_reg_kernel(const ha
     for (int j = 0; j < VPT; ++j) {
         const int64_t v = gl + j * G;
         const char* base = reinterpret_cast<const char*>(xr + static_cast<int64_t>(j) * G * 8);
-        a[j] = live && v < nv ? ld8_stream(reinterpret_cast<const half_t*>(base + lo))
+                a[j] = live && v < nv ? ld8_stream(reinterpret_cast<const half_t*>(base + lo))
                               : h8(-__builtin_huge_valf16());
+    }
+    if constexpr (RAGGED) {
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            const int v = gl + j * G;
+            if (v < nv && win.partial(v)) win.mask(v, a[j]);
+        }
     }
     h2 m2 = h2(-__builtin_huge_valf16());
 #pragma unroll
@@ -264,7 +344,7 @@ __global__ __launch_bounds__(G > 256 ? G : 256) void softmax_reg_kernel(const ha
     // live instead of the 4 * VPT registers of fp16 data.
     float mw = m;
     if constexpr (!kKeepExp) asm volatile("" : "+v"(mw));
-    half_t* yr = y + row * D;
+    half_t* yr = y + off;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int64_t v = gl + j * G;
@@ -276,56 +356,78 @@ __global__ __launch_bounds__(G > 256 ? G : 256) void softmax_reg_kernel(const ha
                     kKeepExp ? e[kKeepExp ? j : 0][k] : exp_shifted((float)a[j][k], mw * kLog2e);
                 o[k] = to_half(t * inv);
             }
-            st8_out<MI_WT_SM>(
-                reinterpret_cast<half_t*>(
-                    reinterpret_cast<char*>(yr + static_cast<int64_t>(j) * G * 8) + lo),
-                o);
+            half_t* p = reinterpret_cast<half_t*>(
+                reinterpret_cast<char*>(yr + static_cast<int64_t>(j) * G * 8) + lo);
+            if constexpr (RAGGED)
+                win.store(static_cast<int>(v), p, o);
+            else
+                st8_out<MI_WT_SM>(p, o);
         }
     }
 }
 
 // Launch shape for softmax_reg_kernel: the fewest lanes per row (8, 16, 32,
-// 64, then 256 or 1024 as whole workgroups) that hold the row in at most
-// kRegVpt vectors each, else 1024 lanes with up to 8.  Returns false when
-// the row needs more than 1024 x 8 vectors.
-#ifndef MI_SOFTMAX_REG_VPT
-#define MI_SOFTMAX_REG_VPT 4
-#endif
-constexpr int kRegVpt = MI_SOFTMAX_REG_VPT;
+// 64, then 128, 256 or 1024 as whole workgroups) that hold the row in at most
+// kRegVpt vectors each, else 1024 lanes with up to 8.  128 lanes stop at
+// kPairMax vectors, where 256 lanes would leave 3/8 of their slots idle:
+// [20000, 2100] (263 vectors) 41.9 -> 31.1 us, but [20000, 3000] (375) 40.6
+// against 42.3 us with 128.  (More than 4 vectors per lane of a single wave:
+// 47.5 against 44.2 us at [28672, 2047].)  Returns false when the row needs
+// more than 1024 x 8 vectors.
+constexpr int kRegVpt = 4;
+constexpr int64_t kPairMax = 320;
 // At most 8 vectors per lane (rows <= 1024 x 8 x 8 = 65536).  12 fit in
 // 110 VGPRs but measured mixed: [256, 98304] 51% -> 57%, [300, 70000]
 // 45% -> 36% (idle lanes and a 17%-full second round); 16 or more spill.
 constexpr int kRegVptMax = 8;
 bool reg_shape(int64_t nv, int& G, int& VPT) {
-    static const int kG[] = {8, 16, 32, 64, 256, 1024};
+    static const int kG[] = {8, 16, 32, 64, 128, 256, 1024};
     G = 0;
-    for (int g : kG)
-        if (nv <= static_cast<int64_t>(kRegVpt) * g) {
+    for (int g : kG) {
+        if (nv <= (g == 128 ? kPairMax : static_cast<int64_t>(kRegVpt) * g)) {
             G = g;
             break;
         }
+    }
     if (G == 0) {
         if (nv > 1024 * kRegVptMax) return false;
         G = 1024;
     }
-    const int64_t v = ceil_div(nv, G);
-    VPT = v <= 1 ? 1 : v <= 2 ? 2 : v <= 4 ? 4 : 8;
-    if (G < 64 && VPT > 4) return false;  // not instantiated (kRegVpt > 4 only)
+    VPT = static_cast<int>(ceil_div(nv, G));
+    if (VPT > 4) VPT = 8;
     return true;
 }
 
-template <int G>
+template <int G, bool RAGGED>
 void launch_reg(const half_t* x, half_t* y, int64_t N, int64_t D, int VPT, hipStream_t s) {
-    constexpr int kThreads = G > 256 ? G : 256;
+    constexpr int kThreads = G > 64 ? G : 256;
     const dim3 g(static_cast<unsigned>(ceil_div(N, kThreads / G))), b(kThreads);
-    if (VPT == 1)
-        softmax_reg_kernel<G, 1><<<g, b, 0, s>>>(x, y, N, D);
-    else if (VPT == 2)
-        softmax_reg_kernel<G, 2><<<g, b, 0, s>>>(x, y, N, D);
-    else if (VPT == 4 || G < 64)  // reg_shape gives fewer than 64 lanes at most 4 vectors
-        softmax_reg_kernel<G, 4><<<g, b, 0, s>>>(x, y, N, D);
-    else if constexpr (G >= 64)
-        softmax_reg_kernel<G, 8><<<g, b, 0, s>>>(x, y, N, D);
+    switch (VPT) {
+#define MI_REG_CASE(V) \
+    case V: softmax_reg_kernel<G, V, RAGGED><<<g, b, 0, s>>>(x, y, N, D); break;
+        MI_REG_CASE(1)
+        MI_REG_CASE(2)
+        MI_REG_CASE(3)
+        MI_REG_CASE(4)
+        default:  // only 1024 lanes hold more (reg_shape)
+            if constexpr (G == 1024) softmax_reg_kernel<G, 8, RAGGED><<<g, b, 0, s>>>(x, y, N, D);
+#undef MI_REG_CASE
+    }
+}
+
+template <bool RAGGED>
+int launch_reg_rows(const half_t* x, half_t* y, int64_t N, int64_t D, int G, int VPT,
+                    hipStream_t s) {
+    switch (G) {
+        case 8: launch_reg<8, RAGGED>(x, y, N, D, VPT, s); break;
+        case 16: launch_reg<16, RAGGED>(x, y, N, D, VPT, s); break;
+        case 32: launch_reg<32, RAGGED>(x, y, N, D, VPT, s); break;
+        case 64: launch_reg<64, RAGGED>(x, y, N, D, VPT, s); break;
+        case 128: launch_reg<128, RAGGED>(x, y, N, D, VPT, s); break;
+        case 256: launch_reg<256, RAGGED>(x, y, N, D, VPT, s); break;
+        default: launch_reg<1024, RAGGED>(x, y, N, D, VPT, s); break;
+    }
+    return launch_status();
 }
 
 template <int VEC>
@@ -872,6 +974,13 @@ bool onelaunch_ok(const void* x, const void* y, int64_t N, int64_t D, bool am = 
            onelaunch_rows(N, D, am) >= 1;
 }
 
+// Whether every row of x and of y has the same RowWindow: fp16-aligned bases
+// at the same offset from a 16-byte boundary.
+bool same_window(const void* x, const void* y) {
+    const auto a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(y);
+    return (a & 1) == 0 && ((a ^ b) & 15) == 0;
+}
+
 int softmax_checked(const void* x, void* y, int64_t N, int64_t D, void* ws, int64_t ws_bytes,
                     Ws layout, void* stream) {
     if (N < 0 || D < 0 || ws_bytes < 0) return MI_ERR_INVALID_ARGUMENT;
@@ -902,19 +1011,15 @@ int softmax_checked(const void* x, void* y, int64_t N, int64_t D, void* ws, int6
     const hipStream_t s = as_stream(stream);
     const bool vec = D % 8 == 0 && aligned16(x) && aligned16(y);
     if (p == Plan::kRow || (p == Plan::kStream && !onelaunch)) {
+        // rows through their aligned windows: up to 7 elements of a
+        // neighbour at each end
+        const bool ragged = !vec && same_window(x, y);
+        const int64_t nv = ragged ? ceil_div(D + 7, 8) : D / 8;
         int G = 0, VPT = 0;
-        if (MI_SOFTMAX_REG && vec && reg_shape(D / 8, G, VPT) &&
-            ceil_div(N, (G > 256 ? G : 256) / G) <= kMaxGridX) {
-            switch (G) {
-                case 8: launch_reg<8>(xh, yh, N, D, VPT, s); break;
-                case 16: launch_reg<16>(xh, yh, N, D, VPT, s); break;
-                case 32: launch_reg<32>(xh, yh, N, D, VPT, s); break;
-                case 64: launch_reg<64>(xh, yh, N, D, VPT, s); break;
-                case 256: launch_reg<256>(xh, yh, N, D, VPT, s); break;
-                default: launch_reg<1024>(xh, yh, N, D, VPT, s); break;
-            }
-            return launch_status();
-        }
+        if (MI_SOFTMAX_REG && (vec || ragged) && reg_shape(nv, G, VPT) &&
+            ceil_div(N, (G > 64 ? G : 256) / G) <= kMaxGridX)
+            return ragged ? launch_reg_rows<true>(xh, yh, N, D, G, VPT, s)
+                          : launch_reg_rows<false>(xh, yh, N, D, G, VPT, s);
         const int64_t want = ceil_div(D, vec ? 8 : 1);
         const int threads = static_cast<int>(ceil_div(want < 1024 ? want : 1024, kWave) * kWave);
         if (vec)

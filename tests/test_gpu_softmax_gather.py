@@ -50,6 +50,43 @@ def test_softmax_shapes(mk, orc, dev, N, D):
     assert_close(y, orc.softmax(x, nthreads=8), what=f"[{N},{D}]")
 
 
+@pytest.mark.parametrize("D", [1, 6, 9, 63, 250, 257, 505, 506, 1017, 1018, 2041, 2042, 2553, 2554,
+                               8185, 8186, 32767])
+@pytest.mark.parametrize("off,inplace", [(0, False), (3, False), (8, True), (5, True)])
+def test_softmax_ragged_rows(mk, orc, dev, D, off, inplace):
+    """Rows that are no whole number of 16-byte vectors, at the sizes where the
+    lanes per row change, from bases off a 16-byte boundary: the result, and
+    that nothing beside the rows is written.  An output is RN16 of an fp32
+    value whose exponent argument (|x - m| < 64) is off by at most 2^-18 and
+    whose sum by less: |y - ref| <= 2^-11 (1 + 2^-5) ref + 2^-25."""
+    import torch
+    N = 600 if D > 8191 else 37
+    _case(f"softmax ragged [{N},{D}] offset {off} in place {inplace}")
+    rng = np.random.default_rng(D * 16 + off)
+    x = normal_f16(rng, (N, D), 0, 4)
+    x[1, 1::2] = -np.inf
+    guard = 64
+
+    def buffer():
+        return torch.full((guard + off + N * D + guard,), 7.0, dtype=torch.float16, device=dev)
+
+    xb = buffer()
+    xd = xb[guard + off:guard + off + N * D].view(N, D)
+    xd.copy_(to_dev(x, dev))
+    yb = xb if inplace else buffer()
+    yd = yb[guard + off:guard + off + N * D].view(N, D)
+    mk.softmax(xd, y=yd)
+    y = to_host(yd).astype(np.float64)
+    x64 = x.astype(np.float64)
+    e = np.exp(x64 - x64.max(-1, keepdims=True))
+    ref = e / e.sum(-1, keepdims=True)
+    assert (np.abs(y - ref) <= 2.0 ** -11 * (1 + 2.0 ** -5) * ref + 2.0 ** -25).all()
+    whole = to_host(yb)
+    assert (whole[:guard + off] == 7).all() and (whole[guard + off + N * D:] == 7).all()
+    if not inplace:
+        assert_bits_equal(to_host(xd), x, what="x")
+
+
 def test_softmax_in_place_and_neg_inf(mk, orc, dev):
     _case("softmax in place, -inf entries")
     rng = np.random.default_rng(52)

@@ -227,8 +227,9 @@ int mi_add_bias_f16(void* y, const void* bias, int64_t M, int64_t N, int64_t bat
  * N < 256 when D <= 65536) are split across workgroups, and so are many rows
  * longer than 32768 (N >= 512, or N >= 256 up to 65536; at most 64 x 8192
  * elements) when the call can run in one launch.  On the legacy default
- * stream (0, the reference's callers' stream) out-of-place aligned calls of
- * these shapes run in one launch, using 1,056,768 bytes of row records that
+ * stream (0, the reference's callers' stream) out-of-place calls of these
+ * shapes (x and y at the same offset from a 16-byte boundary) run in one
+ * launch, using 1,056,768 bytes of row records that
  * the library allocates and zeroes once per device, on first use, and keeps
  * until the process ends.  On other streams, or in place, few long rows take
  * two launches with a stream-ordered workspace for the call, and many long
@@ -248,8 +249,9 @@ int64_t mi_softmax_workspace_bytes(int64_t N, int64_t D);
  * 16-byte aligned), so the call allocates nothing and can be captured into a
  * HIP graph.  The workspace must hold zeros before its first use and then be
  * used only by this function (any shapes); each call leaves it valid for the
- * next.  With y != x and aligned rows of <= 64 x 8192 elements, split rows
- * run in ONE launch: chunks exchange (max, sum) through tagged per-row
+ * next.  With y != x, both at the same offset from a 16-byte boundary, and
+ * rows of <= 64 x 8192 elements (7 fewer when D % 8 != 0 or the offset is
+ * not 0), split rows run in ONE launch: chunks exchange (max, sum) through tagged per-row
  * records, with no atomics on a shared address -- every chunk of the grid
  * resident at once, or, for more rows than that, a resident grid that walks
  * the rows in rounds.  In place, or otherwise, few long rows take the
@@ -281,7 +283,7 @@ int mi_softmax_noalloc_f16(const void* x, void* y, int64_t N, int64_t D, void* s
  * order), reading the logits once.  Replaces launch_softmax + launch_greedy
  * _sample_batched over the same logits (src/kernels/softmax_kernel.cuh:12,
  * sampling_kernel.cuh:25-30).  Shapes the one-launch softmax takes (split
- * or many long rows, aligned, probs != logits) run as one kernel whose chunks
+ * or many long rows, probs != logits) run as one kernel whose chunks
  * also publish their best key; others run the two entry points in turn.
  * The workspace (mi_softmax_argmax_workspace_bytes(N, V) bytes, 16-byte
  * aligned) must hold zeros before its first use and then serve only this
@@ -359,8 +361,8 @@ int mi_paged_kv_scatter_kv_bias_f16(const void* k_src, const void* v_src, void* 
  * with nothing above -inf gives -1.
  * Replaces launch_greedy_sample / launch_greedy_sample_batched
  * (src/kernels/sampling_kernel.cuh:17-30; src/kernels/sampling_kernel.cu:14-76).
- * B < 512 rows of V >= 8192 are split across workgroups: on stream 0 (V % 16
- * == 0, aligned) in one launch with 532,480 bytes of row records the library
+ * B < 512 rows of V >= 8192 are split across workgroups: on stream 0 in one
+ * launch with 532,480 bytes of row records the library
  * holds per device (allocated and zeroed on first use, kept until the process
  * ends), otherwise in two launches with <= 256 KiB of stream-ordered
  * workspace for the call. */
@@ -374,8 +376,8 @@ int64_t mi_greedy_argmax_workspace_bytes(int64_t B, int64_t V);
 /* mi_greedy_argmax_f16 with a caller-provided device workspace (allocates
  * nothing; graph-capturable; 16-byte aligned).  The workspace must hold zeros
  * before its first use and then be used only by this function (any shapes);
- * each call leaves it valid for the next.  Split rows with V % 16 == 0 and
- * V <= 64 x 8192 run in ONE launch: every chunk publishes its best key to a
+ * each call leaves it valid for the next.  Split rows of V <= 64 x 8192 (7
+ * fewer when V % 16 != 0 or unaligned) run in ONE launch: every chunk publishes its best key to a
  * tagged per-row record and only chunk 0 of each row waits to combine them.
  * Calls sharing a workspace must not overlap. */
 int mi_greedy_argmax_ws_f16(const void* logits, int64_t B, int64_t V, int32_t* out,

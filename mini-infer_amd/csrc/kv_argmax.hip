@@ -234,7 +234,9 @@ constexpr int kArgmaxMaxSplits = 1024;
 
 // grid (splits, B).  With one split the index goes straight to `out`;
 // otherwise each chunk's key goes to ws[row * splits + split].
-template <int VEC, int U>
+// RAGGED: chunks of the row's aligned window (RowWindow), the last one to its
+// end ([1024, 32001] 28.5 -> 14.7 us against the 2-byte kernel).
+template <int VEC, int U, bool RAGGED = false>
 __global__ __launch_bounds__(256) void argmax_partial_kernel(const half_t* __restrict__ x,
                                                              int64_t V, int64_t chunk,
                                                              uint64_t* __restrict__ ws,
@@ -244,7 +246,15 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(const half_t* __res
     const int64_t row = blockIdx.y;
     const int64_t b = split * chunk;
     const int64_t e = b + chunk < V ? b + chunk : V;
-    const uint64_t best = chunk_best<VEC, U>(x + row * V, b, e, slots);
+    uint64_t best;
+    if constexpr (RAGGED) {
+        const RowWindow win(x + row * V, V);
+        const int64_t len = static_cast<int64_t>(win.nv) * 8;
+        best = chunk_best_window<U>(x + row * V - win.shift, b, split + 1 == splits ? len : b + chunk,
+                                    win, slots);
+    } else {
+        best = chunk_best<VEC, U>(x + row * V, b, e, slots);
+    }
     if (threadIdx.x == 0) {
         if (splits == 1)
             out[row] = key_index(best);
@@ -339,6 +349,9 @@ __device__ __forceinline__ bool argmax_poll(const uint64_t* set, int splits, uin
     return false;
 }
 
+// RAGGED: chunks of the row's aligned window (RowWindow): [64, 151643] 6.8 us
+// against 11.6 in two launches of 2-byte accesses (aligned [64, 152064]: 6.1).
+template <bool RAGGED>
 __global__ __launch_bounds__(256) void argmax_onepass_kernel(const half_t* __restrict__ x,
                                                              int64_t V, unsigned char* ws,
                                                              int32_t* __restrict__ out,
@@ -355,9 +368,12 @@ __global__ __launch_bounds__(256) void argmax_onepass_kernel(const half_t* __res
     unsigned char* rec = ws + row * kArgmaxRecordBytes;
     uint64_t* epoch = reinterpret_cast<uint64_t*>(rec);
     uint64_t* slot = reinterpret_cast<uint64_t*>(rec + kRecordHeaderBytes);
-    const half_t* xr = x + row * V;
+    const RowWindow win(x + row * V, V);  // RAGGED
+    const int shift = RAGGED ? win.shift : 0;
+    const int64_t len = RAGGED ? win.nv * 8 : V;
+    const half_t* xr = x + row * V - shift;
     const int64_t b = split * kArgmaxOnePassChunk;
-    const int64_t e = b + kArgmaxOnePassChunk < V ? b + kArgmaxOnePassChunk : V;
+    const int64_t e = b + kArgmaxOnePassChunk < len ? b + kArgmaxOnePassChunk : len;
     // The row's epoch, read by every lane (one request per wave) ahead of the
     // chunk's loads and with no branch around it, so its first wait comes at
     // the publish: a lane-0 load followed by its store to LDS made wave 0
@@ -366,8 +382,8 @@ __global__ __launch_bounds__(256) void argmax_onepass_kernel(const half_t* __res
     // (chunk_load).  6.85 -> 6.6 us at [64, 152064].
     const uint64_t E = __hip_atomic_load(epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     h8 a[kArgmaxOnePassU];
-    chunk_load<kArgmaxOnePassU>(xr, b, e, a);
-    const uint64_t best = chunk_best_of<kArgmaxOnePassU>(a, b, slots);  // barrier inside
+    chunk_load<kArgmaxOnePassU>(xr, b, e, a, RAGGED ? &win : nullptr);
+    const uint64_t best = chunk_best_of<kArgmaxOnePassU, RAGGED>(a, b, slots, shift);  // barrier inside
     const uint32_t tag = static_cast<uint32_t>(E + 1);
     if (threadIdx.x == 0) {
         const uint64_t w0 = (static_cast<uint64_t>(tag) << 32) | (best >> 32);
@@ -400,7 +416,8 @@ __global__ __launch_bounds__(256) void argmax_onepass_kernel(const half_t* __res
     const bool fallback = fallback_sh != 0;
     if (fallback) {
         // the whole row from x (slots reused after the barrier above)
-        const uint64_t k = chunk_best<8, 4>(xr, 0, V, slots);
+        const uint64_t k = RAGGED ? chunk_best<1, 8>(xr + shift, 0, V, slots)
+                                  : chunk_best<8, 4>(xr, 0, V, slots);
         if (threadIdx.x == 0) out[row] = key_index(k);
     }
     if (threadIdx.x == 0)
@@ -440,12 +457,23 @@ enum class Ws {
     kRecords,          // the one-launch row records only (library-held, stream 0)
 };
 
+// Rows of whole 16-byte vectors, as the vector kernels take them; other rows
+// of fp16-aligned logits go through their aligned windows, up to 7 elements
+// longer.
+bool argmax_vec(const void* logits, int64_t V) { return V % 16 == 0 && aligned16(logits); }
+bool argmax_ragged(const void* logits, int64_t V) {
+    return !argmax_vec(logits, V) && (reinterpret_cast<uintptr_t>(logits) & 1) == 0;
+}
+int64_t argmax_onepass_splits(const void* logits, int64_t V) {
+    return ceil_div(argmax_vec(logits, V) ? V : V + 7, kArgmaxOnePassChunk);
+}
+
 // Whether [B, V] runs as the one-launch split form given row records.
 bool argmax_onepass_ok(const void* logits, int64_t B, int64_t V) {
     if (!MI_ARGMAX_ONEPASS || B <= 0 || V <= 0 || B > 65535 || V > 0x7fffffff) return false;
     int64_t chunk;
-    return argmax_splits(B, V, chunk) > 1 && V % 16 == 0 && aligned16(logits) &&
-           ceil_div(V, kArgmaxOnePassChunk) <= kArgmaxOnePassMaxSplits;
+    return argmax_splits(B, V, chunk) > 1 && (argmax_vec(logits, V) || argmax_ragged(logits, V)) &&
+           argmax_onepass_splits(logits, V) <= kArgmaxOnePassMaxSplits;
 }
 
 int argmax(const void* logits, int64_t B, int64_t V, int32_t* out, void* ws, int64_t ws_bytes,
@@ -474,13 +502,21 @@ int argmax(const void* logits, int64_t B, int64_t V, int32_t* out, void* ws, int
     }
     const hipStream_t st = as_stream(stream);
     const auto* x = static_cast<const half_t*>(logits);
-    const bool vec = V % 16 == 0 && aligned16(logits);
+    const bool vec = argmax_vec(logits, V);
+    const bool ragged = argmax_ragged(logits, V);
     if (onepass) {
-        const int64_t sp1 = ceil_div(V, kArgmaxOnePassChunk);
+        const int64_t sp1 = argmax_onepass_splits(logits, V);
         const int64_t rows = ceil_div(B, kXcds) * kXcds;  // <= kArgmaxSplitMaxRows
-        argmax_onepass_kernel<<<dim3(static_cast<unsigned>(sp1 * rows)), dim3(256), 0, st>>>(
-            x, V, static_cast<unsigned char*>(ws), out, g_argmax_poll_limit.load(), B,
-            static_cast<int>(sp1), exchange_test_mode().load() == 0 ? 1 : 0);
+        const dim3 g1(static_cast<unsigned>(sp1 * rows));
+        auto* rec = static_cast<unsigned char*>(ws);
+        const int limit = g_argmax_poll_limit.load();
+        const int local = exchange_test_mode().load() == 0 ? 1 : 0;
+        if (ragged)
+            argmax_onepass_kernel<true><<<g1, dim3(256), 0, st>>>(x, V, rec, out, limit, B,
+                                                                  static_cast<int>(sp1), local);
+        else
+            argmax_onepass_kernel<false><<<g1, dim3(256), 0, st>>>(x, V, rec, out, limit, B,
+                                                                   static_cast<int>(sp1), local);
         return launch_status();
     }
     auto* w = reinterpret_cast<uint64_t*>(
@@ -497,6 +533,13 @@ int argmax(const void* logits, int64_t B, int64_t V, int32_t* out, void* ws, int
             argmax_partial_kernel<8, 2><<<g, dim3(256), 0, st>>>(x, V, chunk, w, out);
         else
             argmax_partial_kernel<8, 1><<<g, dim3(256), 0, st>>>(x, V, chunk, w, out);
+    } else if (ragged && V > 0) {
+        if (splits == 1 && V >= MI_ARGMAX_ROW_DEEP)
+            argmax_partial_kernel<8, MI_ARGMAX_ROW_U, true><<<g, dim3(256), 0, st>>>(x, V, chunk, w, out);
+        else if (two)
+            argmax_partial_kernel<8, 2, true><<<g, dim3(256), 0, st>>>(x, V, chunk, w, out);
+        else
+            argmax_partial_kernel<8, 1, true><<<g, dim3(256), 0, st>>>(x, V, chunk, w, out);
     } else {
         argmax_partial_kernel<1, 8><<<g, dim3(256), 0, st>>>(x, V, chunk, w, out);
     }

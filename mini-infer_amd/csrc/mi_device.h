@@ -217,6 +217,74 @@ __device__ __forceinline__ float block_max(float v, float* slots) {
     return t;
 }
 
+// A row whose 16-byte window is not the row itself (D % 8 != 0, or a base
+// that is not 16-byte aligned): the aligned 16-byte vectors that cover it.
+// Element e of the row is at window position e + shift (shift < 8), so only
+// vector 0 and the last one hold elements of other rows.  Those share a
+// 16-byte granule with the row's own, so reading them never reaches another
+// page; they are masked to -inf after the load and never stored.  Two tensors
+// at the same offset from a 16-byte boundary (same_window) have the same shift
+// in every row, so a vector is stored where it was loaded; rows 8 apart have
+// the same shift too (8 D elements are 16 D bytes).
+struct RowWindow {
+    int shift;  // elements of the window before the row
+    int nv;     // vectors of the window
+    int last;   // elements of its last vector up to the row's end (1 .. 8)
+    __device__ __forceinline__ RowWindow(const half_t* row, int64_t D)
+        : shift(static_cast<int>((reinterpret_cast<uintptr_t>(row) & 15) >> 1)),
+          nv(static_cast<int>((shift + D + 7) >> 3)),
+          last(static_cast<int>((shift + D - 1) & 7) + 1) {}
+    __device__ __forceinline__ bool partial(int v) const {
+        return (v == 0 && shift > 0) || (v == nv - 1 && last < 8);
+    }
+    // the elements of vector v that are not the row's become -inf
+    __device__ __forceinline__ void mask(int v, h8& a) const {
+        if (v == 0) {
+#pragma unroll
+            for (int k = 0; k < 7; ++k)
+                if (k < shift) a[k] = -__builtin_huge_valf16();
+        }
+        if (v == nv - 1) {
+#pragma unroll
+            for (int k = 1; k < 8; ++k)
+                if (k >= last) a[k] = -__builtin_huge_valf16();
+        }
+    }
+    // vector v of the row's window to p (16-byte aligned).  A vector that
+    // the row begins in is stored as a 2-, a 4- and an 8-byte piece up to the
+    // granule's end, one that it ends in as an 8-, a 4- and a 2-byte piece
+    // from its start; a row inside one granule element by element.
+    __device__ __forceinline__ void store(int v, half_t* p, h8 a) const {
+        const int l = v == 0 ? shift : 0, h = v == nv - 1 ? last : 8;
+        if (l == 0 && h == 8) {
+            st8_stream(p, a);
+            return;
+        }
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        const u32x4 w = __builtin_bit_cast(u32x4, a);
+        auto* p2 = reinterpret_cast<uint16_t*>(p);
+        auto* p4 = reinterpret_cast<uint32_t*>(p);
+        if (h == 8) {  // elements l .. 7
+            if (l & 1)
+                p2[l] = static_cast<uint16_t>((l < 4 ? (l < 2 ? w[0] : w[1]) : (l < 6 ? w[2] : w[3])) >> 16);
+            const int d = (l + 1) >> 1;  // first whole dword
+            if (d & 1) p4[d] = d == 1 ? w[1] : w[3];
+            if (d <= 2) *reinterpret_cast<u32x2*>(p + 4) = u32x2{w[2], w[3]};
+            if (d == 0) *reinterpret_cast<u32x2*>(p) = u32x2{w[0], w[1]};
+        } else if (l == 0) {  // elements 0 .. h - 1
+            if (h & 4) *reinterpret_cast<u32x2*>(p) = u32x2{w[0], w[1]};
+            if (h & 2) p4[(h & 4) >> 1] = h & 4 ? w[2] : w[0];
+            if (h & 1)
+                p2[h - 1] = static_cast<uint16_t>(h & 4 ? (h & 2 ? w[3] : w[2]) : (h & 2 ? w[1] : w[0]));
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (k >= l && k < h) p[k] = a[k];
+        }
+    }
+};
+
 // Sum of squares of a head's slice pair, x1 (first half) and x2 (second half)
 // of 8 halves each, as every fused Q/K-norm + RoPE kernel forms it (they must
 // agree bit for bit: the one-launch attention pre-processing is checked

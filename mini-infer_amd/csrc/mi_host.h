@@ -16,6 +16,13 @@ namespace mi {
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Whether every row of x and of y has the same RowWindow: fp16-aligned bases
+// at the same offset from a 16-byte boundary.
+inline bool same_window(const void* x, const void* y) {
+    const auto a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(y);
+    return (a & 1) == 0 && ((a ^ b) & 15) == 0;
+}
+
 // True when [a, a+abytes) and [b, b+bbytes) share at least one byte.
 inline bool overlaps(const void* a, int64_t abytes, const void* b, int64_t bbytes) {
     const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);

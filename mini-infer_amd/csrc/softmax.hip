@@ -119,10 +119,11 @@ __device__ __forceinline__ void lane_stats(const half_t* xr, int64_t begin, int6
 // tile's lane maximum comes from packed fp16 max (which passes over NaN, as
 // fmaxf does), then one exp per element against it, and one online merge
 // per tile -- not a rescale per vector.  Out-of-range slots hold -inf, whose
-// exp is 0.
-template <int U>
+// exp is 0.  RAGGED: xr is the row's window `win`, [begin, end) positions in
+// it.
+template <int U, bool RAGGED = false>
 __device__ __forceinline__ void tile_stats(const half_t* xr, int64_t begin, int64_t end, float& m,
-                                           float& s) {
+                                           float& s, const RowWindow* win = nullptr) {
     constexpr int64_t kTile = 256 * 8 * U;
     for (int64_t t0 = begin; t0 < end; t0 += kTile) {
         h8 a[U];
@@ -130,6 +131,14 @@ __device__ __forceinline__ void tile_stats(const half_t* xr, int64_t begin, int6
         for (int j = 0; j < U; ++j) {
             const int64_t i = t0 + (threadIdx.x + j * 256) * 8;
             a[j] = i < end ? ld8(xr + i) : h8(-__builtin_huge_valf16());
+        }
+        if constexpr (RAGGED) {
+#pragma unroll
+            for (int j = 0; j < U; ++j) {
+                const int64_t i = t0 + (threadIdx.x + j * 256) * 8;
+                if (i < end && win->partial(static_cast<int>(i >> 3)))
+                    win->mask(static_cast<int>(i >> 3), a[j]);
+            }
         }
         h2 m2 = h2(-__builtin_huge_valf16());
 #pragma unroll
@@ -154,9 +163,10 @@ __device__ __forceinline__ void tile_stats(const half_t* xr, int64_t begin, int6
 
 // y = exp(x - m) * inv over [begin, end): the last use of x and the only
 // write of y, both streamed.
-template <int VEC>
+template <int VEC, bool RAGGED = false>
 __device__ __forceinline__ void write_range(const half_t* xr, half_t* yr, int64_t begin,
-                                            int64_t end, float m, float inv) {
+                                            int64_t end, float m, float inv,
+                                            const RowWindow* win = nullptr) {
     const int64_t step = static_cast<int64_t>(blockDim.x) * VEC;
     for (int64_t i0 = begin + static_cast<int64_t>(threadIdx.x) * VEC; i0 < end;
          i0 += step * kStatUnroll) {
@@ -175,7 +185,10 @@ __device__ __forceinline__ void write_range(const half_t* xr, half_t* yr, int64_
 #pragma unroll
                     for (int k = 0; k < 8; ++k)
                         o[k] = to_half(exp_shifted((float)h[j][k], m * kLog2e) * inv);
-                    st8_out<MI_WT_SM>(yr + i, o);
+                    if constexpr (RAGGED)
+                        win->store(static_cast<int>(i >> 3), yr + i, o);
+                    else
+                        st8_out<MI_WT_SM>(yr + i, o);
                 }
             }
         } else {
@@ -198,70 +211,6 @@ __device__ __forceinline__ void block_merge(float& m, float& s, float* slots) {
     s = block_sum(part, slots);
     m = M;
 }
-
-// A row whose 16-byte window is not the row itself (D % 8 != 0, or a base
-// that is not 16-byte aligned): the aligned 16-byte vectors that cover it.
-// Element e of the row is at window position e + shift (shift < 8), so only
-// vector 0 and the last one hold elements of other rows.  Those share a
-// 16-byte granule with the row's own, so reading them never reaches another
-// page; they are masked to -inf after the load and never stored.  x and y
-// at the same offset from a 16-byte boundary (the caller checks) have the
-// same shift in every row, so a vector is stored where it was loaded.
-struct RowWindow {
-    int shift;   // elements of the window before the row
-    int nv;      // vectors of the window
-    int64_t end;  // shift + D
-    __device__ __forceinline__ RowWindow(const half_t* row, int64_t D)
-        : shift(static_cast<int>((reinterpret_cast<uintptr_t>(row) & 15) >> 1)),
-          nv(static_cast<int>((shift + D + 7) >> 3)),
-          end(shift + D) {}
-    // elements [lo, hi) of vector v belong to the row
-    __device__ __forceinline__ int lo(int v) const { return v == 0 ? shift : 0; }
-    __device__ __forceinline__ int hi(int v) const {
-        const int64_t left = end - static_cast<int64_t>(v) * 8;
-        return left < 8 ? static_cast<int>(left) : 8;
-    }
-    __device__ __forceinline__ bool partial(int v) const { return lo(v) != 0 || hi(v) != 8; }
-    __device__ __forceinline__ void mask(int v, h8& a) const {
-        const int l = lo(v), h = hi(v);
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            if (k < l || k >= h) a[k] = -__builtin_huge_valf16();
-    }
-    // vector v of the row's window to p (16-byte aligned).  A vector that
-    // the row begins in is stored as a 2-, a 4- and an 8-byte piece up to the
-    // granule's end, one that it ends in as an 8-, a 4- and a 2-byte piece
-    // from its start; a row inside one granule element by element.
-    __device__ __forceinline__ void store(int v, half_t* p, h8 a) const {
-        const int l = lo(v), h = hi(v);
-        if (l == 0 && h == 8) {
-            st8_out<MI_WT_SM>(p, a);
-            return;
-        }
-        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-        const u32x4 w = __builtin_bit_cast(u32x4, a);
-        auto* p2 = reinterpret_cast<uint16_t*>(p);
-        auto* p4 = reinterpret_cast<uint32_t*>(p);
-        if (h == 8) {  // elements l .. 7
-            if (l & 1)
-                p2[l] = static_cast<uint16_t>((l < 4 ? (l < 2 ? w[0] : w[1]) : (l < 6 ? w[2] : w[3])) >> 16);
-            const int d = (l + 1) >> 1;  // first whole dword
-            if (d & 1) p4[d] = d == 1 ? w[1] : w[3];
-            if (d <= 2) *reinterpret_cast<u32x2*>(p + 4) = u32x2{w[2], w[3]};
-            if (d == 0) *reinterpret_cast<u32x2*>(p) = u32x2{w[0], w[1]};
-        } else if (l == 0) {  // elements 0 .. h - 1
-            if (h & 4) *reinterpret_cast<u32x2*>(p) = u32x2{w[0], w[1]};
-            if (h & 2) p4[(h & 4) >> 1] = h & 4 ? w[2] : w[0];
-            if (h & 1)
-                p2[h - 1] = static_cast<uint16_t>(h & 4 ? (h & 2 ? w[3] : w[2]) : (h & 2 ? w[1] : w[0]));
-        } else {
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (k >= l && k < h) p[k] = a[k];
-        }
-    }
-};
 
 // Register-resident rows (16-byte vectors, D <= G * VPT * 8): G lanes per
 // row -- G <= 64: 256 / G rows per workgroup and DPP-only reductions;
@@ -443,7 +392,8 @@ __global__ __launch_bounds__(1024) void softmax_row_kernel(const half_t* x, half
 }
 
 // VEC = 8: U vectors per lane per tile (tile_stats); VEC = 1: lane_stats.
-template <int VEC, int U>
+// RAGGED (VEC = 8): chunks of the row's window, the last one to its end.
+template <int VEC, int U, bool RAGGED = false>
 __global__ __launch_bounds__(256) void softmax_partial_kernel(const half_t* x, float* ws,
                                                               int64_t D, int64_t chunk) {
     __shared__ float slots[256 / kWave];
@@ -452,7 +402,11 @@ __global__ __launch_bounds__(256) void softmax_partial_kernel(const half_t* x, f
     const int64_t b = split * chunk;
     const int64_t e = b + chunk < D ? b + chunk : D;
     float m = -INFINITY, s = 0.0f;
-    if constexpr (VEC == 8)
+    if constexpr (RAGGED) {
+        const RowWindow win(x + row * D, D);
+        tile_stats<U, true>(x + row * D - win.shift, b, split + 1 == splits ? win.nv * 8 : b + chunk,
+                            m, s, &win);
+    } else if constexpr (VEC == 8)
         tile_stats<U>(x + row * D, b, e, m, s);
     else
         lane_stats<VEC>(x + row * D, b, e, m, s);
@@ -464,7 +418,7 @@ __global__ __launch_bounds__(256) void softmax_partial_kernel(const half_t* x, f
     }
 }
 
-template <int VEC>
+template <int VEC, bool RAGGED = false>
 __global__ __launch_bounds__(256) void softmax_finish_kernel(const half_t* x, half_t* y,
                                                              const float* __restrict__ ws,
                                                              int64_t D, int64_t chunk) {
@@ -485,7 +439,14 @@ __global__ __launch_bounds__(256) void softmax_finish_kernel(const half_t* x, ha
     const float S = group_sum<kWave>(m == -INFINITY ? 0.0f : s * fast_exp(m - M));
     const int64_t b = split * chunk;
     const int64_t e = b + chunk < D ? b + chunk : D;
-    write_range<VEC>(x + row * D, y + row * D, b, e, M, 1.0f / S);
+    if constexpr (RAGGED) {
+        const RowWindow win(x + row * D, D);
+        const int64_t off = row * D - win.shift;
+        write_range<VEC, true>(x + off, y + off, b, split + 1 == splits ? win.nv * 8 : b + chunk, M,
+                               1.0f / S, &win);
+    } else {
+        write_range<VEC>(x + row * D, y + row * D, b, e, M, 1.0f / S);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -681,10 +642,14 @@ __device__ __forceinline__ void row_poll(const uint64_t* slots, int64_t mirror, 
 }
 // The row's statistics from x itself (the fallback when polling runs out; x
 // is not written: y != x).  Barriers: called by the whole workgroup.
+template <bool RAGGED>
 __device__ __forceinline__ void row_stats_from_x(const half_t* xr, int64_t D, float& M, float& S,
                                                  float* slots) {
     float fm = -INFINITY, fs = 0.0f;
-    tile_stats<2>(xr, 0, D, fm, fs);
+    if constexpr (RAGGED)
+        lane_stats<1>(xr, 0, D, fm, fs);
+    else
+        tile_stats<2>(xr, 0, D, fm, fs);
     __syncthreads();  // slots reused
     block_merge(fm, fs, slots);
     __syncthreads();  // every wave has read slots before a later round writes them
@@ -704,9 +669,11 @@ __device__ __forceinline__ void lane_load(const half_t* row, uint32_t lo, const 
         a[j] = ok[j] ? ld8_stream(p) : h8(-__builtin_huge_valf16());
     }
 }
-template <int U>
+// RAGGED: row is the row's window, v0 the lane's first vector in it.
+template <int U, bool RAGGED>
 __device__ __forceinline__ void lane_store(const h8 (&a)[U], half_t* row, uint32_t lo,
-                                           const bool (&ok)[U], float M, float inv) {
+                                           const bool (&ok)[U], float M, float inv,
+                                           const RowWindow& win, int v0) {
     // y = exp(x - M) / S = exp2(x log2(e) - (M log2(e) + log2(S))): the division folded into
     // the exponent's constant c, one fma and the exp per element ([512, 131072] 46.4 -> 46.0
     // us; c carries the same rounding as M log2(e) alone, well under an fp16 ulp of y)
@@ -719,7 +686,11 @@ __device__ __forceinline__ void lane_store(const h8 (&a)[U], half_t* row, uint32
 #pragma unroll
             for (int k = 0; k < 8; ++k)
                 o[k] = to_half(__builtin_amdgcn_exp2f(fmaf((float)a[j][k], kLog2e, -c)));
-            st8_out<MI_WT_SM>(reinterpret_cast<half_t*>(base + j * 256 * 16), o);
+            half_t* p = reinterpret_cast<half_t*>(base + j * 256 * 16);
+            if constexpr (RAGGED)
+                win.store(v0 + j * 256, p, o);
+            else
+                st8_out<MI_WT_SM>(p, o);
         }
     }
 }
@@ -735,7 +706,16 @@ __device__ __forceinline__ void lane_store(const h8 (&a)[U], half_t* row, uint32
 // (AM: held to 5 waves per SIMD, <= 96 VGPRs, so that 1216 chunk workgroups
 // of [64, 152064] stay resident at once; the compiler otherwise settles at
 // 98 and the grid needs a second round.)
-template <int U, bool AM>
+// RAGGED: chunks of the row's aligned window (RowWindow) -- rows of a slot are
+// R (a multiple of 8) apart, so one window shape serves all its rounds.
+// Against the 2-byte two-launch forms: [64, 151643] 32.1 -> 9.9 us (softmax),
+// 37.1 -> 11.0 (with the argmax); aligned [64, 152064] 9.0 / 10.2.
+// ONE (ragged rows only): every row in one round, so no next row's registers
+// and no conditions kept across rounds -- 44-68 VGPRs against 73-96 and, with
+// AM, spills: [64, 151643] softmax + argmax 14.2 -> 11.0 us, [200, 32001]
+// softmax 10.2 -> 8.2.  (For aligned rows, which have no such conditions, it
+// measured slower: [64, 152064] 9.0 -> 9.6 and 10.2 -> 11.1 us.)
+template <int U, bool AM, bool RAGGED, bool ONE>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(AM ? 5 : 1))) void softmax_stream_kernel(const half_t* x, half_t* y,
                                                              unsigned char* ws, int64_t N,
@@ -759,29 +739,44 @@ __attribute__((amdgpu_waves_per_eu(AM ? 5 : 1))) void softmax_stream_kernel(cons
     uint64_t* epoch = reinterpret_cast<uint64_t*>(rec);
     uint64_t* sets = reinterpret_cast<uint64_t*>(rec + kRecordHeaderBytes);
     constexpr int64_t kMirror = 2 * SW * kOnePassMaxSplits;  // words from a set to its mirror
-    const int64_t K = (N - r0 + R - 1) / R;  // rounds of this row slot (>= 1)
+    const int64_t K = ONE ? 1 : (N - r0 + R - 1) / R;  // rounds of this row slot (>= 1)
+    RowWindow win(x + r0 * D, D);  // RAGGED
+    const int64_t shift = RAGGED ? win.shift : 0;
+    const int64_t len = RAGGED ? win.nv * 8 : D;
     const int64_t b = split * kChunk;
-    const int64_t e = b + kChunk < D ? b + kChunk : D;
+    const int64_t e = b + kChunk < len ? b + kChunk : len;
     const uint32_t lo = static_cast<uint32_t>(b + threadIdx.x * 8) * 2;
+    const int v0 = static_cast<int>(b >> 3) + static_cast<int>(threadIdx.x);
     bool ok[U];
 #pragma unroll
     for (int j = 0; j < U; ++j) ok[j] = b + (threadIdx.x + j * 256) * 8 < e;
 
     if (threadIdx.x == 0)
         epoch_sh = __hip_atomic_load(epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    h8 a[U], n[U];
-    lane_load<U>(x + r0 * D, lo, ok, a);
+    h8 a[U], n[ONE ? 1 : U];
+    lane_load<U>(x + r0 * D - shift, lo, ok, a);
     bool gave_up = false;  // workgroup-uniform: set after the first fallback
     for (int64_t k = 0; k < K; ++k) {
         const int64_t row = r0 + k * R;
         // The guard is always true (256 lanes); written out, it keeps the
         // statistics in a block of their own, which measured 64 VGPRs with
         // no spill against 80 without it.
+        if constexpr (RAGGED) {
+            // workgroup-uniform: the row's first or last vector.  (win made
+            // opaque in each round: its conditions otherwise stay in
+            // registers across the rounds, some 250 of them)
+            asm volatile("" : "+s"(win.shift), "+s"(win.last));
+            if (split == 0 || e == len) {
+#pragma unroll
+                for (int j = 0; j < U; ++j)
+                    if (ok[j]) win.mask(v0 + j * 256, a[j]);
+            }
+        }
         float m = -INFINITY, s = 0.0f;
         if (threadIdx.x < 256) chunk_lane_stats<U>(a, m, s);
         if constexpr (AM) {
             // vectors past the row hold -inf (lane_load), whose key is 0
-            const uint64_t kw = wave_max_u64(lane_best_key<U>(a, b));
+            const uint64_t kw = wave_max_u64(lane_best_key<U, RAGGED>(a, b, static_cast<int>(shift)));
             if ((threadIdx.x & (kWave - 1)) == 0) kslots[threadIdx.x / kWave] = kw;
         }
         block_merge(m, s, slots);  // barriers: epoch_sh (first round) and kslots visible after
@@ -794,7 +789,9 @@ __attribute__((amdgpu_waves_per_eu(AM ? 5 : 1))) void softmax_stream_kernel(cons
         const uint32_t tag = static_cast<uint32_t>(E + 1 + k);
         uint64_t* set = sets + (k & 1) * (SW * kOnePassMaxSplits);
         chunk_publish<AM>(set, kMirror, split, tag, m, s, key);
-        if (k + 1 < K) lane_load<U>(x + (row + R) * D, lo, ok, n);
+        if constexpr (!ONE) {
+            if (k + 1 < K) lane_load<U>(x + (row + R) * D - shift, lo, ok, n);
+        }
         if (gave_up) {
             if (threadIdx.x == 0) row_stats[2] = 1.0f;
         } else if (threadIdx.x < kWave) {
@@ -806,12 +803,13 @@ __attribute__((amdgpu_waves_per_eu(AM ? 5 : 1))) void softmax_stream_kernel(cons
         float M = row_stats[0], S = row_stats[1];
         const bool fallback = row_stats[2] != 0.0f;
         gave_up = gave_up || fallback;
-        if (fallback) row_stats_from_x(x + row * D, D, M, S, slots);
+        if (fallback) row_stats_from_x<RAGGED>(x + row * D, D, M, S, slots);
         if constexpr (AM) {
             if (split == 0) {  // workgroup-uniform: chunk_best has barriers
                 uint64_t rk = row_key;
                 if (fallback) {
-                    rk = chunk_best<8, 4>(x + row * D, 0, D, kslots);
+                    rk = RAGGED ? chunk_best<1, 8>(x + row * D, 0, D, kslots)
+                                : chunk_best<8, 4>(x + row * D, 0, D, kslots);
                     __syncthreads();  // kslots are written again by the next round
                 }
                 if (threadIdx.x == 0) out[row] = key_index(rk);
@@ -820,10 +818,13 @@ __attribute__((amdgpu_waves_per_eu(AM ? 5 : 1))) void softmax_stream_kernel(cons
         if (threadIdx.x == 0 && (fallback || (split == 0 && k + 1 == K)))
             __hip_atomic_fetch_max(epoch, fallback ? E + K + 1 : E + K, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
-        lane_store<U>(a, y + row * D, lo, ok, M, 1.0f / S);
-        if (k + 1 < K) {
+        if constexpr (RAGGED) asm volatile("" : "+s"(win.shift), "+s"(win.last));
+        lane_store<U, RAGGED>(a, y + row * D - shift, lo, ok, M, 1.0f / S, win, v0);
+        if constexpr (!ONE) {
+            if (k + 1 < K) {
 #pragma unroll
-            for (int j = 0; j < U; ++j) a[j] = n[j];
+                for (int j = 0; j < U; ++j) a[j] = n[j];
+            }
         }
     }
 }
@@ -919,66 +920,99 @@ int onelaunch_u(int64_t N, int64_t D) {
         return kSmall;
     return kOnePassU;
 }
-const void* onelaunch_kernel(int u, bool am) {
-    if (am)
-        return u == kOnePassU
-                   ? reinterpret_cast<const void*>(softmax_stream_kernel<kOnePassU, true>)
-                   : reinterpret_cast<const void*>(softmax_stream_kernel<kOnePassU / 2, true>);
-    return u == kOnePassU ? reinterpret_cast<const void*>(softmax_stream_kernel<kOnePassU, false>)
-                          : reinterpret_cast<const void*>(softmax_stream_kernel<kOnePassU / 2, false>);
+template <bool AM, bool RAGGED, bool ONE>
+const void* stream_kernel(int u) {
+    return u == kOnePassU
+               ? reinterpret_cast<const void*>(softmax_stream_kernel<kOnePassU, AM, RAGGED, ONE>)
+               : reinterpret_cast<const void*>(softmax_stream_kernel<kOnePassU / 2, AM, RAGGED, ONE>);
+}
+// one: the single-round kernel (ragged rows)
+const void* onelaunch_kernel(int u, bool am, bool ragged, bool one) {
+    if (!ragged) return am ? stream_kernel<true, false, false>(u) : stream_kernel<false, false, false>(u);
+    if (one) return am ? stream_kernel<true, true, true>(u) : stream_kernel<false, true, true>(u);
+    return am ? stream_kernel<true, true, false>(u) : stream_kernel<false, true, false>(u);
 }
 
-// Rows of the one-launch grid: as many as stay resident next to each other
-// with every chunk of a row (at most the record rows).
-int64_t onelaunch_rows(int64_t N, int64_t D, bool am = false) {
-    const int u = onelaunch_u(N, D);
-    const int64_t sp1 = ceil_div(D, 2048 * u);
-    int64_t R = resident_workgroups(onelaunch_kernel(u, am), 256) / sp1;
-    if (R > N) R = N;
-    if (R > kSplitMaxRows) R = kSplitMaxRows;
-    return R;
+// The one-launch form of a row: whole 16-byte vectors at D % 8 == 0 and
+// aligned bases, else the row's window, up to 7 elements longer.
+bool onelaunch_ragged(const void* x, const void* y, int64_t D) {
+    return !(D % 8 == 0 && aligned16(x) && aligned16(y));
 }
+int64_t onelaunch_len(int64_t D, bool ragged) { return ragged ? D + 7 : D; }
 
 // The one-launch grid: `splits` chunks per row, R row slots (a multiple of
 // kXcds, so that chunk_of keeps each slot's chunks on one XCD; slots past
 // N - 1 exit at once), 1-D.  `local`: whether polls start on the L2 copy.
 struct OneLaunchGrid {
-    int splits, R, local;
+    int u, splits, R, local;
+    bool one;
     unsigned blocks() const { return static_cast<unsigned>(splits) * static_cast<unsigned>(R); }
 };
-OneLaunchGrid onelaunch_grid(int64_t N, int64_t D, bool am) {
+OneLaunchGrid onelaunch_grid(int64_t N, int64_t D, bool am, bool ragged) {
     OneLaunchGrid g;
-    const int u = onelaunch_u(N, D);
-    g.splits = static_cast<int>(ceil_div(D, 2048 * u));
+    const int64_t len = onelaunch_len(D, ragged);
+    g.u = onelaunch_u(N, len);
+    g.splits = static_cast<int>(ceil_div(len, 2048 * g.u));
     // row slots that stay resident next to each other (at most the records;
     // at least 20 = 1280 resident workgroups / 64 chunks)
-    int64_t cap = resident_workgroups(onelaunch_kernel(u, am), 256) / g.splits;
-    if (cap > kSplitMaxRows) cap = kSplitMaxRows;
+    auto slots = [&](bool one) {
+        const int64_t cap = resident_workgroups(onelaunch_kernel(g.u, am, ragged, one), 256) / g.splits;
+        return cap < kSplitMaxRows ? cap : int64_t{kSplitMaxRows};
+    };
     // every row in one round when a whole number of groups of that many
     // slots fits (slots past N - 1 idle), else the largest whole number of
     // groups that does (rows in rounds)
-    const int64_t up = ceil_div(N < cap ? N : cap, kXcds) * kXcds;
-    g.R = static_cast<int>(up <= cap ? up : cap / kXcds * kXcds);
+    const int64_t all = ceil_div(N < kSplitMaxRows ? N : kSplitMaxRows, kXcds) * kXcds;
+    g.one = ragged && N <= all && all <= slots(true);
+    if (g.one) {
+        g.R = static_cast<int>(all);
+    } else {
+        const int64_t cap = slots(false);
+        const int64_t up = ceil_div(N < cap ? N : cap, kXcds) * kXcds;
+        g.R = static_cast<int>(up <= cap ? up : cap / kXcds * kXcds);
+    }
     g.local = exchange_test_mode().load() == 0 ? 1 : 0;
     return g;
 }
 
 // Whether [N, D] runs as the one-launch form given row records: a split or
-// kStream shape, aligned rows, y != x (the fallback re-reads x), at most 64
-// chunks per row.
+// kStream shape, y != x (the fallback re-reads x), rows of x and y with the
+// same window, at most 64 chunks per row.
 bool onelaunch_ok(const void* x, const void* y, int64_t N, int64_t D, bool am = false) {
     int64_t splits, chunk;
     if (!MI_SOFTMAX_ONEPASS || plan(N, D, splits, chunk) == Plan::kRow) return false;
-    return D % 8 == 0 && aligned16(x) && aligned16(y) && x != y &&
-           ceil_div(D, 2048 * onelaunch_u(N, D)) <= kOnePassMaxSplits &&
-           onelaunch_rows(N, D, am) >= 1;
+    if (x == y || !same_window(x, y)) return false;
+    const bool ragged = onelaunch_ragged(x, y, D);
+    const int64_t len = onelaunch_len(D, ragged);
+    const int u = onelaunch_u(N, len);
+    const int64_t sp1 = ceil_div(len, 2048 * u);
+    return sp1 <= kOnePassMaxSplits &&
+           resident_workgroups(onelaunch_kernel(u, am, ragged, false), 256) / sp1 >= 1;
 }
 
-// Whether every row of x and of y has the same RowWindow: fp16-aligned bases
-// at the same offset from a 16-byte boundary.
-bool same_window(const void* x, const void* y) {
-    const auto a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(y);
-    return (a & 1) == 0 && ((a ^ b) & 15) == 0;
+// One launch of softmax_stream_kernel (onelaunch_ok holds).
+template <bool AM>
+int launch_stream(const half_t* x, half_t* y, unsigned char* rec, int32_t* out, int64_t N,
+                  int64_t D, hipStream_t s) {
+    const bool ragged = onelaunch_ragged(x, y, D);
+    const OneLaunchGrid g = onelaunch_grid(N, D, AM, ragged);
+    const dim3 gr(g.blocks()), b(256);
+#define MI_STREAM(UU, RR, ONE)                                                                  \
+    softmax_stream_kernel<UU, AM, RR, ONE><<<gr, b, 0, s>>>(x, y, rec, N, D, g_poll_limit.load(), \
+                                                            out, g.splits, g.R, g.local)
+    const bool large = g.u == kOnePassU;
+    if (!ragged) {
+        if (large) MI_STREAM(kOnePassU, false, false);
+        else MI_STREAM(kOnePassU / 2, false, false);
+    } else if (g.one) {
+        if (large) MI_STREAM(kOnePassU, true, true);
+        else MI_STREAM(kOnePassU / 2, true, true);
+    } else {
+        if (large) MI_STREAM(kOnePassU, true, false);
+        else MI_STREAM(kOnePassU / 2, true, false);
+    }
+#undef MI_STREAM
+    return launch_status();
 }
 
 int softmax_checked(const void* x, void* y, int64_t N, int64_t D, void* ws, int64_t ws_bytes,
@@ -992,7 +1026,13 @@ int softmax_checked(const void* x, void* y, int64_t N, int64_t D, void* ws, int6
     if (x != y && overlaps(x, bytes, y, bytes)) return MI_ERR_ALIASING;
     int64_t splits, chunk;
     const Plan p = plan(N, D, splits, chunk);
-    const bool onelaunch = layout != Ws::kPairs && onelaunch_ok(x, y, N, D);
+    bool onelaunch = layout != Ws::kPairs && onelaunch_ok(x, y, N, D);
+    // many long ragged rows need no workspace (a workgroup per row): the
+    // one-launch form only with a usable one
+    if (onelaunch && p == Plan::kStream && onelaunch_ragged(x, y, D) &&
+        (!ws || ws_bytes < kOnePassRegion || reinterpret_cast<uintptr_t>(ws) % 16 != 0 ||
+         overlaps(ws, kOnePassRegion, x, bytes) || overlaps(ws, kOnePassRegion, y, bytes)))
+        onelaunch = false;
     if (layout == Ws::kRecords && p == Plan::kTwoPass && !onelaunch)
         return MI_ERR_UNSUPPORTED;  // no pairs to fall back on (callers check onelaunch_ok)
     const int64_t need = p == Plan::kRow ? 0
@@ -1028,18 +1068,8 @@ int softmax_checked(const void* x, void* y, int64_t N, int64_t D, void* ws, int6
             softmax_row_kernel<1><<<dim3(static_cast<unsigned>(N)), dim3(threads), 0, s>>>(xh, yh, D);
         return launch_status();
     }
-    if (onelaunch) {
-        const int u = onelaunch_u(N, D);
-        const OneLaunchGrid g = onelaunch_grid(N, D, false);
-        auto* rec = static_cast<unsigned char*>(ws);
-        if (u == kOnePassU)
-            softmax_stream_kernel<kOnePassU, false><<<dim3(g.blocks()), dim3(256), 0, s>>>(
-                xh, yh, rec, N, D, g_poll_limit.load(), nullptr, g.splits, g.R, g.local);
-        else
-            softmax_stream_kernel<kOnePassU / 2, false><<<dim3(g.blocks()), dim3(256), 0, s>>>(
-                xh, yh, rec, N, D, g_poll_limit.load(), nullptr, g.splits, g.R, g.local);
-        return launch_status();
-    }
+    if (onelaunch)
+        return launch_stream<false>(xh, yh, static_cast<unsigned char*>(ws), nullptr, N, D, s);
     auto* part = reinterpret_cast<float*>(static_cast<unsigned char*>(ws) +
                                           (layout == Ws::kRecordsThenPairs ? kOnePassRegion : 0));
     const dim3 g(static_cast<unsigned>(splits), static_cast<unsigned>(N));
@@ -1049,6 +1079,12 @@ int softmax_checked(const void* x, void* y, int64_t N, int64_t D, void* ws, int6
         else
             softmax_partial_kernel<8, 1><<<g, dim3(256), 0, s>>>(xh, part, D, chunk);
         softmax_finish_kernel<8><<<g, dim3(256), 0, s>>>(xh, yh, part, D, chunk);
+    } else if (same_window(x, y)) {
+        if (split_tile(N, D) == 4096)
+            softmax_partial_kernel<8, 2, true><<<g, dim3(256), 0, s>>>(xh, part, D, chunk);
+        else
+            softmax_partial_kernel<8, 1, true><<<g, dim3(256), 0, s>>>(xh, part, D, chunk);
+        softmax_finish_kernel<8, true><<<g, dim3(256), 0, s>>>(xh, yh, part, D, chunk);
     } else {
         softmax_partial_kernel<1, 1><<<g, dim3(256), 0, s>>>(xh, part, D, chunk);
         softmax_finish_kernel<1><<<g, dim3(256), 0, s>>>(xh, yh, part, D, chunk);
@@ -1170,20 +1206,9 @@ extern "C" int mi_softmax_argmax_ws_f16(const void* logits, void* probs, int32_t
         return MI_ERR_ALIASING;
     auto* ws = static_cast<unsigned char*>(workspace);
     const hipStream_t s = mi::as_stream(stream);
-    if (mi::onelaunch_ok(logits, probs, N, V, true)) {
-        const int u = mi::onelaunch_u(N, V);
-        const mi::OneLaunchGrid g = mi::onelaunch_grid(N, V, true);
-        const auto* xh = static_cast<const mi::half_t*>(logits);
-        auto* yh = static_cast<mi::half_t*>(probs);
-        if (u == mi::kOnePassU)
-            mi::softmax_stream_kernel<mi::kOnePassU, true><<<dim3(g.blocks()), dim3(256), 0, s>>>(
-                xh, yh, ws, N, V, mi::g_poll_limit.load(), out, g.splits, g.R, g.local);
-        else
-            mi::softmax_stream_kernel<mi::kOnePassU / 2, true>
-                <<<dim3(g.blocks()), dim3(256), 0, s>>>(xh, yh, ws, N, V, mi::g_poll_limit.load(),
-                                                        out, g.splits, g.R, g.local);
-        return mi::launch_status();
-    }
+    if (mi::onelaunch_ok(logits, probs, N, V, true))
+        return mi::launch_stream<true>(static_cast<const mi::half_t*>(logits),
+                                       static_cast<mi::half_t*>(probs), ws, out, N, V, s);
     // separately: argmax first (in place, softmax would overwrite the logits)
     const int64_t sw = mi::workspace_bytes(N, V);
     unsigned char* aw = ws + kFusedRegion + sw;

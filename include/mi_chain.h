@@ -123,7 +123,10 @@ enum {
     MI_CHAIN_SAMPLE = 8          /* probs = softmax(logits), next_tokens = argmax(logits) */
 };
 
-/* Validates `d` against every stage up to last_stage (MI_ERR_* of
+/* (A run to MI_CHAIN_FINAL_NORM or beyond, whose buffers do not overlap, may
+ * issue the stages in another order or several in one launch: every output
+ * is as after the stages in their order.)
+ * Validates `d` against every stage up to last_stage (MI_ERR_* of
  * mi_kernels.h when a pointer or size is missing or out of range; nothing is
  * launched then), then enqueues the stages on `stream` (hipStream_t; NULL =
  * the null stream) and returns without synchronising.  Allocates nothing, so

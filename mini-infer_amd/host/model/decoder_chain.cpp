@@ -4,9 +4,11 @@
 #include "model/decoder_chain.h"
 
 #include <cmath>
+#include <initializer_list>
 #include <stdexcept>
 #include <string>
 
+#include "chain_step.h"
 #include "mi_kernels.h"
 
 namespace mini_infer {
@@ -131,6 +133,112 @@ bool DecoderChain::rope_kv_fused(hipStream_t s) const {
     return true;
 }
 
+// Whether no buffer that the chain writes shares memory with another of its
+// buffers, so that stages may run in another order than the chain's, or
+// together.  (act_out on gate or up, and probs on logits, are one stage's own
+// in-place forms.)  A caller may reuse one scratch buffer for several stages:
+// then the chain's order is what gives each its meaning.
+bool DecoderChain::buffers_apart() const {
+    const mi_chain_desc& d = d_;
+    struct Range {
+        uintptr_t begin, end;
+        bool written;
+        int in_place;  // buffers of one non-zero mark may coincide
+    };
+    Range r[64];
+    int n = 0;
+    bool fits = true;
+    auto put = [&](const void* p, std::initializer_list<int64_t> dims, bool written = false,
+                   int in_place = 0) {
+        int64_t bytes = 1;
+        for (int64_t f : dims)
+            if (f < 0 || __builtin_mul_overflow(bytes, f, &bytes) || bytes > (int64_t{1} << 62))
+                fits = false;
+        if (!fits || !p || bytes == 0) return;
+        const auto b = reinterpret_cast<uintptr_t>(p);
+        r[n++] = Range{b, b + static_cast<uintptr_t>(bytes), written, in_place};
+    };
+    const int64_t T = d.T, D = d.hidden_size, I = d.intermediate_size;
+    const int64_t qd = d.num_heads * d.head_dim, kd = d.num_kv_heads * d.head_dim;
+    put(d.ids, {T, 8});
+    put(d.positions, {T, 8});
+    put(d.embed, {d.vocab, D, 2});
+    for (const void* w : {d.input_norm, d.post_attn_norm, d.pre_ff_norm, d.post_ff_norm, d.final_norm})
+        put(w, {D, 2});
+    put(d.q_norm, {d.head_dim, 2});
+    put(d.k_norm, {d.head_dim, 2});
+    put(d.q_bias, {qd, 2});
+    put(d.k_bias, {kd, 2});
+    put(d.v_bias, {kd, 2});
+    for (const mi_chain_kv_segment& g : segs_) {
+        if (n > 40) return false;  // more segments than r has room for
+        put(g.block_table, {g.B, g.max_blocks_per_seq, 4});
+        put(g.seq_len, {g.B, 4});
+        put(g.start_pos, {g.B, 4});
+    }
+    put(d.hidden, {T, D, 2}, true);
+    put(d.normed, {T, D, 2}, true);
+    put(d.post_normed, {T, D, 2}, true);
+    put(d.final_normed, {T, D, 2}, true);
+    put(d.attn_out, {T, D, 2}, d.double_norm != 0);
+    put(d.mlp_out, {T, D, 2}, d.double_norm != 0);
+    put(d.q, {T, qd, 2}, true);
+    put(d.k, {T, kd, 2}, true);
+    put(d.v, {T, kd, 2});
+    if (!segs_.empty())
+        for (const void* c : {d.k_cache, d.v_cache})
+            put(c, {d.layer + 1, d.num_blocks, kd, d.block_size, 2}, true);
+    put(d.gate, {T, I, 2}, false, 1);
+    put(d.up, {T, I, 2}, false, 1);
+    put(d.act_out, {T, I, 2}, true, 1);
+    if (last_ >= MI_CHAIN_SAMPLE) {
+        put(d.logits, {d.logit_rows, d.vocab, 2}, false, 2);
+        put(d.probs, {d.logit_rows, d.vocab, 2}, true, 2);
+        put(d.next_tokens, {d.logit_rows, 4}, true);
+        put(d.sample_ws, {d.sample_ws_bytes}, true);
+    }
+    if (!fits) return false;
+    for (int i = 0; i < n; ++i) {
+        if (!r[i].written) continue;
+        for (int j = 0; j < n; ++j)
+            if (j != i && r[i].begin < r[j].end && r[j].begin < r[i].end &&
+                !(r[i].in_place && r[i].in_place == r[j].in_place && r[i].begin == r[j].begin))
+                return false;
+    }
+    return true;
+}
+
+// Stages 1-2, 5 and 7 in one launch (chain_step.h), which keeps the residual
+// stream in registers between them.  False (nothing launched) for shapes it
+// does not take.
+bool DecoderChain::rows_fused(hipStream_t s) const {
+    const mi_chain_desc& d = d_;
+    mi::ChainRows c{};
+    c.ids = d.ids;
+    c.table = d.embed;
+    c.hidden = d.hidden;
+    c.normed = d.normed;
+    c.post_normed = d.post_normed;
+    c.final_normed = d.final_normed;
+    c.attn = d.attn_out;
+    c.mlp = d.mlp_out;
+    c.w_in = d.input_norm;
+    c.w_post = d.double_norm ? d.pre_ff_norm : d.post_attn_norm;
+    c.w_final = d.final_norm;
+    c.w_attn = d.double_norm ? d.post_attn_norm : nullptr;
+    c.w_mlp = d.double_norm ? d.post_ff_norm : nullptr;
+    c.T = d.T;
+    c.D = d.hidden_size;
+    c.vocab = d.vocab;
+    c.scale = d.embed_scale ? std::sqrt(static_cast<float>(d.hidden_size)) : 1.0f;
+    c.eps = d.rms_eps;
+    c.add_one = d.norm_add_one;
+    const int st = mi::chain_rows(c, sv(s));
+    if (st == MI_ERR_UNSUPPORTED) return false;
+    check(st, "gather + residual adds + norms");
+    return true;
+}
+
 void DecoderChain::run(hipStream_t s, DecoderChainHooks* hooks) const {
     DecoderChainHooks none;
     DecoderChainHooks& h = hooks ? *hooks : none;
@@ -151,9 +259,13 @@ void DecoderChain::run(hipStream_t s, DecoderChainHooks* hooks) const {
             check(mi_scale_inplace_f16(d.hidden, scale, T * D, sv(s)), "embed scale");
         return;
     }
-    check(mi_embedding_rmsnorm_f16(d.ids, d.embed, d.hidden, d.input_norm, d.normed, T, D,
-                                   d.vocab, scale, eps, add1, sv(s)),
-          "gather + input norm");
+    // without hooks every GEMM output is there already, so stages 1-2, 5 and 7
+    // need not wait for one another: one launch for all three
+    const bool rows = !hooks && last_ >= MI_CHAIN_FINAL_NORM && buffers_apart() && rows_fused(s);
+    if (!rows)
+        check(mi_embedding_rmsnorm_f16(d.ids, d.embed, d.hidden, d.input_norm, d.normed, T, D,
+                                       d.vocab, scale, eps, add1, sv(s)),
+              "gather + input norm");
     if (last_ == MI_CHAIN_INPUT_NORM) return;
 
     // 3. QKV GEMMs, then Q/K-norm + RoPE in one in-place pass
@@ -216,7 +328,9 @@ void DecoderChain::run(hipStream_t s, DecoderChainHooks* hooks) const {
     // 5. attention + O GEMM, then residual add fused with the post-attention
     //    norm (transformer_model.cpp:591-603, 605-625)
     h.attention(d, s);
-    if (d.double_norm) {
+    if (rows) {
+        // done with the gather above
+    } else if (d.double_norm) {
         check(mi_rmsnorm_f16(d.attn_out, d.post_attn_norm, d.attn_out, T, D, eps, add1, sv(s)),
               "post-attn norm");
         check(mi_fused_add_rmsnorm_f16(d.attn_out, d.hidden, d.pre_ff_norm, d.post_normed, T, D,
@@ -242,12 +356,14 @@ void DecoderChain::run(hipStream_t s, DecoderChainHooks* hooks) const {
     //    (transformer_model.cpp:627-660; the next layer's input norm in a
     //    deeper model)
     h.down(d, s);
-    if (d.double_norm)
-        check(mi_rmsnorm_f16(d.mlp_out, d.post_ff_norm, d.mlp_out, T, D, eps, add1, sv(s)),
-              "post-ff norm");
-    check(mi_fused_add_rmsnorm_f16(d.mlp_out, d.hidden, d.final_norm, d.final_normed, T, D, eps,
-                                   add1, sv(s)),
-          "residual add + final norm");
+    if (!rows) {
+        if (d.double_norm)
+            check(mi_rmsnorm_f16(d.mlp_out, d.post_ff_norm, d.mlp_out, T, D, eps, add1, sv(s)),
+                  "post-ff norm");
+        check(mi_fused_add_rmsnorm_f16(d.mlp_out, d.hidden, d.final_norm, d.final_normed, T, D, eps,
+                                       add1, sv(s)),
+              "residual add + final norm");
+    }
     if (last_ == MI_CHAIN_FINAL_NORM) return;
 
     // 8. LM head, then the sampling step: softmax and greedy argmax of the

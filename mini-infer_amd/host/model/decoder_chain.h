@@ -48,6 +48,8 @@ public:
 private:
     void validate_() const;
     bool rope_kv_fused(hipStream_t stream) const;
+    bool buffers_apart() const;
+    bool rows_fused(hipStream_t stream) const;
 
     mi_chain_desc d_;
     int last_;

@@ -1,0 +1,89 @@
+"""GPU parity of the chain's row-wise stages in one launch (hookless chains that
+run to the final norm) against the same stages issued one by one through the C
+ABI: the residual stream bit for bit without the blocks' output norms, and every
+norm within one fp16 ulp of the separate kernel's (the two may sum the squares
+of a row in another order).  A caller that reuses one scratch buffer for several
+stages gets the sequential result."""
+import numpy as np
+import pytest
+
+import mi_chain
+
+pytestmark = pytest.mark.gpu
+Stage = mi_chain.Stage
+
+
+def _work(dev, D, double, seed=3, n_decode=5, **kw):
+    return mi_chain.Workload(dev, seed=seed, n_decode=n_decode, prefills=(3,), logit_rows=2,
+                             hidden_size=D, intermediate_size=64, num_heads=2, num_kv_heads=1,
+                             head_dim=16, vocab=200, double_norm=int(double),
+                             norm_add_one=int(double), embed_scale=int(double), **kw)
+
+
+def _one_by_one(mk, w):
+    """The stages as separate calls; returns the tensors by the chain's names."""
+    t, c = w.t, w.cfg
+    add1, eps = bool(c["norm_add_one"]), c["rms_eps"]
+    scale = float(np.sqrt(np.float32(c["hidden_size"]))) if c["embed_scale"] else 1.0
+    attn, mlp = t["attn_out"].clone(), t["mlp_out"].clone()
+    hidden, normed = mk.embedding_rmsnorm(t["ids"], t["embed"], t["input_norm"], scale=scale,
+                                          eps=eps, add_one=add1)
+    if c["double_norm"]:
+        mk.rmsnorm(attn, t["post_attn_norm"], y=attn, eps=eps, add_one=add1)
+        mk.rmsnorm(mlp, t["post_ff_norm"], y=mlp, eps=eps, add_one=add1)
+    post = mk.fused_add_rmsnorm(attn, hidden, t["pre_ff_norm" if c["double_norm"] else
+                                                "post_attn_norm"], eps=eps, add_one=add1)
+    fin = mk.fused_add_rmsnorm(mlp, hidden, t["final_norm"], eps=eps, add_one=add1)
+    return dict(hidden=hidden, normed=normed, post_normed=post, final_normed=fin, attn_out=attn,
+                mlp_out=mlp)
+
+
+def _ulps(a, b):
+    """Largest distance in fp16 values between a and b."""
+    def order(x):
+        i = x.cpu().numpy().view(np.int16).astype(np.int32)
+        return np.where(i < 0, -32768 - i, i)
+    return int(np.abs(order(a) - order(b)).max())
+
+
+# one vector, the edges of the vectors per lane, the longest row, and rows the
+# single launch does not take
+@pytest.mark.parametrize("D", [8, 2040, 2048, 2056, 4104, 6152, 8192, 8200, 100])
+@pytest.mark.parametrize("double", [False, True])
+def test_rows_in_one_launch(mk, dev, D, double):
+    import torch
+    print(f"[case] chain rows D={D} double={double}", flush=True)
+    w = _work(dev, D, double)
+    w.t["ids"][2] = -1    # zero rows
+    w.t["ids"][3] = 200
+    want = _one_by_one(mk, w)
+    w.run(Stage.FINAL_NORM)
+    torch.cuda.synchronize()
+    for n, ref in want.items():
+        exact = not double and n in ("hidden", "attn_out", "mlp_out")
+        # DOUBLE: a norm one ulp off moves the residual, and the norm of that
+        far = 0 if exact else 1 if not double else 3
+        got = w.t[n]
+        if double and n == "hidden":  # cancelling sums: an absolute bound, an ulp of the addends
+            assert (got.float() - ref.float()).abs().max() <= 2 ** -10 * 2 * max(
+                w.t["attn_out"].abs().max().item(), w.t["mlp_out"].abs().max().item(), 1.0), n
+        elif double and n in ("post_normed", "final_normed"):
+            d = (got.float() - ref.float()).abs()
+            assert (d <= 2 ** -9 * (ref.float().abs() + 1)).all(), n
+        else:
+            assert _ulps(got, ref) <= far, n
+
+
+@pytest.mark.parametrize("double", [False, True])
+def test_shared_scratch_keeps_the_order(mk, dev, double):
+    """normed, post_normed and final_normed one buffer; mlp_out normalised into it."""
+    import torch
+    print(f"[case] chain rows, one scratch buffer, double={double}", flush=True)
+    w = _work(dev, 256, double)
+    want = _one_by_one(mk, w)
+    w.t["post_normed"] = w.t["final_normed"] = w.t["normed"]
+    w.desc, w.keep = mi_chain.make_desc(w.shapes, w.t, w.segments)
+    w.run(Stage.FINAL_NORM)
+    torch.cuda.synchronize()
+    assert torch.equal(w.t["hidden"], want["hidden"])
+    assert torch.equal(w.t["final_normed"], want["final_normed"])

@@ -6,6 +6,8 @@
 
 #include <stdint.h>
 
+#include "mi_kernels.h"
+
 namespace mi {
 
 // hidden = table[ids] (* scale); normed = rmsnorm(hidden, w_in);
@@ -29,5 +31,14 @@ struct ChainRows {
 // caller then issues the stages one by one.  The buffers must not overlap
 // one another (the caller checks).
 int chain_rows(const ChainRows& r, void* stream);
+
+// mi_rope_kv_scatter_f16 / mi_qk_norm_rope_kv_scatter_f16 (rope.hip), `wide` with
+// up to 768 (head, slice) units per token.
+int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const void* k_bias,
+                   const void* v_bias, const void* q_weight, const void* k_weight, float eps,
+                   int add_one, const int64_t* positions, const float* inv_freq_host, int64_t T,
+                   int64_t Hq, int64_t Hkv, int64_t head_dim, void* k_cache, void* v_cache,
+                   int64_t layer, int64_t num_blocks, int64_t block_size,
+                   const mi_kv_segment* segments, int num_segments, bool wide, void* stream);
 
 }  // namespace mi

@@ -27,64 +27,16 @@
 //   units, so with 2 tokens per workgroup each lane has two units in flight.
 #include <math.h>
 
+#include <algorithm>
+
+#include "chain_step.h"
 #include "mi_device.h"
 #include "mi_host.h"
-#include "rope_sincos.h"
-
-// Stores of the in-place RoPE and fused Q/K-norm + RoPE kernels: write-through
-// ("nt sc1", st8_stream_wt) measured 1-3 points faster than plain non-temporal.
-#ifndef MI_WT_ROPE
-#define MI_WT_ROPE 1
-#endif
-#ifndef MI_WT_QKNR
-#define MI_WT_QKNR 1
-#endif
+#include "rope_kv.h"
+#include "rope_math.h"
 
 namespace mi {
 namespace {
-
-constexpr int kMaxHalf = 256;  // head_dim <= 512
-
-// LDS position of element i of a half-row of n entries (n a multiple of 8),
-// for lanes that each read the 8 entries c*8 .. c*8+7 as two 16-byte LDS
-// reads: entries 0-3 of every lane's group sit together in the first n/2
-// slots and entries 4-7 in the second, so lane c reads slots 4c .. 4c+3 and
-// n/2 + 4c .. n/2 + 4c+3.  Eight consecutive lanes then cover 32 distinct
-// banks per read; with the plain layout (lane c at 8c) lanes c and c+4 fall
-// on the same banks and every read took a second pass (rocprof
-// LdsBankConflict 0.97 conflicts per access).
-__device__ __forceinline__ int quad_split(int i, int n) {
-    return ((i & 4) ? (n >> 1) : 0) + ((i >> 3) << 2) + (i & 3);
-}
-
-// Host-computed inverse frequencies travel by value in the kernel arguments.
-struct InvFreq {
-    float v[kMaxHalf];
-};
-
-// fp16 cos/sin of an fp32 angle, equal to half(RN32(exact)) (see file header).
-// |ang| <= 2^20: the fp32 Cody-Waite form, re-evaluated in fp64 when a value
-// lies within rope_guard_width of an fp16 rounding boundary; larger angles
-// (positions beyond 2^20 / inv_freq) go straight to the fp64 form
-// (rope_sincos_any: Cody-Waite to 2^24, Payne-Hanek above), which covers
-// every fp32 angle -- so every int64 position -- with no range limit.
-__device__ __forceinline__ bool near_half_boundary(float v) {
-    const float d = rope_guard_width(v);
-    return to_half(v - d) != to_half(v + d);
-}
-
-__device__ __forceinline__ void cos_sin_half(float ang, half_t& hc, half_t& hs) {
-    float s, c;
-    rope_sincos_f32(ang, &s, &c);
-    if (!rope_sincos_f32_ok(ang) || near_half_boundary(c) || near_half_boundary(s)) {
-        double sd, cd;
-        rope_sincos_any(ang, &sd, &cd);
-        c = static_cast<float>(cd);
-        s = static_cast<float>(sd);
-    }
-    hc = to_half(c);
-    hs = to_half(s);
-}
 
 template <int VEC>
 struct HVec;
@@ -730,49 +682,36 @@ int launch_qk_norm_rope(half_t* q, int64_t Hq, half_t* k, int64_t Hkv, const hal
 
 // ---------------------------------------------------------------------------
 // RoPE of Q and K in place, with K's rotated rows and V's rows also written
-// into the paged KV cache, one workgroup per token: the attention
+// into the paged KV cache, one workgroup per token (rope_kv.h): the attention
 // pre-processing of a model without Q/K norm (Qwen2: with the q/k/v_proj
-// bias) -- the reference's RoPE pair and two launch_paged_kv_scatter calls
-// per sequence group (src/layers/attention.cpp:779-780, :823-846) in one
-// launch.  K is not re-read for the scatter.  256 lanes take the (head,
-// slice) units of the token as rope_kernel does, and lane j also carries V's
-// 16-byte vector j (a 256-lane workgroup keeps rope_kernel's residency of
-// 8 workgroups per CU; 64 extra V lanes made it 6: 0.4-0.9 us slower at
-// Qwen2.5's shape, T = 6064).  Cache rows are written through to memory ("nt sc1"), as the
-// scatter kernel writes them.  The token's cache slot comes from the segment
-// holding it (workgroup-uniform scalar lookups issued with the data loads).
+// bias) or with it (Gemma 3) -- the reference's RoPE pair and two
+// launch_paged_kv_scatter calls per sequence group
+// (src/layers/attention.cpp:779-780, :823-846) in one launch.  K is not re-read
+// for the scatter.  256 lanes whatever the token's units (64 extra V lanes made
+// rope_kernel's residency of 8 workgroups per CU 6: 0.4-0.9 us slower at
+// Qwen2.5's shape, T = 6064).
 // ---------------------------------------------------------------------------
-constexpr int kMaxKvSegs = 8;
-struct KvSegs {
-    int n;
-    int64_t off[kMaxKvSegs], B[kMaxKvSegs], S[kMaxKvSegs], mb[kMaxKvSegs];
-    const int* bt[kMaxKvSegs];
-    const int* sl[kMaxKvSegs];
-    const int* sp[kMaxKvSegs];
-};
+template <bool BIAS, bool NORM, int CPH, int P, int NF, int LPT>
+__global__ __launch_bounds__(256) void rope_kv_scatter_kernel(RopeKv a, InvFreqN<NF> inv,
+                                                              int64_t T) {
+    __shared__ __attribute__((aligned(16))) float cs[(256 / LPT) * 2 * kMaxHalf];
+    rope_kv_block<BIAS, NORM, CPH, P, LPT>(a, inv.v, blockIdx.x, T, cs);
+}
 
-// NORM (Gemma 3): the per-head Q/K RMSNorm of qk_norm_rope_kernel first --
-// the CPH = hd/16 lanes of a head sum their squares by DPP, the normalised
-// value is rounded to fp16 where the reference stores it, and the rotation
-// takes it from registers.  CPH = head_dim / 16 at compile time (shifts for
-// the lane -> (head, slice) split: 0.3-0.4 us less than CPH = 0 at Qwen2.5's
-// shapes); CPH = 0: head_dim known at run time (no norm).
-// SEG = false: RoPE (+ bias or norm) alone -- no cache segment, no V, no
-// cache stores (a distinct kernel in traces, with none of that code).
+// RoPE of Q and K in place, one workgroup per token, no cache: NORM (Gemma 3)
+// the per-head Q/K RMSNorm first, BIAS the projection bias, as rope_kv_token
+// forms them.  CPH = head_dim / 16 at compile time, or 0.
 // `inv` is the first parameter: it sits at offset 0 of the kernel-argument
-// block, which the SEG = false form reads directly (below).
-template <bool BIAS, bool NORM, int CPH, bool SEG = true>
-__global__ __launch_bounds__(256) void rope_kv_kernel(InvFreq inv, half_t* q, half_t* k,
-                                                       const half_t* v, int Hq, int Hkv, int hd,
-                                                       const int64_t* __restrict__ positions,
-                                                       const half_t* __restrict__ bq,
-                                                       const half_t* __restrict__ bk,
-                                                       const half_t* __restrict__ bv,
-                                                       const half_t* __restrict__ wq,
-                                                       const half_t* __restrict__ wk, float eps,
-                                                       float w_bias, half_t* k_cache,
-                                                       half_t* v_cache, KvSegs sg, int64_t layer,
-                                                       int64_t num_blocks, int64_t bs) {
+// block, which the kernel reads directly (below).
+template <bool BIAS, bool NORM, int CPH>
+__global__ __launch_bounds__(256) void rope_token_kernel(InvFreq inv, half_t* q, half_t* k, int Hq,
+                                                         int Hkv, int hd,
+                                                         const int64_t* __restrict__ positions,
+                                                         const half_t* __restrict__ bq,
+                                                         const half_t* __restrict__ bk,
+                                                         const half_t* __restrict__ wq,
+                                                         const half_t* __restrict__ wk, float eps,
+                                                         float w_bias) {
     static_assert(!(BIAS && NORM), "no model adds a QKV bias before a Q/K norm");
     static_assert(!NORM || (CPH >= 1 && CPH <= 32), "the norm needs head_dim / 16 at compile time");
     __shared__ __attribute__((aligned(16))) float cs[2 * kMaxHalf];
@@ -785,14 +724,14 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(InvFreq inv, half_t* q, ha
     h8 x1 = h8(0), x2 = h8(0), b1 = h8(0), b2 = h8(0);
     half_t* hp = nullptr;
     int h = 0, c = 0;
-    // SEG = false: this lane's inverse frequency read from the kernel-argument
-    // block ahead of the data, and the data loads straight-line (an idle lane
-    // reads head 0's first slice and stores nothing), so the sincos below
-    // waits for that one load only -- not, as when the compiler sinks the
-    // argument load behind the data (the counter is in order), for every
-    // data load first.  Q/K-norm + RoPE at T = 6064: 18.2 -> ... us.
+    // This lane's inverse frequency read from the kernel-argument block ahead
+    // of the data, and the data loads straight-line (an idle lane reads head
+    // 0's first slice and stores nothing), so the sincos below waits for that
+    // one load only -- not, as when the compiler sinks the argument load behind
+    // the data (the counter is in order), for every data load first.  Q/K-norm
+    // + RoPE at T = 6064: 17.9 -> 17.15 us.
     float inv_l = 0.0f;
-    if constexpr (!SEG) {
+    {
         const float* ip =
             reinterpret_cast<const float*>(
                 reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr())) +
@@ -823,61 +762,11 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(InvFreq inv, half_t* q, ha
         // the inverse frequency has landed once only the loads after it remain
         asm volatile("s_waitcnt vmcnt(%0)" : : "n"((BIAS || NORM) ? 4 : 2) : "memory");
         asm volatile("" : "+v"(inv_l));
-    } else if (tid < units) {
-        if constexpr (CPH != 0) {
-            h = tid / CPH;
-            c = tid & (CPH - 1);
-        } else {
-            h = small_div(tid, 1.0f / static_cast<float>(cph));  // units < 2^22: exact
-            c = tid - h * cph;
-        }
-        hp = h < Hq ? q + (tok * Hq + h) * (2 * half) : k + (tok * Hkv + (h - Hq)) * (2 * half);
-        x1 = ld8_stream(hp + c * 8);
-        x2 = ld8_stream(hp + half + c * 8);
-        if constexpr (BIAS) {  // a few KB every token re-reads: plain loads
-            const half_t* bp = h < Hq ? bq + h * (2 * half) : bk + (h - Hq) * (2 * half);
-            b1 = ld8(bp + c * 8);
-            b2 = ld8(bp + half + c * 8);
-        }
-        if constexpr (NORM) {  // the norm weights [hd], as the biases
-            const half_t* wp = h < Hq ? wq : wk;
-            b1 = ld8(wp + c * 8);
-            b2 = ld8(wp + half + c * 8);
-        }
-    }
-    const int vj = tid;  // V vector of this lane (Hkv * hd / 8 <= 256)
-    const bool vlane = SEG && sg.n > 0 && vj < Hkv * (half >> 2);  // no segment: V not read
-    h8 vv = h8(0), vb = h8(0);
-    if (vlane) {
-        vv = ld8_stream(v + tok * Hkv * (2 * half) + vj * 8);
-        if constexpr (BIAS) vb = ld8(bv + vj * 8);
     }
     const float fpos = static_cast<float>(positions[tok]);
-    // the token's cache row (-1: not scattered), as launch_paged_kv_scatter
-    // places it (src/kernels/model_utils_kernel.cu:108-164); looked up after
-    // the data loads are issued, so its dependent scalar loads overlap them
-    // (token indices and segment sizes fit 32 bits: T <= kMaxGridX)
-    int64_t dst_base = -1;
-    const int itok = static_cast<int>(tok);
-    for (int i = 0; SEG && i < sg.n; ++i) {
-        const int r = itok - static_cast<int>(sg.off[i]);
-        const int S = static_cast<int>(sg.S[i]);
-        if (r < 0 || r >= static_cast<int>(sg.B[i]) * S) continue;
-        const int b = static_cast<int>(static_cast<uint32_t>(r) / static_cast<uint32_t>(S));
-        const int64_t pos = static_cast<int64_t>(sg.sp[i][b]) + (r - b * S);
-        const int len = sg.sl[i][b];
-        if (pos < 0 || pos >= len) break;
-        // 0 <= pos < len and bs < 2^31: 32-bit division
-        const int blk = static_cast<int>(static_cast<uint32_t>(pos) / static_cast<uint32_t>(bs));
-        if (blk >= sg.mb[i]) break;
-        const int64_t phys = sg.bt[i][b * sg.mb[i] + blk];
-        if (phys >= 0 && phys < num_blocks)
-            dst_base = ((layer * num_blocks + phys) * Hkv * bs + (pos - blk * bs)) * (2 * half);
-        break;
-    }
     if (tid < half) {
         half_t hc, hs;
-        cos_sin_half(fpos * (SEG ? inv.v[tid] : inv_l), hc, hs);
+        cos_sin_half(fpos * inv_l, hc, hs);
         const int li = quad_split(tid, half);
         cs[li] = (float)hc;
         cs[kMaxHalf + li] = (float)hs;
@@ -916,25 +805,6 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(InvFreq inv, half_t* q, ha
         }
         st8_out<NORM ? MI_WT_QKNR : MI_WT_ROPE>(hp + c * 8, y1);
         st8_out<NORM ? MI_WT_QKNR : MI_WT_ROPE>(hp + half + c * 8, y2);
-        if (SEG && h >= Hq && dst_base >= 0) {
-            half_t* kd = k_cache + dst_base + static_cast<int64_t>(h - Hq) * bs * (2 * half);
-            st8_stream_wt(kd + c * 8, y1);
-            st8_stream_wt(kd + half + c * 8, y2);
-        }
-    }
-    if (SEG && vlane && dst_base >= 0) {
-        if constexpr (BIAS) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) vv[e] = to_half((float)vv[e] + (float)vb[e]);
-        }
-        const int per_head = half >> 2;
-        int vh;
-        if constexpr (CPH != 0)
-            vh = vj / (CPH * 2);
-        else
-            vh = small_div(vj, 1.0f / static_cast<float>(per_head));
-        const int vd = (vj - vh * per_head) * 8;
-        st8_stream_wt(v_cache + dst_base + static_cast<int64_t>(vh) * bs * (2 * half) + vd, vv);
     }
 }
 
@@ -952,12 +822,12 @@ __global__ __launch_bounds__(256) void rope_kv_kernel(InvFreq inv, half_t* q, ha
 // it.  On the same access pattern with no arithmetic (floors.hip,
 // mi_floor_rope_inplace), 4 tokens per workgroup with paced non-temporal
 // stores move 67 MB in place in 11.5 us, one token per workgroup (the
-// rope_kv_kernel shape) in 12.3 us.
-// The arithmetic is rope_kv_kernel's, operation for operation -- the bias add
+// rope_token_kernel shape) in 12.3 us.
+// The arithmetic is rope_token_kernel's, operation for operation -- the bias add
 // rounded to fp16, the Q/K norm's per-lane sum over (x1[e], x2[e]) pairs and
 // its DPP sum over the X lanes of a half head (the first-half and second-half
 // lanes each form the same sum), the rotation with one rounding to fp32 -- so
-// the outputs equal rope_kv_kernel's bit for bit.  Only plain RoPE takes this
+// the outputs equal rope_token_kernel's bit for bit.  Only plain RoPE takes this
 // kernel by default: with the bias (Qwen2's q/k_proj bias) it measured 21.1
 // against 18.3 us at T = 6064, with the Q/K norm 19.7-21.0 against 18.0 us
 // (MI_ROPE_ROWS_BIAS / MI_ROPE_ROWS_NORM switch them on).
@@ -1181,7 +1051,7 @@ void rope_rows_go(int tpw, dim3 g, hipStream_t s, const InvFreq& inv, half_t* q,
 // for R = 3, 4) whose grid fits 4 workgroups per CU -- one resident round
 // with every CU equally loaded -- else the most.  Measured at Qwen2.5's
 // 28 + 4 heads of 128 (R = 2): T = 4096, 4 tokens (1024 workgroups) 11.7 us
-// against 12.6 us for rope_kv_kernel's one token per workgroup; T = 6064,
+// against 12.6 us for rope_token_kernel's one token per workgroup; T = 6064,
 // 6 tokens (1011 workgroups) 17.5 us against 17.8 us, while 4 tokens
 // (1516 workgroups, an uneven round) took 20.1 us.
 int rope_rows_tpw(int64_t T, int R) {
@@ -1194,7 +1064,7 @@ int rope_rows_tpw(int64_t T, int R) {
 }
 
 // rope_rows_kernel for head_dim 64 / 128 / 256 and up to 1024 vectors per
-// token; MI_ERR_UNSUPPORTED otherwise (the caller takes rope_kv_kernel).
+// token; MI_ERR_UNSUPPORTED otherwise (the caller takes rope_token_kernel).
 int rope_qk_rows(half_t* q, half_t* k, const half_t* bq, const half_t* bk,
                  const int64_t* positions, const InvFreq& inv, int64_t T, int64_t Hq,
                  int64_t Hkv, int64_t head_dim, hipStream_t s, const half_t* wq,
@@ -1245,8 +1115,8 @@ int rope_qk_rows(half_t* q, half_t* k, const half_t* bq, const half_t* bk,
     return launch_status();
 }
 
-// RoPE of Q and K from positions (+ the Q/K bias, or the Q/K norm) through rope_kv_kernel
-// with no segment: one token per 256-lane workgroup, head_dim's lane split at
+// RoPE of Q and K from positions (+ the Q/K bias, or the Q/K norm) through
+// rope_token_kernel: one token per 256-lane workgroup, head_dim's lane split at
 // compile time.  Against rope_kernel at T = 6064 (plain / with the bias):
 // 256 (head, slice) units per token 17.9 -> 17.6 / 19.2 -> 18.7 us (at T =
 // 4096: 12.8 -> 12.5 us), 192 units 15.1 -> 13.7 / 16.2 -> 14.5, 144 units
@@ -1280,31 +1150,27 @@ int rope_qk_one_token(half_t* q, half_t* k, const half_t* bq, const half_t* bk,
         (bq && !aligned16(bq)) || (bk && Hkv > 0 && !aligned16(bk)) ||
         (norm && (!aligned16(wq) || (Hkv > 0 && !aligned16(wk)))))
         return MI_ERR_UNSUPPORTED;
-    KvSegs sg{};
-    sg.n = 0;
     const dim3 g(static_cast<unsigned>(T)), b(256);
     const int hq = static_cast<int>(Hq), hk = static_cast<int>(Hkv), d = static_cast<int>(head_dim);
-#define MI_RQ_ARGS                                                                          \
-    inv, q, k, k, hq, hk, d, positions, bq, bk, nullptr, wq, wk, eps, w_bias, nullptr, nullptr, \
-        sg, 0, 0, 1
+#define MI_RQ_ARGS inv, q, k, hq, hk, d, positions, bq, bk, wq, wk, eps, w_bias
 #define MI_RQ_CPH(BIAS)                                                                     \
     switch (head_dim / 16) {                                                                \
-        case 1: rope_kv_kernel<BIAS, false, 1, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
-        case 2: rope_kv_kernel<BIAS, false, 2, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
-        case 4: rope_kv_kernel<BIAS, false, 4, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
-        case 8: rope_kv_kernel<BIAS, false, 8, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
-        case 16: rope_kv_kernel<BIAS, false, 16, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break; \
-        case 32: rope_kv_kernel<BIAS, false, 32, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break; \
-        default: rope_kv_kernel<BIAS, false, 0, false><<<g, b, 0, s>>>(MI_RQ_ARGS);         \
+        case 1: rope_token_kernel<BIAS, false, 1><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
+        case 2: rope_token_kernel<BIAS, false, 2><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
+        case 4: rope_token_kernel<BIAS, false, 4><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
+        case 8: rope_token_kernel<BIAS, false, 8><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
+        case 16: rope_token_kernel<BIAS, false, 16><<<g, b, 0, s>>>(MI_RQ_ARGS); break; \
+        case 32: rope_token_kernel<BIAS, false, 32><<<g, b, 0, s>>>(MI_RQ_ARGS); break; \
+        default: rope_token_kernel<BIAS, false, 0><<<g, b, 0, s>>>(MI_RQ_ARGS);         \
     }
     if (norm) {
         switch (head_dim / 16) {
-            case 1: rope_kv_kernel<false, true, 1, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
-            case 2: rope_kv_kernel<false, true, 2, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
-            case 4: rope_kv_kernel<false, true, 4, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
-            case 8: rope_kv_kernel<false, true, 8, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
-            case 16: rope_kv_kernel<false, true, 16, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
-            case 32: rope_kv_kernel<false, true, 32, false><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
+            case 1: rope_token_kernel<false, true, 1><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
+            case 2: rope_token_kernel<false, true, 2><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
+            case 4: rope_token_kernel<false, true, 4><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
+            case 8: rope_token_kernel<false, true, 8><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
+            case 16: rope_token_kernel<false, true, 16><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
+            case 32: rope_token_kernel<false, true, 32><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
             default: return MI_ERR_UNSUPPORTED;
         }
     } else if (bq) {
@@ -1438,14 +1304,59 @@ extern "C" int mi_bias_rope_neox_qk_f16(void* q, void* k, const void* q_bias, co
 namespace mi {
 namespace {
 
-// Shared checks and launch of rope_kv_kernel.  q_bias / k_bias / v_bias (all
-// or none) and q_weight / k_weight (NORM) exclude each other.
+template <bool BIAS, bool NORM, int CPH, int P, int LPT>
+int rope_kv_p(const RopeKv& a, const float* inv_host, int64_t T, hipStream_t s) {
+    constexpr int NF = CPH ? CPH * 8 : kMaxHalf;
+    InvFreqN<NF> inv;
+    const int half = a.hd / 2;
+    for (int i = 0; i < NF; ++i) inv.v[i] = i < half ? inv_host[i] : 0.0f;
+    rope_kv_scatter_kernel<BIAS, NORM, CPH, P, NF, LPT>
+        <<<dim3(static_cast<unsigned>(ceil_div(T, 256 / LPT))), dim3(256), 0, s>>>(a, inv, T);
+    return launch_status();
+}
+// slots: the larger of the token's units and V vectors
+template <bool BIAS, bool NORM, int CPH>
+int rope_kv_cph(const RopeKv& a, const float* inv, int64_t T, int64_t slots, hipStream_t s) {
+    const int64_t lanes = std::max<int64_t>(slots, a.hd / 2);  // a lane per cos/sin entry too
+    if (lanes <= 64) return rope_kv_p<BIAS, NORM, CPH, 1, 64>(a, inv, T, s);
+    if (lanes <= 128) return rope_kv_p<BIAS, NORM, CPH, 1, 128>(a, inv, T, s);
+    if (slots <= 256) return rope_kv_p<BIAS, NORM, CPH, 1, 256>(a, inv, T, s);
+    if constexpr (CPH == 1 || CPH == 2) {
+        return MI_ERR_UNSUPPORTED;  // more than 128 heads of 16 or 32
+    } else {
+        if (slots <= 512) return rope_kv_p<BIAS, NORM, CPH, 2, 256>(a, inv, T, s);
+        return rope_kv_p<BIAS, NORM, CPH, 3, 256>(a, inv, T, s);
+    }
+}
+template <bool BIAS, bool NORM>
+int rope_kv_go(const RopeKv& a, const float* inv, int64_t T, int64_t slots, hipStream_t s) {
+    switch (a.hd / 16) {
+        case 1: return rope_kv_cph<BIAS, NORM, 1>(a, inv, T, slots, s);
+        case 2: return rope_kv_cph<BIAS, NORM, 2>(a, inv, T, slots, s);
+        case 4: return rope_kv_cph<BIAS, NORM, 4>(a, inv, T, slots, s);
+        case 8: return rope_kv_cph<BIAS, NORM, 8>(a, inv, T, slots, s);
+        case 16: return rope_kv_cph<BIAS, NORM, 16>(a, inv, T, slots, s);
+        case 32: return rope_kv_cph<BIAS, NORM, 32>(a, inv, T, slots, s);
+        default:
+            if constexpr (NORM)
+                return MI_ERR_UNSUPPORTED;  // head_dim not 16 * 2^k
+            else
+                return rope_kv_cph<BIAS, false, 0>(a, inv, T, slots, s);
+    }
+}
+
+// Shared checks and launch of rope_kv_scatter_kernel.  q_bias / k_bias / v_bias (all
+// or none) and q_weight / k_weight (NORM) exclude each other.  wide: tokens of
+// up to 768 units too, two or three per lane -- the chain's one-launch form
+// of steps its caller would otherwise issue apart; the C ABI's entry points
+// refuse them.
+}  // namespace
 int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const void* k_bias,
                    const void* v_bias, const void* q_weight, const void* k_weight, float eps,
                    int add_one, const int64_t* positions, const float* inv_freq_host, int64_t T,
                    int64_t Hq, int64_t Hkv, int64_t head_dim, void* k_cache, void* v_cache,
                    int64_t layer, int64_t num_blocks, int64_t block_size,
-                   const mi_kv_segment* segments, int num_segments, void* stream) {
+                   const mi_kv_segment* segments, int num_segments, bool wide, void* stream) {
     if (T < 0 || Hq < 0 || Hkv < 0 || head_dim < 0 || layer < 0 || layer >= (int64_t{1} << 62) ||
         num_blocks < 0 || block_size <= 0 || num_segments < 0)
         return MI_ERR_INVALID_ARGUMENT;
@@ -1457,9 +1368,11 @@ int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const vo
         (norm && (!q_weight || !k_weight)) || (bias && norm))
         return MI_ERR_INVALID_ARGUMENT;
     // one 256-lane workgroup per token: its Q/K slices and V's vectors one
-    // per lane (both <= 256), 16-byte vectors, few segments
-    if (head_dim % 16 != 0 || head_dim / 2 > kMaxHalf || (Hq + Hkv) * (head_dim / 16) > 256 ||
-        Hkv * head_dim / 8 > 256 || num_segments > kMaxKvSegs || T > kMaxGridX ||
+    // per lane (both <= 256; wide: up to three per lane), 16-byte vectors, few
+    // segments
+    if (head_dim % 16 != 0 || head_dim / 2 > kMaxHalf || Hq + Hkv > 1024) return MI_ERR_UNSUPPORTED;
+    const int64_t slots = std::max((Hq + Hkv) * (head_dim / 16), Hkv * head_dim / 8);
+    if (slots > (wide ? 768 : 256) || num_segments > kMaxKvSegs || T > kMaxGridX ||
         block_size > INT32_MAX)
         return MI_ERR_UNSUPPORTED;
     for (const void* p : {static_cast<const void*>(q), static_cast<const void*>(k), v,
@@ -1477,7 +1390,8 @@ int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const vo
     for (int i = 0; i < 5; ++i)
         for (int j = i + 1; j < 5; ++j)
             if (overlaps(bufs[i], lens[i], bufs[j], lens[j])) return MI_ERR_ALIASING;
-    KvSegs sg{};
+    RopeKv a{};
+    KvSegs& sg = a.sg;
     sg.n = num_segments;
     for (int i = 0; i < num_segments; ++i) {
         const mi_kv_segment& g = segments[i];
@@ -1505,50 +1419,32 @@ int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const vo
         sg.sl[i] = g.seq_len;
         sg.sp[i] = g.start_pos;
     }
-    InvFreq inv;
-    if (!load_inv_freq(inv_freq_host, head_dim / 2, inv)) return MI_ERR_INVALID_ARGUMENT;
-    const dim3 g(static_cast<unsigned>(T)), b(256);
-    auto* qh = static_cast<half_t*>(q);
-    auto* kh = static_cast<half_t*>(k);
-    const auto* vh = static_cast<const half_t*>(v);
-    const auto* bqh = static_cast<const half_t*>(q_bias);
-    const auto* bkh = static_cast<const half_t*>(k_bias);
-    const auto* bvh = static_cast<const half_t*>(v_bias);
-    const auto* wqh = static_cast<const half_t*>(q_weight);
-    const auto* wkh = static_cast<const half_t*>(k_weight);
-    auto* kc = static_cast<half_t*>(k_cache);
-    auto* vc = static_cast<half_t*>(v_cache);
+    if (!inv_freq_host) return MI_ERR_INVALID_ARGUMENT;
+    a.q = static_cast<half_t*>(q);
+    a.k = static_cast<half_t*>(k);
+    a.v = static_cast<const half_t*>(v);
+    a.Hq = static_cast<int>(Hq);
+    a.Hkv = static_cast<int>(Hkv);
+    a.hd = static_cast<int>(head_dim);
+    a.positions = positions;
+    a.bq = static_cast<const half_t*>(q_bias);
+    a.bk = static_cast<const half_t*>(k_bias);
+    a.bv = static_cast<const half_t*>(v_bias);
+    a.wq = static_cast<const half_t*>(q_weight);
+    a.wk = static_cast<const half_t*>(k_weight);
+    a.eps = eps;
+    a.w_bias = add_one ? 1.0f : -0.0f;  // w + (-0) == w, also for w = -0
+    a.k_cache = static_cast<half_t*>(k_cache);
+    a.v_cache = static_cast<half_t*>(v_cache);
+    a.layer = layer;
+    a.num_blocks = num_blocks;
+    a.bs = block_size;
     const hipStream_t s = as_stream(stream);
-    const int hq = static_cast<int>(Hq), hk = static_cast<int>(Hkv), d = static_cast<int>(head_dim);
-    const float wb = add_one ? 1.0f : -0.0f;  // w + (-0) == w, also for w = -0
-#define MI_RKV_ARGS                                                                           \
-    inv, qh, kh, vh, hq, hk, d, positions, bqh, bkh, bvh, wqh, wkh, eps, wb, kc, vc, sg, layer, \
-        num_blocks, block_size
-#define MI_RKV_CPH(BIAS, NORM)                                                            \
-    switch (head_dim / 16) {                                                              \
-        case 1: rope_kv_kernel<BIAS, NORM, 1><<<g, b, 0, s>>>(MI_RKV_ARGS); break;       \
-        case 2: rope_kv_kernel<BIAS, NORM, 2><<<g, b, 0, s>>>(MI_RKV_ARGS); break;       \
-        case 4: rope_kv_kernel<BIAS, NORM, 4><<<g, b, 0, s>>>(MI_RKV_ARGS); break;       \
-        case 8: rope_kv_kernel<BIAS, NORM, 8><<<g, b, 0, s>>>(MI_RKV_ARGS); break;       \
-        case 16: rope_kv_kernel<BIAS, NORM, 16><<<g, b, 0, s>>>(MI_RKV_ARGS); break;     \
-        case 32: rope_kv_kernel<BIAS, NORM, 32><<<g, b, 0, s>>>(MI_RKV_ARGS); break;     \
-        default:                                                                          \
-            if (NORM) return MI_ERR_UNSUPPORTED; /* head_dim not 16 * 2^k */             \
-            rope_kv_kernel<BIAS, false, 0><<<g, b, 0, s>>>(MI_RKV_ARGS);                 \
-    }
-    if (norm) {
-        MI_RKV_CPH(false, true)
-    } else if (bias) {
-        MI_RKV_CPH(true, false)
-    } else {
-        MI_RKV_CPH(false, false)
-    }
-#undef MI_RKV_CPH
-#undef MI_RKV_ARGS
-    return launch_status();
+    if (norm) return rope_kv_go<false, true>(a, inv_freq_host, T, slots, s);
+    if (bias) return rope_kv_go<true, false>(a, inv_freq_host, T, slots, s);
+    return rope_kv_go<false, false>(a, inv_freq_host, T, slots, s);
 }
 
-}  // namespace
 }  // namespace mi
 
 extern "C" int mi_rope_kv_scatter_f16(void* q, void* k, const void* v, const void* q_bias,
@@ -1561,7 +1457,8 @@ extern "C" int mi_rope_kv_scatter_f16(void* q, void* k, const void* v, const voi
                                       void* stream) {
     return mi::rope_kv_launch(q, k, v, q_bias, k_bias, v_bias, nullptr, nullptr, 0.0f, 0,
                               positions, inv_freq_host, T, Hq, Hkv, head_dim, k_cache, v_cache,
-                              layer, num_blocks, block_size, segments, num_segments, stream);
+                              layer, num_blocks, block_size, segments, num_segments, false,
+                              stream);
 }
 
 extern "C" int mi_qk_norm_rope_kv_scatter_f16(void* q, void* k, const void* v,
@@ -1577,7 +1474,7 @@ extern "C" int mi_qk_norm_rope_kv_scatter_f16(void* q, void* k, const void* v,
     return mi::rope_kv_launch(q, k, v, nullptr, nullptr, nullptr, q_weight, k_weight, eps,
                               add_one, positions, inv_freq_host, T, Hq, Hkv, head_dim, k_cache,
                               v_cache, layer, num_blocks, block_size, segments, num_segments,
-                              stream);
+                              false, stream);
 }
 
 extern "C" int mi_qk_norm_rope_f16(void* q, void* k, const void* q_weight, const void* k_weight,

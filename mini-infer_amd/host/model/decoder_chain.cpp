@@ -116,17 +116,13 @@ bool DecoderChain::rope_kv_fused(hipStream_t s) const {
         fs[n++] = mi_kv_segment{g.token_offset, g.B, g.S, g.block_table, g.seq_len,
                                 g.start_pos, g.max_blocks_per_seq};
     }
-    const int st =
-        d.use_qk_norm
-            ? mi_qk_norm_rope_kv_scatter_f16(d.q, d.k, d.v, d.q_norm, d.k_norm, d.positions,
-                                             inv_freq_.data(), d.T, d.num_heads, d.num_kv_heads,
-                                             d.head_dim, d.qk_norm_eps, /*add_one=*/0, d.k_cache,
-                                             d.v_cache, d.layer, d.num_blocks, d.block_size, fs,
-                                             n, sv(s))
-            : mi_rope_kv_scatter_f16(d.q, d.k, d.v, d.q_bias, d.k_bias, d.v_bias, d.positions,
-                                     inv_freq_.data(), d.T, d.num_heads, d.num_kv_heads,
-                                     d.head_dim, d.k_cache, d.v_cache, d.layer, d.num_blocks,
-                                     d.block_size, fs, n, sv(s));
+    const bool norm = d.use_qk_norm != 0;
+    const int st = mi::rope_kv_launch(
+        d.q, d.k, d.v, bias ? d.q_bias : nullptr, bias ? d.k_bias : nullptr,
+        bias ? d.v_bias : nullptr, norm ? d.q_norm : nullptr, norm ? d.k_norm : nullptr,
+        norm ? d.qk_norm_eps : 0.0f, /*add_one=*/0, d.positions, inv_freq_.data(), d.T, d.num_heads,
+        d.num_kv_heads, d.head_dim, d.k_cache, d.v_cache, d.layer, d.num_blocks, d.block_size, fs, n,
+        /*wide=*/true, sv(s));
     if (st == MI_ERR_UNSUPPORTED) return false;
     check(st, d.use_qk_norm ? "qk norm + rope + kv scatter"
                             : (bias ? "bias + rope + kv scatter" : "rope + kv scatter"));

@@ -87,3 +87,41 @@ def test_shared_scratch_keeps_the_order(mk, dev, double):
     torch.cuda.synchronize()
     assert torch.equal(w.t["hidden"], want["hidden"])
     assert torch.equal(w.t["final_normed"], want["final_normed"])
+
+
+# one slot per lane exactly, one unit more, two and three slots, and past them
+@pytest.mark.parametrize("Hq,Hkv,hd", [(28, 4, 128), (32, 1, 128), (32, 8, 128), (24, 24, 128),
+                                       (64, 8, 128), (80, 16, 128), (96, 8, 128), (32, 32, 80),
+                                       (40, 1, 256), (5, 60, 64)])
+@pytest.mark.parametrize("kind", ["plain", "bias", "norm"])
+def test_wide_tokens_into_the_cache(mk, dev, Hq, Hkv, hd, kind):
+    """RoPE and the cache writes in the chain's one launch against the RoPE entry
+    point and the scatters, bit for bit."""
+    import torch
+    if kind == "norm" and hd == 80:
+        pytest.skip("the norm takes heads of 16 * 2^k")
+    print(f"[case] chain rope + scatter {Hq}|{Hkv}x{hd} {kind}", flush=True)
+    w = mi_chain.Workload(dev, seed=Hq * hd + Hkv, n_decode=7, prefills=(37, 37), logit_rows=2,
+                          hidden_size=64, intermediate_size=64, num_heads=Hq, num_kv_heads=Hkv,
+                          head_dim=hd, vocab=200, use_qk_norm=int(kind == "norm"),
+                          qkv_bias=int(kind == "bias"))
+    t, c = w.t, w.cfg
+    q, k, v = (t[n].clone() for n in "qkv")
+    kc, vc = t["k_cache"].clone(), t["v_cache"].clone()
+    inv = mk.rope_inv_freq(hd, c["rope_theta"])
+    if kind == "norm":
+        mk.qk_norm_rope(q, k, t["q_norm"], t["k_norm"], t["positions"], inv, eps=c["qk_norm_eps"])
+    elif kind == "bias":
+        mk.bias_rope_neox_qk(q, k, t["q_bias"], t["k_bias"], t["positions"], inv)
+    else:
+        mk.rope_neox_qk(q, k, t["positions"], inv)
+    for g in w.segments:
+        B, S, at = g["B"], g["S"], g["token_offset"]
+        part = slice(at, at + B * S)
+        mk.paged_kv_scatter(k[part].view(B, S, Hkv, hd), kc, g["block_table"], g["seq_len"],
+                            g["start_pos"], 1, 16, v_src=v[part].view(B, S, Hkv, hd), v_cache=vc,
+                            v_bias=t["v_bias"] if kind == "bias" else None)
+    w.run(Stage.KV_SCATTER)
+    torch.cuda.synchronize()
+    assert torch.equal(t["q"], q) and torch.equal(t["k"], k) and torch.equal(t["v"], v)
+    assert torch.equal(t["k_cache"], kc) and torch.equal(t["v_cache"], vc)

@@ -1,4 +1,4 @@
-// chain_step.h -- the decoder step's row-wise stages as one launch, for a
+// chain_step.h -- the decoder step's stages several in one launch, for a
 // caller that has every GEMM output of the step in hand before it starts
 // (mi_decoder_chain_run).  Called by the host layer's DecoderChain, not part
 // of the C ABI.
@@ -40,5 +40,37 @@ int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const vo
                    int64_t Hq, int64_t Hkv, int64_t head_dim, void* k_cache, void* v_cache,
                    int64_t layer, int64_t num_blocks, int64_t block_size,
                    const mi_kv_segment* segments, int num_segments, bool wide, void* stream);
+
+// The whole step: the rows, the attention pre-processing into the cache, the
+// activation and the sampling step, each with its entry point's arguments.
+struct ChainStep {
+    ChainRows rows;
+    void *q, *k;
+    const void *v, *q_bias, *k_bias, *v_bias, *q_weight, *k_weight;
+    float qk_eps;
+    const int64_t* positions;
+    const float* inv_freq_host;
+    int64_t Hq, Hkv, head_dim;
+    void *k_cache, *v_cache;
+    int64_t layer, num_blocks, block_size;
+    const mi_kv_segment* segments;
+    int num_segments;
+    const void *gate, *up;
+    void* act_out;
+    int64_t act_n;
+    int gelu;  // 0: SwiGLU, 1: GeGLU
+    const void* logits;
+    void* probs;
+    int32_t* next_tokens;
+    int64_t N, vocab;
+    void* workspace;
+    int64_t workspace_bytes;
+};
+
+// One launch for the step.  MI_OK, a hipError_t, or
+// MI_ERR_UNSUPPORTED (nothing launched) for steps it does not take.  The buffers
+// must not overlap one another but in the stages' own in-place forms (the caller
+// checks).
+int chain_step(const ChainStep& c, void* stream);
 
 }  // namespace mi

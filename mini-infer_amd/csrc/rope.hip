@@ -1345,18 +1345,19 @@ int rope_kv_go(const RopeKv& a, const float* inv, int64_t T, int64_t slots, hipS
     }
 }
 
-// Shared checks and launch of rope_kv_scatter_kernel.  q_bias / k_bias / v_bias (all
+// Shared checks and arguments of rope_kv_scatter_kernel.  q_bias / k_bias / v_bias (all
 // or none) and q_weight / k_weight (NORM) exclude each other.  wide: tokens of
 // up to 768 units too, two or three per lane -- the chain's one-launch form
 // of steps its caller would otherwise issue apart; the C ABI's entry points
 // refuse them.
 }  // namespace
-int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const void* k_bias,
+int rope_kv_plan(void* q, void* k, const void* v, const void* q_bias, const void* k_bias,
                    const void* v_bias, const void* q_weight, const void* k_weight, float eps,
                    int add_one, const int64_t* positions, const float* inv_freq_host, int64_t T,
                    int64_t Hq, int64_t Hkv, int64_t head_dim, void* k_cache, void* v_cache,
                    int64_t layer, int64_t num_blocks, int64_t block_size,
-                   const mi_kv_segment* segments, int num_segments, bool wide, void* stream) {
+                   const mi_kv_segment* segments, int num_segments, bool wide,
+                 RopeKv& a, int64_t& slots) {
     if (T < 0 || Hq < 0 || Hkv < 0 || head_dim < 0 || layer < 0 || layer >= (int64_t{1} << 62) ||
         num_blocks < 0 || block_size <= 0 || num_segments < 0)
         return MI_ERR_INVALID_ARGUMENT;
@@ -1371,7 +1372,7 @@ int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const vo
     // per lane (both <= 256; wide: up to three per lane), 16-byte vectors, few
     // segments
     if (head_dim % 16 != 0 || head_dim / 2 > kMaxHalf || Hq + Hkv > 1024) return MI_ERR_UNSUPPORTED;
-    const int64_t slots = std::max((Hq + Hkv) * (head_dim / 16), Hkv * head_dim / 8);
+    slots = std::max((Hq + Hkv) * (head_dim / 16), Hkv * head_dim / 8);
     if (slots > (wide ? 768 : 256) || num_segments > kMaxKvSegs || T > kMaxGridX ||
         block_size > INT32_MAX)
         return MI_ERR_UNSUPPORTED;
@@ -1390,7 +1391,7 @@ int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const vo
     for (int i = 0; i < 5; ++i)
         for (int j = i + 1; j < 5; ++j)
             if (overlaps(bufs[i], lens[i], bufs[j], lens[j])) return MI_ERR_ALIASING;
-    RopeKv a{};
+    a = RopeKv{};
     KvSegs& sg = a.sg;
     sg.n = num_segments;
     for (int i = 0; i < num_segments; ++i) {
@@ -1439,9 +1440,24 @@ int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const vo
     a.layer = layer;
     a.num_blocks = num_blocks;
     a.bs = block_size;
+    return MI_OK;
+}
+
+int rope_kv_launch(void* q, void* k, const void* v, const void* q_bias, const void* k_bias,
+                   const void* v_bias, const void* q_weight, const void* k_weight, float eps,
+                   int add_one, const int64_t* positions, const float* inv_freq_host, int64_t T,
+                   int64_t Hq, int64_t Hkv, int64_t head_dim, void* k_cache, void* v_cache,
+                   int64_t layer, int64_t num_blocks, int64_t block_size,
+                   const mi_kv_segment* segments, int num_segments, bool wide, void* stream) {
+    RopeKv a;
+    int64_t slots = 0;
+    const int st = rope_kv_plan(q, k, v, q_bias, k_bias, v_bias, q_weight, k_weight, eps, add_one,
+                                positions, inv_freq_host, T, Hq, Hkv, head_dim, k_cache, v_cache,
+                                layer, num_blocks, block_size, segments, num_segments, wide, a, slots);
+    if (st != MI_OK || T == 0) return st;
     const hipStream_t s = as_stream(stream);
-    if (norm) return rope_kv_go<false, true>(a, inv_freq_host, T, slots, s);
-    if (bias) return rope_kv_go<true, false>(a, inv_freq_host, T, slots, s);
+    if (q_weight) return rope_kv_go<false, true>(a, inv_freq_host, T, slots, s);
+    if (q_bias) return rope_kv_go<true, false>(a, inv_freq_host, T, slots, s);
     return rope_kv_go<false, false>(a, inv_freq_host, T, slots, s);
 }
 

@@ -4,6 +4,7 @@
 // decoder step (chain_step.hip).
 #pragma once
 
+#include "mi_kernels.h"
 #include "rope_math.h"
 
 namespace mi {
@@ -35,6 +36,17 @@ struct RopeKv {
     int64_t layer, num_blocks, bs;
     KvSegs sg;
 };
+
+// Checks a call of the one-launch attention pre-processing and fills its device
+// arguments (rope.hip); slots: the larger of a token's (head, slice) units and its
+// V vectors.  MI_OK, or the entry points' status for the call.
+int rope_kv_plan(void* q, void* k, const void* v, const void* q_bias, const void* k_bias,
+                 const void* v_bias, const void* q_weight, const void* k_weight, float eps,
+                 int add_one, const int64_t* positions, const float* inv_freq_host, int64_t T,
+                 int64_t Hq, int64_t Hkv, int64_t head_dim, void* k_cache, void* v_cache,
+                 int64_t layer, int64_t num_blocks, int64_t block_size,
+                 const mi_kv_segment* segments, int num_segments, bool wide, RopeKv& a,
+                 int64_t& slots);
 
 // The token's cache row, in elements from the cache's start (-1: not
 // scattered), as launch_paged_kv_scatter places it

@@ -89,6 +89,13 @@ template <bool LOCAL, int SW>
 __device__ __forceinline__ void load_slot(const uint64_t* base, uint32_t byte_off,
                                           uint64_t (&w)[SW]) {
     static_assert(SW == 2 || SW == 4, "a slot is 2 or 4 words");
+    // the "s" operand has to be an SGPR pair; where the compiler cannot see that
+    // the base is uniform, it does not make one by itself
+    const auto bits = reinterpret_cast<uint64_t>(base);
+    base = reinterpret_cast<const uint64_t*>(
+        (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+             static_cast<int>(bits >> 32)))) << 32) |
+        static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(bits))));
     u32x4 a, b;
     if constexpr (SW == 2) {
         if constexpr (LOCAL)

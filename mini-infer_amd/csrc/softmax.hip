@@ -39,11 +39,7 @@
 #include "mi_device.h"
 #include "mi_host.h"
 #include "row_exchange.h"
-
-// Softmax stores: plain non-temporal (1 = write-through "nt sc1"; measured neutral).
-#ifndef MI_WT_SM
-#define MI_WT_SM 0
-#endif
+#include "softmax_stream.h"
 
 namespace mi {
 namespace {
@@ -57,109 +53,6 @@ constexpr int kMaxSplits = 1024;    // chunk pairs of a row, folded by one wave
 #define MI_SOFTMAX_TARGET_WGS 2048
 #endif
 constexpr int64_t kSplitTargetWgs = MI_SOFTMAX_TARGET_WGS;
-
-// exp(x - m) for every element of a row against one m, with m * log2(e)
-// formed once: one fma and the exp per element instead of a subtract, a
-// multiply and the exp (the VALU work sits on the critical path before and
-// after a one-launch row's exchange: 9.5 -> 8.9 us at [64, 152064]).
-constexpr float kLog2e = 1.4426950408889634f;
-__device__ __forceinline__ float exp_shifted(float x, float m_log2e) {
-    return __builtin_amdgcn_exp2f(fmaf(x, kLog2e, -m_log2e));
-}
-
-// Fold one loaded value group into the lane's online (m, s).
-template <int VEC>
-__device__ __forceinline__ void fold(const float (&v)[VEC], float& m, float& s) {
-    float vm = v[0];
-#pragma unroll
-    for (int k = 1; k < VEC; ++k) vm = fmaxf(vm, v[k]);
-    const float mn = fmaxf(m, vm);
-    if (mn == -INFINITY) return;  // nothing but -inf so far
-    float acc = s * fast_exp(m - mn);
-    const float mnl = mn * kLog2e;
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) acc += exp_shifted(v[k], mnl);
-    s = acc;
-    m = mn;
-}
-
-// Accumulate elements [begin, end) of a row into this lane's (m, s).  Loads
-// are issued kStatUnroll groups at a time, before the math that consumes them.
-constexpr int kStatUnroll = 4;
-template <int VEC>
-__device__ __forceinline__ void lane_stats(const half_t* xr, int64_t begin, int64_t end, float& m,
-                                           float& s) {
-    const int64_t step = static_cast<int64_t>(blockDim.x) * VEC;
-    for (int64_t i0 = begin + static_cast<int64_t>(threadIdx.x) * VEC; i0 < end;
-         i0 += step * kStatUnroll) {
-        float v[kStatUnroll][VEC];
-#pragma unroll
-        for (int j = 0; j < kStatUnroll; ++j) {
-            const int64_t i = i0 + j * step;
-            if (i < end) {
-                if constexpr (VEC == 8) {
-                    const h8 h = ld8(xr + i);
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) v[j][k] = (float)h[k];
-                } else {
-                    v[j][0] = (float)xr[i];
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < VEC; ++k) v[j][k] = -INFINITY;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < kStatUnroll; ++j) fold<VEC>(v[j], m, s);
-    }
-}
-
-// Vector form for split rows: [begin, end) is walked in tiles of 2048 * U
-// elements (U vectors per lane), all loads of a tile issued first.  The
-// tile's lane maximum comes from packed fp16 max (which passes over NaN, as
-// fmaxf does), then one exp per element against it, and one online merge
-// per tile -- not a rescale per vector.  Out-of-range slots hold -inf, whose
-// exp is 0.  RAGGED: xr is the row's window `win`, [begin, end) positions in
-// it.
-template <int U, bool RAGGED = false>
-__device__ __forceinline__ void tile_stats(const half_t* xr, int64_t begin, int64_t end, float& m,
-                                           float& s, const RowWindow* win = nullptr) {
-    constexpr int64_t kTile = 256 * 8 * U;
-    for (int64_t t0 = begin; t0 < end; t0 += kTile) {
-        h8 a[U];
-#pragma unroll
-        for (int j = 0; j < U; ++j) {
-            const int64_t i = t0 + (threadIdx.x + j * 256) * 8;
-            a[j] = i < end ? ld8(xr + i) : h8(-__builtin_huge_valf16());
-        }
-        if constexpr (RAGGED) {
-#pragma unroll
-            for (int j = 0; j < U; ++j) {
-                const int64_t i = t0 + (threadIdx.x + j * 256) * 8;
-                if (i < end && win->partial(static_cast<int>(i >> 3)))
-                    win->mask(static_cast<int>(i >> 3), a[j]);
-            }
-        }
-        h2 m2 = h2(-__builtin_huge_valf16());
-#pragma unroll
-        for (int j = 0; j < U; ++j) {
-#pragma unroll
-            for (int k = 0; k < 8; k += 2) m2 = __builtin_elementwise_max(m2, h2{a[j][k], a[j][k + 1]});
-        }
-        const float mt = (float)__builtin_elementwise_max(m2.x, m2.y);
-        if (!(mt > -INFINITY)) continue;  // nothing but -inf (or NaN) in this lane's tile
-        float st = 0.0f;
-        const float mtl = mt * kLog2e;
-#pragma unroll
-        for (int j = 0; j < U; ++j) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) st += exp_shifted((float)a[j][k], mtl);
-        }
-        const float mn = fmaxf(m, mt);
-        s = s * fast_exp(m - mn) + st * fast_exp(mt - mn);
-        m = mn;
-    }
-}
 
 // y = exp(x - m) * inv over [begin, end): the last use of x and the only
 // write of y, both streamed.
@@ -199,17 +92,6 @@ __device__ __forceinline__ void write_range(const half_t* xr, half_t* yr, int64_
             }
         }
     }
-}
-
-// Workgroup-wide merge of per-lane (m, s): max first, then rescaled sums.
-// (A one-barrier form -- wave (max, sum) pairs folded after a single barrier
-// -- measured no faster at [64, 152064].)  `slots` needs one float per wave.
-__device__ __forceinline__ void block_merge(float& m, float& s, float* slots) {
-    const float M = block_max(m, slots);
-    const float part = (m == -INFINITY) ? 0.0f : s * fast_exp(m - M);
-    __syncthreads();  // slots are reused by the sum
-    s = block_sum(part, slots);
-    m = M;
 }
 
 // Register-resident rows (16-byte vectors, D <= G * VPT * 8): G lanes per
@@ -449,385 +331,18 @@ __global__ __launch_bounds__(256) void softmax_finish_kernel(const half_t* x, ha
     }
 }
 
-// ---------------------------------------------------------------------------
-// One-launch split rows (row records: mi_softmax_ws_f16, or stream 0; x != y):
-// each workgroup holds an 8192-element chunk of a row in registers, publishes
-// the chunk's (max, sum), and reads every chunk's pair of its row to finish --
-// one launch, one read of x, no atomics on a contended address.  The grid is
-// `chunks per row` x R row slots, all resident; slot r handles rows r, r + R,
-// ... in rounds (one round when every row fits), and issues its next row's
-// loads before it polls for the current row's statistics.
-//
-// Workspace (zero before first use; every call leaves it valid for the
-// next): row slot r owns a fixed record at r * kRowRecordBytes -- a 64-bit
-// epoch word (128-byte header), then two sets of kOnePassMaxSplits slots of
-// two 64-bit words {tag << 32 | bits(max)}, {tag << 32 | bits(sum)}, and a
-// mirror of both sets (row_exchange.h: each word is published into the XCD's
-// L2 and through to memory; polls read the L2 copy first).  A call
-// reads the slot's epoch E; round k publishes into set k & 1 with tag = the
-// low 32 bits of E + 1 + k and polls the set until every chunk's pair carries
-// that tag.  Because slots are fixed per (row slot, chunk) whatever the
-// call's shape, and an epoch only grows (64 bits: it cannot wrap), a slot
-// left by an earlier call never carries the tag a later call waits for --
-// short of a slot left unwritten for 2^32 of its epochs and read again at
-// exactly a multiple of 2^32 later:
-//   * the chunk-0 workgroup raises the epoch to E + K (atomic max) after the
-//     last (K-th) round, when every workgroup of the slot has published it --
-//     so every one of them has already read E;
-//   * a workgroup whose polling runs out (kPollLimit polls or kPollTicks of
-//     the 100 MHz constant clock, whichever comes first; not expected when
-//     the grid fits the GPU) computes that row's statistics itself from x and
-//     raises the epoch to E + K + 1 at once, past every tag the launch writes
-//     for the slot.  A workgroup that starts after that reads the higher
-//     epoch, its tags match nobody's, and it takes the same fallback for its
-//     rows: slower, still correct.  A workgroup that has fallen back once
-//     stops polling for its remaining rounds (its row-mates may be out of
-//     step with it for good), so a late start costs at most one poll bound
-//     per workgroup, not one per round.  Polling is bounded: no workgroup
-//     can wait forever.
-// A workgroup publishes round k + 2 into a set only after it has seen every
-// chunk's round k + 1 pair, which its row-mates publish after they have read
-// round k: no pair is overwritten before it is read.  Each 64-bit word is
-// stored and loaded whole, so a tag always travels with its value.
-// The grid is 1-D and places every chunk of a row slot on one XCD
-// (chunk_of), so the L2 copy normally serves the polls.
-// ---------------------------------------------------------------------------
-constexpr int kOnePassMaxSplits = 64;
-#ifndef MI_SOFTMAX_ONEPASS_U
-#define MI_SOFTMAX_ONEPASS_U 4
-#endif
-constexpr int kOnePassU = MI_SOFTMAX_ONEPASS_U;     // vectors per lane
-constexpr int64_t kOnePassChunk = 2048 * kOnePassU;  // elements per workgroup
-// header, then two sets of slots (alternated by round) and their mirror; a
-// slot is the chunk's tagged (max, sum) pair, plus its tagged argmax key (two
-// words) in the fused softmax + argmax pass
-constexpr int64_t kRowRecordBytes = kRecordHeaderBytes + 4 * kOnePassMaxSplits * 16;
-constexpr int64_t kRowRecordBytesAM = kRecordHeaderBytes + 4 * kOnePassMaxSplits * 32;
-template <bool AM>
-constexpr int64_t record_bytes() { return AM ? kRowRecordBytesAM : kRowRecordBytes; }
-constexpr int kPollLimit = 1 << 16;
-std::atomic<int> g_poll_limit{kPollLimit};  // mi_softmax_test_poll_limit
-
-__device__ __forceinline__ uint64_t tagged(uint32_t tag, float v) {
-    return (static_cast<uint64_t>(tag) << 32) | __builtin_bit_cast(uint32_t, v);
-}
-
-// The pieces of a one-launch chunk workgroup.
-// The lane's (max, sum) over its vectors: packed fp16 maximum, one exp per
-// element.
-template <int U>
-__device__ __forceinline__ void chunk_lane_stats(const h8 (&a)[U], float& m, float& s) {
-    h2 m2 = h2(-__builtin_huge_valf16());
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-#pragma unroll
-        for (int k = 0; k < 8; k += 2) m2 = __builtin_elementwise_max(m2, h2{a[j][k], a[j][k + 1]});
-    }
-    m = (float)__builtin_elementwise_max(m2.x, m2.y);
-    s = 0.0f;
-    if (m > -INFINITY) {
-        const float ml = m * kLog2e;
-#pragma unroll
-        for (int j = 0; j < U; ++j) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                s += exp_shifted((float)a[j][k], ml);
-        }
-    } else {
-        m = -INFINITY;  // NaN-free lane maximum of an all -inf (or NaN) lane
-    }
-}
-// Thread 0 publishes the chunk's pair (and, AM, its argmax key) into slot
-// `split` of `slots` (SW = 2 or 4 words per slot) and of its mirror
-// (`mirror` words on).
-template <bool AM>
-__device__ __forceinline__ void chunk_publish(uint64_t* slots, int64_t mirror, int split,
-                                              uint32_t tag, float m, float s, uint64_t key) {
-    constexpr int SW = AM ? 4 : 2;
-    if (threadIdx.x == 0) {
-        uint64_t w[SW];
-        w[0] = tagged(tag, m);
-        w[1] = tagged(tag, s);
-        if constexpr (AM) {
-            const uint64_t t = static_cast<uint64_t>(tag) << 32;
-            w[2] = t | (key >> 32);
-            w[3] = t | (key & 0xffffffffu);
-        }
-        uint64_t* p = slots + SW * split;
-#pragma unroll
-        for (int i = 0; i < SW; ++i) local_store(&p[i], w[i]);
-#pragma unroll
-        for (int i = 0; i < SW; ++i) device_store(&p[mirror + i], w[i]);
-    }
-}
-// Wave 0 (the caller calls it there) polls the row's `splits` slots (lane j
-// reads chunk j) until all carry `tag`, at most poll_limit rounds -- the L2
-// copy (local) for up to kLocalPollTicks, then the mirror `mirror` words on
-// at device scope (row_exchange.h) -- and leaves
-// the row's (M, S) in row_stats[0..1] (AM with want_key: its best key in
-// *row_key, the key words polled too; without, only the pair words, half
-// the bytes per poll: 12.9 -> 12.0 us at [64, 152064]) and row_stats[2] = 0,
-// or row_stats[2] = 1 when polling ran out.  The caller's barrier publishes
-// them.
-// Polls of one phase (LOCAL: the L2 copy, else the device-scope mirror) of
-// `set` (workgroup-uniform) until every chunk's slot carries `tag`, `it`
-// reaches poll_limit or the clock passes t0 + ticks; lane j < splits reads
-// slot j.  Returns whether every slot was seen.
-template <bool AM, bool LOCAL>
-__device__ __forceinline__ bool poll_phase(const uint64_t* set, int splits, uint32_t tag,
-                                           bool want_key, int& it, int poll_limit, uint64_t t0,
-                                           uint64_t ticks, float& mj, float& sj, uint64_t& kj) {
-    constexpr int SW = AM ? 4 : 2;
-    const int lane = threadIdx.x & (kWave - 1);
-    const uint32_t off = static_cast<uint32_t>(lane) * (SW * 8);
-    for (; it < poll_limit; ++it) {
-        if (it > 0 && __builtin_amdgcn_s_memrealtime() - t0 > ticks) return false;
-        bool mine = true;
-        if (lane < splits) {
-            // chunk 0 alone writes the index, so only it reads the key words
-            uint64_t w[SW];
-            if (AM && want_key)
-                load_slot<LOCAL, SW>(set, off, w);
-            else
-                load_slot<LOCAL, 2>(set, off, reinterpret_cast<uint64_t(&)[2]>(w));
-            mine = static_cast<uint32_t>(w[0] >> 32) == tag && static_cast<uint32_t>(w[1] >> 32) == tag;
-            mj = __builtin_bit_cast(float, static_cast<uint32_t>(w[0]));
-            sj = __builtin_bit_cast(float, static_cast<uint32_t>(w[1]));
-            if constexpr (AM) {
-                if (want_key) {
-                    mine = mine && static_cast<uint32_t>(w[2] >> 32) == tag &&
-                           static_cast<uint32_t>(w[3] >> 32) == tag;
-                    kj = (w[2] << 32) | (w[3] & 0xffffffffu);
-                }
-            }
-        }
-        if (__all(mine)) return true;
-        __builtin_amdgcn_s_sleep(2);
-    }
-    return false;
-}
-
-template <bool AM>
-__device__ __forceinline__ void row_poll(const uint64_t* slots, int64_t mirror, bool local,
-                                         int splits, uint32_t tag, int poll_limit,
-                                         float* row_stats, uint64_t* row_key, bool want_key) {
-    const int lane = threadIdx.x & (kWave - 1);
-    float mj = -INFINITY, sj = 0.0f;
-    uint64_t kj = 0;
-    const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-    int it = 0;
-    bool all = local && poll_phase<AM, true>(slots, splits, tag, want_key, it, poll_limit, t0,
-                                             kLocalPollTicks, mj, sj, kj);
-    if (!all)
-        all = poll_phase<AM, false>(slots + mirror, splits, tag, want_key, it, poll_limit, t0,
-                                    kPollTicks, mj, sj, kj);
-    if (all) {
-        if (lane >= splits) {
-            mj = -INFINITY;
-            sj = 0.0f;
-            kj = 0;
-        }
-        const float M = group_max<kWave>(mj);
-        const float S = group_sum<kWave>(mj == -INFINITY ? 0.0f : sj * fast_exp(mj - M));
-        if (AM && want_key) kj = wave_max_u64(kj);
-        if (lane == 0) {
-            row_stats[0] = M;
-            row_stats[1] = S;
-            row_stats[2] = 0.0f;
-            if (AM && want_key) *row_key = kj;
-        }
-    } else if (lane == 0) {
-        row_stats[2] = 1.0f;
-    }
-}
-// The row's statistics from x itself (the fallback when polling runs out; x
-// is not written: y != x).  Barriers: called by the whole workgroup.
-template <bool RAGGED>
-__device__ __forceinline__ void row_stats_from_x(const half_t* xr, int64_t D, float& M, float& S,
-                                                 float* slots) {
-    float fm = -INFINITY, fs = 0.0f;
-    if constexpr (RAGGED)
-        lane_stats<1>(xr, 0, D, fm, fs);
-    else
-        tile_stats<2>(xr, 0, D, fm, fs);
-    __syncthreads();  // slots reused
-    block_merge(fm, fs, slots);
-    __syncthreads();  // every wave has read slots before a later round writes them
-    M = fm;
-    S = fs;
-}
-// The persistent kernel's per-lane view of its chunk: the same in every
-// round, so one 32-bit byte offset (rows are < 2^31 bytes) and a valid flag
-// per vector, against a row base that is uniform across the workgroup.
-template <int U>
-__device__ __forceinline__ void lane_load(const half_t* row, uint32_t lo, const bool (&ok)[U],
-                                          h8 (&a)[U]) {
-    const char* base = reinterpret_cast<const char*>(row) + lo;
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-        const half_t* p = reinterpret_cast<const half_t*>(base + j * 256 * 16);
-        a[j] = ok[j] ? ld8_stream(p) : h8(-__builtin_huge_valf16());
-    }
-}
-// RAGGED: row is the row's window, v0 the lane's first vector in it.
-template <int U, bool RAGGED>
-__device__ __forceinline__ void lane_store(const h8 (&a)[U], half_t* row, uint32_t lo,
-                                           const bool (&ok)[U], float M, float inv,
-                                           const RowWindow& win, int v0) {
-    // y = exp(x - M) / S = exp2(x log2(e) - (M log2(e) + log2(S))): the division folded into
-    // the exponent's constant c, one fma and the exp per element ([512, 131072] 46.4 -> 46.0
-    // us; c carries the same rounding as M log2(e) alone, well under an fp16 ulp of y)
-    const float c = M * kLog2e - __builtin_amdgcn_logf(inv);
-    char* base = reinterpret_cast<char*>(row) + lo;
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-        if (ok[j]) {
-            h8 o;
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                o[k] = to_half(__builtin_amdgcn_exp2f(fmaf((float)a[j][k], kLog2e, -c)));
-            half_t* p = reinterpret_cast<half_t*>(base + j * 256 * 16);
-            if constexpr (RAGGED)
-                win.store(v0 + j * 256, p, o);
-            else
-                st8_out<MI_WT_SM>(p, o);
-        }
-    }
-}
-
-// 64 VGPRs, so 8 workgroups per CU (per-lane 32-bit offsets, not 64-bit
-// indices: 68 VGPRs and 7 workgroups per CU with them measured 5-10 points
-// lower; amdgpu_waves_per_eu(8) also measured ~8 points lower at the same
-// 64 VGPRs); wave 0 publishes and polls.
-// U vectors per lane: chunks of 2048 * U elements.  AM: the fused softmax +
-// greedy argmax pass -- each chunk also forms its best argmax key from the
-// registers it already holds, publishes it with its (max, sum), and chunk 0
-// writes the row's index to `out` (the fallback scans the row from x).
-// (AM: held to 5 waves per SIMD, <= 96 VGPRs, so that 1216 chunk workgroups
-// of [64, 152064] stay resident at once; the compiler otherwise settles at
-// 98 and the grid needs a second round.)
-// RAGGED: chunks of the row's aligned window (RowWindow) -- rows of a slot are
-// R (a multiple of 8) apart, so one window shape serves all its rounds.
-// Against the 2-byte two-launch forms: [64, 151643] 32.1 -> 9.9 us (softmax),
-// 37.1 -> 11.0 (with the argmax); aligned [64, 152064] 9.0 / 10.2.
-// ONE (ragged rows only): every row in one round, so no next row's registers
-// and no conditions kept across rounds -- 44-68 VGPRs against 73-96 and, with
-// AM, spills: [64, 151643] softmax + argmax 14.2 -> 11.0 us, [200, 32001]
-// softmax 10.2 -> 8.2.  (For aligned rows, which have no such conditions, it
-// measured slower: [64, 152064] 9.0 -> 9.6 and 10.2 -> 11.1 us.)
+// softmax_stream.h: the one-launch split rows
 template <int U, bool AM, bool RAGGED, bool ONE>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(AM ? 5 : 1))) void softmax_stream_kernel(const half_t* x, half_t* y,
-                                                             unsigned char* ws, int64_t N,
-                                                             int64_t D, int poll_limit,
-                                                             int32_t* out, int splits, int R,
-                                                             int local) {
-    constexpr int64_t kChunk = 2048 * U;
-    constexpr int SW = AM ? 4 : 2;
-    __shared__ float slots[256 / kWave];
-    __shared__ float row_stats[3];  // M, S, fallback flag
-    __shared__ uint64_t epoch_sh;
-    __shared__ uint64_t kslots[AM ? 256 / kWave : 1];  // per-wave keys (AM)
-    __shared__ uint64_t row_key;                        // the row's best key (AM)
-    // 1-D grid of splits x R (R a multiple of kXcds): a row slot's chunks
-    // share one XCD (row_exchange.h); slots past N-1 have no rows
-    int split, slot;
-    chunk_of(blockIdx.x, splits, split, slot);
-    const int64_t r0 = slot;
-    if (r0 >= N) return;  // workgroup-uniform, before any barrier
-    unsigned char* rec = ws + r0 * record_bytes<AM>();
-    uint64_t* epoch = reinterpret_cast<uint64_t*>(rec);
-    uint64_t* sets = reinterpret_cast<uint64_t*>(rec + kRecordHeaderBytes);
-    constexpr int64_t kMirror = 2 * SW * kOnePassMaxSplits;  // words from a set to its mirror
-    const int64_t K = ONE ? 1 : (N - r0 + R - 1) / R;  // rounds of this row slot (>= 1)
-    RowWindow win(x + r0 * D, D);  // RAGGED
-    const int64_t shift = RAGGED ? win.shift : 0;
-    const int64_t len = RAGGED ? win.nv * 8 : D;
-    const int64_t b = split * kChunk;
-    const int64_t e = b + kChunk < len ? b + kChunk : len;
-    const uint32_t lo = static_cast<uint32_t>(b + threadIdx.x * 8) * 2;
-    const int v0 = static_cast<int>(b >> 3) + static_cast<int>(threadIdx.x);
-    bool ok[U];
-#pragma unroll
-    for (int j = 0; j < U; ++j) ok[j] = b + (threadIdx.x + j * 256) * 8 < e;
-
-    if (threadIdx.x == 0)
-        epoch_sh = __hip_atomic_load(epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    h8 a[U], n[ONE ? 1 : U];
-    lane_load<U>(x + r0 * D - shift, lo, ok, a);
-    bool gave_up = false;  // workgroup-uniform: set after the first fallback
-    for (int64_t k = 0; k < K; ++k) {
-        const int64_t row = r0 + k * R;
-        // The guard is always true (256 lanes); written out, it keeps the
-        // statistics in a block of their own, which measured 64 VGPRs with
-        // no spill against 80 without it.
-        if constexpr (RAGGED) {
-            // workgroup-uniform: the row's first or last vector.  (win made
-            // opaque in each round: its conditions otherwise stay in
-            // registers across the rounds, some 250 of them)
-            asm volatile("" : "+s"(win.shift), "+s"(win.last));
-            if (split == 0 || e == len) {
-#pragma unroll
-                for (int j = 0; j < U; ++j)
-                    if (ok[j]) win.mask(v0 + j * 256, a[j]);
-            }
-        }
-        float m = -INFINITY, s = 0.0f;
-        if (threadIdx.x < 256) chunk_lane_stats<U>(a, m, s);
-        if constexpr (AM) {
-            // vectors past the row hold -inf (lane_load), whose key is 0
-            const uint64_t kw = wave_max_u64(lane_best_key<U, RAGGED>(a, b, static_cast<int>(shift)));
-            if ((threadIdx.x & (kWave - 1)) == 0) kslots[threadIdx.x / kWave] = kw;
-        }
-        block_merge(m, s, slots);  // barriers: epoch_sh (first round) and kslots visible after
-        uint64_t key = 0;
-        if constexpr (AM) {
-#pragma unroll
-            for (int w = 0; w < 256 / kWave; ++w) key = max_u64(key, kslots[w]);
-        }
-        const uint64_t E = epoch_sh;
-        const uint32_t tag = static_cast<uint32_t>(E + 1 + k);
-        uint64_t* set = sets + (k & 1) * (SW * kOnePassMaxSplits);
-        chunk_publish<AM>(set, kMirror, split, tag, m, s, key);
-        if constexpr (!ONE) {
-            if (k + 1 < K) lane_load<U>(x + (row + R) * D - shift, lo, ok, n);
-        }
-        if (gave_up) {
-            if (threadIdx.x == 0) row_stats[2] = 1.0f;
-        } else if (threadIdx.x < kWave) {
-            // only chunk 0 writes the index, so only it polls the key words
-            row_poll<AM>(set, kMirror, local != 0, splits, tag, poll_limit, row_stats, &row_key,
-                         split == 0);
-        }
-        __syncthreads();
-        float M = row_stats[0], S = row_stats[1];
-        const bool fallback = row_stats[2] != 0.0f;
-        gave_up = gave_up || fallback;
-        if (fallback) row_stats_from_x<RAGGED>(x + row * D, D, M, S, slots);
-        if constexpr (AM) {
-            if (split == 0) {  // workgroup-uniform: chunk_best has barriers
-                uint64_t rk = row_key;
-                if (fallback) {
-                    rk = RAGGED ? chunk_best<1, 8>(x + row * D, 0, D, kslots)
-                                : chunk_best<8, 4>(x + row * D, 0, D, kslots);
-                    __syncthreads();  // kslots are written again by the next round
-                }
-                if (threadIdx.x == 0) out[row] = key_index(rk);
-            }
-        }
-        if (threadIdx.x == 0 && (fallback || (split == 0 && k + 1 == K)))
-            __hip_atomic_fetch_max(epoch, fallback ? E + K + 1 : E + K, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-        if constexpr (RAGGED) asm volatile("" : "+s"(win.shift), "+s"(win.last));
-        lane_store<U, RAGGED>(a, y + row * D - shift, lo, ok, M, 1.0f / S, win, v0);
-        if constexpr (!ONE) {
-            if (k + 1 < K) {
-#pragma unroll
-                for (int j = 0; j < U; ++j) a[j] = n[j];
-            }
-        }
-    }
+__attribute__((amdgpu_waves_per_eu(AM ? 5 : 1))) void softmax_stream_kernel(
+    const half_t* x, half_t* y, unsigned char* ws, int64_t N, int64_t D, int poll_limit, int32_t* out,
+    int splits, int R, int local) {
+    const int block = blockIdx.x;
+#include "softmax_stream_body.h"
 }
+
+constexpr int kPollLimit = 1 << 16;
+std::atomic<int> g_poll_limit{kPollLimit};  // mi_softmax_test_poll_limit
 
 // kStream: many rows long enough that chunking them beats a workgroup per
 // row; with row records and y != x they run as softmax_stream_kernel,
@@ -1187,9 +702,9 @@ extern "C" int64_t mi_softmax_argmax_workspace_bytes(int64_t N, int64_t V) {
     return kFusedRegion + mi::workspace_bytes(N, V) + mi_greedy_argmax_workspace_bytes(N, V);
 }
 
-extern "C" int mi_softmax_argmax_ws_f16(const void* logits, void* probs, int32_t* out, int64_t N,
-                                        int64_t V, void* workspace, int64_t workspace_bytes,
-                                        void* stream) {
+namespace {
+int softmax_argmax_check(const void* logits, const void* probs, const void* out, int64_t N,
+                         int64_t V, const void* workspace, int64_t workspace_bytes) {
     if (N < 0 || V < 0 || workspace_bytes < 0) return MI_ERR_INVALID_ARGUMENT;
     if (N == 0 || V == 0) return MI_OK;
     if (!logits || !probs || !out || !workspace) return MI_ERR_INVALID_ARGUMENT;
@@ -1204,6 +719,30 @@ extern "C" int mi_softmax_argmax_ws_f16(const void* logits, void* probs, int32_t
         mi::overlaps(out, N * 4, logits, bytes) || mi::overlaps(out, N * 4, probs, bytes) ||
         mi::overlaps(out, N * 4, workspace, need))
         return MI_ERR_ALIASING;
+    return MI_OK;
+}
+}  // namespace
+
+bool mi::softmax_argmax_plan(const void* logits, const void* probs, const void* out, int64_t N,
+                             int64_t V, const void* workspace, int64_t workspace_bytes,
+                             StreamPlan& p) {
+    if (softmax_argmax_check(logits, probs, out, N, V, workspace, workspace_bytes) != MI_OK ||
+        N <= 0 || V <= 0 || N > kSplitMaxRows || !onelaunch_ok(logits, probs, N, V, true))
+        return false;
+    p.ragged = onelaunch_ragged(logits, probs, V);
+    const int64_t len = onelaunch_len(V, p.ragged);
+    p.u = onelaunch_u(N, len);
+    p.splits = static_cast<int>(ceil_div(len, 2048 * p.u));
+    p.poll_limit = g_poll_limit.load();
+    p.local = exchange_test_mode().load() == 0 ? 1 : 0;
+    return true;
+}
+
+extern "C" int mi_softmax_argmax_ws_f16(const void* logits, void* probs, int32_t* out, int64_t N,
+                                        int64_t V, void* workspace, int64_t workspace_bytes,
+                                        void* stream) {
+    const int st0 = softmax_argmax_check(logits, probs, out, N, V, workspace, workspace_bytes);
+    if (st0 != MI_OK || N == 0 || V == 0) return st0;
     auto* ws = static_cast<unsigned char*>(workspace);
     const hipStream_t s = mi::as_stream(stream);
     if (mi::onelaunch_ok(logits, probs, N, V, true))

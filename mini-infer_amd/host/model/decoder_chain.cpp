@@ -31,6 +31,18 @@ void need(bool ok, const char* what) {
 
 void* sv(hipStream_t s) { return reinterpret_cast<void*>(s); }
 
+// The segments that hold tokens, as the C ABI's; -1 for more than 8.
+int live_segments(const std::vector<mi_chain_kv_segment>& segs, mi_kv_segment (&out)[8]) {
+    int n = 0;
+    for (const mi_chain_kv_segment& g : segs) {
+        if (g.B * g.S == 0) continue;
+        if (n == 8) return -1;
+        out[n++] = mi_kv_segment{g.token_offset, g.B, g.S, g.block_table, g.seq_len,
+                                 g.start_pos, g.max_blocks_per_seq};
+    }
+    return n;
+}
+
 }  // namespace
 
 DecoderChain::DecoderChain(const mi_chain_desc& d, int last_stage) : d_(d), last_(last_stage) {
@@ -109,13 +121,8 @@ bool DecoderChain::rope_kv_fused(hipStream_t s) const {
     const bool bias = d.q_bias != nullptr;
     if ((d.use_qk_norm && bias) || d.num_heads <= 0 || d.num_kv_heads <= 0) return false;
     mi_kv_segment fs[8];
-    int n = 0;
-    for (const mi_chain_kv_segment& g : segs_) {
-        if (g.B * g.S == 0) continue;
-        if (n == 8) return false;
-        fs[n++] = mi_kv_segment{g.token_offset, g.B, g.S, g.block_table, g.seq_len,
-                                g.start_pos, g.max_blocks_per_seq};
-    }
+    const int n = live_segments(segs_, fs);
+    if (n < 0) return false;
     const bool norm = d.use_qk_norm != 0;
     const int st = mi::rope_kv_launch(
         d.q, d.k, d.v, bias ? d.q_bias : nullptr, bias ? d.k_bias : nullptr,
@@ -204,10 +211,7 @@ bool DecoderChain::buffers_apart() const {
     return true;
 }
 
-// Stages 1-2, 5 and 7 in one launch (chain_step.h), which keeps the residual
-// stream in registers between them.  False (nothing launched) for shapes it
-// does not take.
-bool DecoderChain::rows_fused(hipStream_t s) const {
+mi::ChainRows DecoderChain::rows_args() const {
     const mi_chain_desc& d = d_;
     mi::ChainRows c{};
     c.ids = d.ids;
@@ -229,9 +233,65 @@ bool DecoderChain::rows_fused(hipStream_t s) const {
     c.scale = d.embed_scale ? std::sqrt(static_cast<float>(d.hidden_size)) : 1.0f;
     c.eps = d.rms_eps;
     c.add_one = d.norm_add_one;
-    const int st = mi::chain_rows(c, sv(s));
+    return c;
+}
+
+// Stages 1-2, 5 and 7 in one launch (chain_step.h), which keeps the residual
+// stream in registers between them.  False (nothing launched) for shapes it
+// does not take.
+bool DecoderChain::rows_fused(hipStream_t s) const {
+    const int st = mi::chain_rows(rows_args(), sv(s));
     if (st == MI_ERR_UNSUPPORTED) return false;
     check(st, "gather + residual adds + norms");
+    return true;
+}
+
+// The whole step in one launch (chain_step.h).  False (nothing launched) for
+// steps it does not take.
+bool DecoderChain::step_fused(hipStream_t s) const {
+    const mi_chain_desc& d = d_;
+    const bool bias = d.q_bias != nullptr, norm = d.use_qk_norm != 0;
+    if ((norm && bias) || d.num_heads <= 0 || d.num_kv_heads <= 0) return false;
+    mi_kv_segment fs[8];
+    mi::ChainStep c{};
+    c.num_segments = live_segments(segs_, fs);
+    if (c.num_segments < 0) return false;
+    c.segments = fs;
+    c.rows = rows_args();
+    c.q = d.q;
+    c.k = d.k;
+    c.v = d.v;
+    c.q_bias = bias ? d.q_bias : nullptr;
+    c.k_bias = bias ? d.k_bias : nullptr;
+    c.v_bias = bias ? d.v_bias : nullptr;
+    c.q_weight = norm ? d.q_norm : nullptr;
+    c.k_weight = norm ? d.k_norm : nullptr;
+    c.qk_eps = norm ? d.qk_norm_eps : 0.0f;
+    c.positions = d.positions;
+    c.inv_freq_host = inv_freq_.data();
+    c.Hq = d.num_heads;
+    c.Hkv = d.num_kv_heads;
+    c.head_dim = d.head_dim;
+    c.k_cache = d.k_cache;
+    c.v_cache = d.v_cache;
+    c.layer = d.layer;
+    c.num_blocks = d.num_blocks;
+    c.block_size = d.block_size;
+    c.gate = d.gate;
+    c.up = d.up;
+    c.act_out = d.act_out;
+    c.act_n = d.T * d.intermediate_size;
+    c.gelu = d.act;
+    c.logits = d.logits;
+    c.probs = d.probs;
+    c.next_tokens = d.next_tokens;
+    c.N = d.logit_rows;
+    c.vocab = d.vocab;
+    c.workspace = d.sample_ws;
+    c.workspace_bytes = d.sample_ws_bytes;
+    const int st = mi::chain_step(c, sv(s));
+    if (st == MI_ERR_UNSUPPORTED) return false;
+    check(st, "the step in one launch");
     return true;
 }
 
@@ -257,7 +317,9 @@ void DecoderChain::run(hipStream_t s, DecoderChainHooks* hooks) const {
     }
     // without hooks every GEMM output is there already, so stages 1-2, 5 and 7
     // need not wait for one another: one launch for all three
-    const bool rows = !hooks && last_ >= MI_CHAIN_FINAL_NORM && buffers_apart() && rows_fused(s);
+    const bool apart = !hooks && last_ >= MI_CHAIN_FINAL_NORM && buffers_apart();
+    if (apart && last_ == MI_CHAIN_SAMPLE && step_fused(s)) return;
+    const bool rows = apart && rows_fused(s);
     if (!rows)
         check(mi_embedding_rmsnorm_f16(d.ids, d.embed, d.hidden, d.input_norm, d.normed, T, D,
                                        d.vocab, scale, eps, add1, sv(s)),

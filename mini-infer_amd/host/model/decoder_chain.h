@@ -13,6 +13,7 @@
 #include <string>
 #include <vector>
 
+#include "chain_step.h"
 #include "mi_chain.h"
 
 namespace mini_infer {
@@ -49,7 +50,9 @@ private:
     void validate_() const;
     bool rope_kv_fused(hipStream_t stream) const;
     bool buffers_apart() const;
+    mi::ChainRows rows_args() const;
     bool rows_fused(hipStream_t stream) const;
+    bool step_fused(hipStream_t stream) const;
 
     mi_chain_desc d_;
     int last_;

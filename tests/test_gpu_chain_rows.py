@@ -1,6 +1,6 @@
-"""GPU parity of the chain's row-wise stages in one launch (hookless chains that
-run to the final norm) against the same stages issued one by one through the C
-ABI: the residual stream bit for bit without the blocks' output norms, and every
+"""GPU parity of the chain's stages in shared launches.  The row-wise stages (hookless
+chains that run to the final norm) against the same stages issued one by one
+through the C ABI: the residual stream bit for bit without the blocks' output norms, and every
 norm within one fp16 ulp of the separate kernel's (the two may sum the squares
 of a row in another order).  A caller that reuses one scratch buffer for several
 stages gets the sequential result."""
@@ -125,3 +125,52 @@ def test_wide_tokens_into_the_cache(mk, dev, Hq, Hkv, hd, kind):
     torch.cuda.synchronize()
     assert torch.equal(t["q"], q) and torch.equal(t["k"], k) and torch.equal(t["v"], v)
     assert torch.equal(t["k_cache"], kc) and torch.equal(t["v_cache"], vc)
+
+
+SMALL = dict(hidden_size=64, intermediate_size=72, num_heads=2, num_kv_heads=1, head_dim=64,
+             vocab=9000, use_qk_norm=0)
+
+
+# one token; the tiles' and vectors' edges; every rotation and head width; chunks of
+# either size, ragged vocabularies, and more logit rows than one launch keeps resident
+@pytest.mark.parametrize("n_decode,prefill,rows,kw", [
+    (1, 0, 1, {}),
+    (3, 0, 2, dict(vocab=8192, hidden_size=2048, intermediate_size=2048)),
+    (5, 6, 3, dict(vocab=8201, hidden_size=2056, head_dim=128, qkv_bias=1)),
+    (2, 40, 9, dict(vocab=16391, hidden_size=4096, num_heads=28, num_kv_heads=5, head_dim=128,
+                    use_qk_norm=1)),
+    (7, 33, 5, dict(head_dim=256, num_heads=8, num_kv_heads=4, use_qk_norm=1, double_norm=1,
+                    norm_add_one=1, embed_scale=1, act=1)),
+    (4, 0, 60, dict(vocab=152064, num_heads=4, qkv_bias=1)),
+    (4, 0, 24, dict(vocab=262144, double_norm=1)),
+    (4, 0, 500, dict(vocab=32001)),
+    (4, 0, 3, dict(hidden_size=4104)),
+    (4, 0, 3, dict(intermediate_size=7)),
+    (4, 0, 3, dict(head_dim=80)),
+])
+@pytest.mark.parametrize("polls", [True, False])
+def test_step_in_one_launch(mk, dev, n_decode, prefill, rows, kw, polls):
+    """A whole step against the rows, rotation and activation as launches of their
+    own and the sampling entry point: the same bits but for the probabilities,
+    whose row sums may be taken in chunks of another size (one fp16 ulp)."""
+    import torch
+    print(f"[case] step T={n_decode + 2 * prefill} rows={rows} {kw} polls={polls}", flush=True)
+    args = dict(seed=11, n_decode=n_decode, prefills=(prefill,) * 2 if prefill else (),
+                logit_rows=rows, **dict(SMALL, **kw))
+    ref, w = mi_chain.Workload(dev, **args), mi_chain.Workload(dev, **args)
+    ref.run(Stage.FINAL_NORM)
+    probs, tokens = mk.softmax_argmax(ref.t["logits"], ref.t["sample_ws"])
+    names = [n for n in mi_chain._BUFS if n not in ("probs", "next_tokens")]
+    prev = mk.softmax_test_poll_limit(1 << 16 if polls else 0)
+    try:
+        for i in range(2):  # the records serve the next call
+            if i:
+                w.reload("q", "k", "attn_out", "mlp_out")
+            w.run()
+            torch.cuda.synchronize()
+            for n in names:
+                assert torch.equal(w.t[n], ref.t[n]), n
+            assert torch.equal(w.t["next_tokens"], tokens)
+            assert _ulps(w.t["probs"], probs) <= 1
+    finally:
+        mk.softmax_test_poll_limit(prev)

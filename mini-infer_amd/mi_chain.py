@@ -103,13 +103,16 @@ def make_desc(shapes: dict, tensors: dict, segments) -> tuple:
 def run(desc: ChainDesc, last_stage: int = Stage.SAMPLE, stream=None) -> None:
     """Enqueue the chain up to `last_stage` on `stream` (default: torch's
     current stream)."""
-    import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    lib = load_library()
-    st = lib.mi_decoder_chain_run(ctypes.byref(desc), int(last_stage), ctypes.c_void_p(s.cuda_stream))
+    fast = mi_kernels._fast or mi_kernels._load_fast()
+    st = None
+    if type(desc) is ChainDesc:
+        st = fast.chain_run(ctypes.addressof(desc), last_stage, stream)
+    if st is None:
+        st = load_library().mi_decoder_chain_run(ctypes.byref(desc), int(last_stage),
+                                                 mi_kernels._stream(stream))
     if st != 0:
         raise RuntimeError(f"mi_decoder_chain_run failed: status {st} "
-                           f"({lib.mi_decoder_chain_last_error().decode()})")
+                           f"({load_library().mi_decoder_chain_last_error().decode()})")
 
 
 # ---------------------------------------------------------------------------

@@ -14,6 +14,8 @@ ops (``fused_add_rmsnorm``, ``geglu``) and the positions-driven
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from pathlib import Path
 
@@ -114,10 +116,31 @@ def _torch():
     return torch
 
 
+_fast = None
+
+
+def _load_fast():
+    """The native calls (host/python/fast_calls.cpp): each takes the wrapper's arguments
+    and returns its result, or None when it has launched nothing and the wrapper
+    is to check, call and raise by itself."""
+    global _fast
+    load_library()
+    _torch()  # the module is built on torch's libraries
+    p = _HERE / "_mi_fast.so"
+    if not p.exists():
+        raise RuntimeError(f"{p} is not built; run __graft_entry__.build() (or `make -C mini-infer_amd`)")
+    loader = importlib.machinery.ExtensionFileLoader("_mi_fast", str(p))
+    spec = importlib.util.spec_from_file_location("_mi_fast", str(p), loader=loader)
+    mod = importlib.util.module_from_spec(spec)
+    loader.exec_module(mod)
+    _fast = mod
+    return mod
+
+
 def _stream(stream):
-    torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is None:
+        return ctypes.c_void_p((_fast or _load_fast()).current_stream())
+    return ctypes.c_void_p(stream.cuda_stream)
 
 
 def _ptr(t) -> ctypes.c_void_p:
@@ -146,6 +169,9 @@ def _f16():
 
 def rmsnorm(x, weight, y=None, eps: float = 1e-6, add_one: bool = False, stream=None):
     """y = x * rsqrt(mean(x^2) + eps) * (1 + w if add_one else w); x: [N, D]."""
+    r = (_fast or _load_fast()).rmsnorm(x, weight, y, eps, add_one, stream)
+    if r is not None:
+        return r
     _need(x, _f16(), "x"); _need(weight, _f16(), "weight")
     if x.dim() != 2:
         raise ValueError("x must be 2-D [N, D]")
@@ -165,6 +191,9 @@ def rmsnorm(x, weight, y=None, eps: float = 1e-6, add_one: bool = False, stream=
 def fused_add_rmsnorm(x, residual, weight, y=None, eps: float = 1e-6, add_one: bool = False,
                       stream=None):
     """residual <- half(residual + x); y = rmsnorm(residual).  Returns y."""
+    r = (_fast or _load_fast()).fused_add_rmsnorm(x, residual, weight, y, eps, add_one, stream)
+    if r is not None:
+        return r
     _need(x, _f16(), "x"); _need(residual, _f16(), "residual"); _need(weight, _f16(), "weight")
     if x.dim() != 2 or residual.shape != x.shape:
         raise ValueError("x and residual must be 2-D [N, D] of the same shape")
@@ -195,6 +224,9 @@ def _inv_freq_buffer(inv_freq):
 
 def rope_neox(x, cos_t, sin_t, y=None, stream=None):
     """Table-driven NeoX RoPE; x: [B, S, H, D], tables [B*S, D/2]; y may be x."""
+    r = (_fast or _load_fast()).rope_neox(x, cos_t, sin_t, y, stream)
+    if r is not None:
+        return r
     _need(x, _f16(), "x"); _need(cos_t, _f16(), "cos_t"); _need(sin_t, _f16(), "sin_t")
     if x.dim() != 4:
         raise ValueError("x must be 4-D [B, S, H, D]")
@@ -225,6 +257,9 @@ def rope_inv_freq(head_dim: int, theta: float = 1e6):
 
 def rope_tables(inv_freq, positions, cos_t=None, sin_t=None, stream=None):
     """fp16 cos/sin tables [N, half] for device int64 positions [N]."""
+    r = (_fast or _load_fast()).rope_tables(inv_freq, positions, cos_t, sin_t, stream)
+    if r is not None:
+        return r
     torch = _torch()
     _need(positions, torch.int64, "positions")
     arr, p = _inv_freq_buffer(inv_freq)
@@ -244,6 +279,9 @@ def rope_tables(inv_freq, positions, cos_t=None, sin_t=None, stream=None):
 
 def rope_neox_qk(q, k, positions, inv_freq, stream=None):
     """In-place NeoX RoPE of q [T, Hq, hd] and k [T, Hkv, hd] (k may be None)."""
+    r = (_fast or _load_fast()).rope_neox_qk(q, k, positions, inv_freq, stream)
+    if r is not None:
+        return r
     torch = _torch()
     _need(q, _f16(), "q"); _need(positions, torch.int64, "positions")
     if q.dim() != 3:
@@ -269,6 +307,9 @@ def rope_neox_qk(q, k, positions, inv_freq, stream=None):
 def bias_rope_neox_qk(q, k, q_bias, k_bias, positions, inv_freq, stream=None):
     """In place: q = rope(half(q + q_bias)), k = rope(half(k + k_bias)) for
     q [T, Hq, hd], k [T, Hkv, hd] (k may be None), biases [Hq * hd] / [Hkv * hd]."""
+    r = (_fast or _load_fast()).bias_rope_neox_qk(q, k, q_bias, k_bias, positions, inv_freq, stream)
+    if r is not None:
+        return r
     torch = _torch()
     _need(q, _f16(), "q"); _need(q_bias, _f16(), "q_bias"); _need(positions, torch.int64, "positions")
     if q.dim() != 3:
@@ -425,6 +466,10 @@ def qk_norm_rope(q, k, q_weight, k_weight, positions, inv_freq, eps: float = 1e-
                  add_one: bool = False, stream=None):
     """In place: per-head RMSNorm of q [T, Hq, hd] / k [T, Hkv, hd] (k may be
     None) with q_weight / k_weight [hd], then NeoX RoPE at device positions."""
+    r = (_fast or _load_fast()).qk_norm_rope(q, k, q_weight, k_weight, positions, inv_freq, eps,
+                                           add_one, stream)
+    if r is not None:
+        return r
     torch = _torch()
     _need(q, _f16(), "q"); _need(q_weight, _f16(), "q_weight")
     _need(positions, torch.int64, "positions")
@@ -472,10 +517,16 @@ def _binary(fn_name, a, b, out, stream):
 
 
 def swiglu(gate, up, out=None, stream=None):
+    r = (_fast or _load_fast()).swiglu(gate, up, out, stream)
+    if r is not None:
+        return r
     return _binary("mi_swiglu_f16", gate, up, out, stream)
 
 
 def geglu(gate, up, out=None, stream=None):
+    r = (_fast or _load_fast()).geglu(gate, up, out, stream)
+    if r is not None:
+        return r
     return _binary("mi_geglu_f16", gate, up, out, stream)
 
 
@@ -546,6 +597,9 @@ def softmax(x, y=None, workspace=None, stream=None):
     split rows run in one launch.  Without it, split rows run in one launch on
     stream 0 (row records held by the library) and in two launches with a
     per-call workspace on other streams."""
+    r = (_fast or _load_fast()).softmax(x, y, workspace, stream)
+    if r is not None:
+        return r
     _need(x, _f16(), "x")
     if x.dim() != 2:
         raise ValueError("x must be 2-D [N, D]")
@@ -575,6 +629,9 @@ def softmax_argmax(logits, workspace, probs=None, out=None, stream=None):
     """probs = softmax(logits) and out = greedy argmax(logits) in one pass over
     logits [N, V]; `workspace` (softmax_argmax_workspace_bytes bytes) must be
     zero before its first use and kept for this function.  Returns (probs, out)."""
+    r = (_fast or _load_fast()).softmax_argmax(logits, workspace, probs, out, stream)
+    if r is not None:
+        return r
     torch = _torch()
     _need(logits, _f16(), "logits")
     if logits.dim() != 2:
@@ -637,6 +694,9 @@ def exchange_test_mode(mode: int) -> int:
 
 def embedding_gather(ids, table, out=None, check_range: bool = True, stream=None):
     """out[t] = table[ids[t]]; ids int64 (any shape), table [V, H]."""
+    r = (_fast or _load_fast()).embedding_gather(ids, table, out, check_range, stream)
+    if r is not None:
+        return r
     torch = _torch()
     _need(ids, torch.int64, "ids"); _need(table, _f16(), "table")
     if table.dim() != 2:
@@ -659,6 +719,10 @@ def embedding_rmsnorm(ids, table, weight, hidden=None, y=None, scale: float = 1.
                       stream=None):
     """hidden[t] = half(table[ids[t]] * scale), y = rmsnorm(hidden) in one pass;
     returns (hidden, y), each [*ids.shape, D]."""
+    r = (_fast or _load_fast()).embedding_rmsnorm(ids, table, weight, hidden, y, scale, eps, add_one,
+                                                check_range, stream)
+    if r is not None:
+        return r
     torch = _torch()
     _need(ids, torch.int64, "ids"); _need(table, _f16(), "table"); _need(weight, _f16(), "weight")
     if table.dim() != 2:
@@ -757,6 +821,9 @@ def greedy_argmax_test_poll_limit(limit: int) -> int:
 def top_p_sample(logits, p: float, temperature: float, seed: int, out=None, stream=None):
     """int32 [B] top-p samples of logits [B, V] (or [V]) with the reference's
     rule (greedy above 30000 logits); row b draws with seed + b."""
+    r = (_fast or _load_fast()).top_p_sample(logits, p, temperature, seed, out, stream)
+    if r is not None:
+        return r
     torch = _torch()
     _need(logits, _f16(), "logits")
     x = logits if logits.dim() == 2 else logits.view(1, -1)
@@ -777,6 +844,9 @@ def greedy_argmax(logits, out=None, workspace=None, stream=None):
     `workspace` (greedy_argmax_workspace_bytes bytes) must be zero before its
     first use and kept for argmax calls only; split rows then run in one
     launch."""
+    r = (_fast or _load_fast()).greedy_argmax(logits, out, workspace, stream)
+    if r is not None:
+        return r
     torch = _torch()
     _need(logits, _f16(), "logits")
     x = logits if logits.dim() == 2 else logits.view(1, -1)

@@ -199,12 +199,16 @@ __global__ __launch_bounds__(G > 64 ? G : 256) void softmax_reg_kernel(const hal
 
 // Launch shape for softmax_reg_kernel: the fewest lanes per row (8, 16, 32,
 // 64, then 128, 256 or 1024 as whole workgroups) that hold the row in at most
-// kRegVpt vectors each, else 1024 lanes with up to 8.  128 lanes stop at
+// 3 vectors each (of 8 to 64 lanes) or 4, else 1024 lanes with up to 8.  (3
+// against 4 in a wave: [57344, 512] 20.7 -> 20.05 us, [14336, 1001] 13.2 -> 12.3,
+// [20000, 256] 5.04 -> 4.69, [500, 1000] 2.99 -> 2.72, [17108, 1203] level; 2:
+// 18.7 at 1203.)  128 lanes stop at
 // kPairMax vectors, where 256 lanes would leave 3/8 of their slots idle:
 // [20000, 2100] (263 vectors) 41.9 -> 31.1 us, but [20000, 3000] (375) 40.6
 // against 42.3 us with 128.  (More than 4 vectors per lane of a single wave:
 // 47.5 against 44.2 us at [28672, 2047].)  Returns false when the row needs
 // more than 1024 x 8 vectors.
+constexpr int kWaveVpt = 3;
 constexpr int kRegVpt = 4;
 constexpr int64_t kPairMax = 320;
 // At most 8 vectors per lane (rows <= 1024 x 8 x 8 = 65536).  12 fit in
@@ -215,7 +219,7 @@ bool reg_shape(int64_t nv, int& G, int& VPT) {
     static const int kG[] = {8, 16, 32, 64, 128, 256, 1024};
     G = 0;
     for (int g : kG) {
-        if (nv <= (g == 128 ? kPairMax : static_cast<int64_t>(kRegVpt) * g)) {
+        if (nv <= (g == 128 ? kPairMax : static_cast<int64_t>(g <= 64 ? kWaveVpt : kRegVpt) * g)) {
             G = g;
             break;
         }

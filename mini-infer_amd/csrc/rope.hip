@@ -62,6 +62,24 @@ __device__ __forceinline__ void set_elem(typename HVec<VEC>::T& v, int k, float 
     if constexpr (VEC == 1) v = to_half(f); else v[k] = to_half(f);
 }
 
+// The caller's inverse frequencies on the host, for the duration of a call.
+struct InvFreq {
+    const float* v = nullptr;
+    int half = 0;
+};
+bool load_inv_freq(const float* host, int64_t half, InvFreq& out) {
+    if (!host || half <= 0 || half > kMaxHalf) return false;
+    out.v = host;
+    out.half = static_cast<int>(half);
+    return true;
+}
+template <int NF>
+InvFreqN<NF> sized(const InvFreq& inv) {
+    InvFreqN<NF> r;
+    for (int i = 0; i < NF; ++i) r.v[i] = i < inv.half ? inv.v[i] : 0.0f;
+    return r;
+}
+
 // Tokens per 256-lane workgroup, chosen per launch from {1, 2, 4, 8} (see
 // fill_tokens_per_wg); each lane issues the loads of TPW units (one per
 // token for a 256-unit token, the Qwen2.5 case) before the table work.
@@ -75,14 +93,14 @@ __device__ __forceinline__ void set_elem(typename HVec<VEC>::T& v, int k, float 
 // (src/kernels/model_utils_kernel.cu:19), and the sum rotated.
 // (8 tokens: held to 128 VGPRs, 4 waves per SIMD; the compiler otherwise
 // settles at 130 and the residency drops to 3)
-template <int VEC, bool FROM_POS, int TPW, bool BIAS = false>
+template <int VEC, bool FROM_POS, int TPW, bool BIAS, int NF>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(TPW == 8 ? 4 : 1))) void rope_kernel(const half_t* q_in, half_t* q_out, int Hq,
                                                    const half_t* k_in, half_t* k_out, int Hkv,
                                                    const int64_t* __restrict__ positions,
                                                    const half_t* __restrict__ cos_t,
                                                    const half_t* __restrict__ sin_t, int64_t T,
-                                                   int hd, InvFreq inv,
+                                                   int hd, InvFreqN<NF> inv,
                                                    const half_t* __restrict__ bq = nullptr,
                                                    const half_t* __restrict__ bk = nullptr) {
     typedef HVec<VEC> V;
@@ -228,7 +246,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(half_t* q, int Hq, ha
                                                            const half_t* __restrict__ wk,
                                                            const int64_t* __restrict__ positions,
                                                            int64_t T, float eps, float w_bias,
-                                                           InvFreq inv) {
+                                                           InvFreqN<CPH * 8> inv) {
     constexpr int HALF = CPH * 8;
     constexpr int HD = 2 * HALF;
     __shared__ float cs[TPW][2 * kMaxHalf];
@@ -349,7 +367,7 @@ template <int CPH, int P>
 __global__ __launch_bounds__(256) void qk_norm_rope_pipe_kernel(
     half_t* q, int Hq, half_t* k, int Hkv, const half_t* __restrict__ wq,
     const half_t* __restrict__ wk, const int64_t* __restrict__ positions, int64_t T, int G,
-    float eps, float w_bias, InvFreq inv) {
+    float eps, float w_bias, InvFreqN<CPH * 8> inv) {
     constexpr int HALF = CPH * 8;
     constexpr int HD = 2 * HALF;
     constexpr int kTab = 256;  // cos (or sin) entries per table half: G * HALF <= kTab
@@ -480,10 +498,11 @@ __global__ __launch_bounds__(256) void qk_norm_rope_pipe_kernel(
     }
 }
 
+template <int NF>
 __global__ __launch_bounds__(256) void rope_table_kernel(const int64_t* __restrict__ positions,
                                                          half_t* __restrict__ cos_t,
                                                          half_t* __restrict__ sin_t, int64_t N,
-                                                         int half, InvFreq inv) {
+                                                         int half, InvFreqN<NF> inv) {
     const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (idx >= N * half) return;
     const int64_t n = idx / half;
@@ -492,13 +511,6 @@ __global__ __launch_bounds__(256) void rope_table_kernel(const int64_t* __restri
     cos_sin_half(static_cast<float>(positions[n]) * inv.v[i], hc, hs);
     cos_t[idx] = hc;
     sin_t[idx] = hs;
-}
-
-bool load_inv_freq(const float* host, int64_t half, InvFreq& out) {
-    if (!host || half <= 0 || half > kMaxHalf) return false;
-    for (int64_t i = 0; i < half; ++i) out.v[i] = host[i];
-    for (int64_t i = half; i < kMaxHalf; ++i) out.v[i] = 0.0f;
-    return true;
 }
 
 // Tokens per 256-lane workgroup for the one-round kernels: the fewest (1, 2,
@@ -538,11 +550,11 @@ int pick_tokens_per_wg(int64_t T, K1 k1, K2 k2, K4 k4, K8 k8) {
     return best;
 }
 
-template <int VEC, bool FROM_POS, bool BIAS = false>
-int launch_rope_t(const half_t* q_in, half_t* q_out, int hq, const half_t* k_in, half_t* k_out,
+template <int VEC, bool FROM_POS, bool BIAS, int NF>
+int launch_rope_n(const half_t* q_in, half_t* q_out, int hq, const half_t* k_in, half_t* k_out,
                   int hk, const int64_t* positions, const half_t* cos_t, const half_t* sin_t,
                   int64_t T, int d, const InvFreq& inv, hipStream_t s,
-                  const half_t* bq = nullptr, const half_t* bk = nullptr) {
+                  const half_t* bq, const half_t* bk) {
     int tpw = fill_tokens_per_wg((hq + hk) * (d / 2 / VEC));
     // the bias form holds twice the registers per token: 8 tokens of 16-byte
     // units spill (236 bytes of scratch), 4 fit in 122 VGPRs
@@ -555,8 +567,8 @@ int launch_rope_t(const half_t* q_in, half_t* q_out, int hq, const half_t* k_in,
     switch (tpw) {
 #define MI_ROPE_CASE(P)                                                                        \
     case P:                                                                                    \
-        rope_kernel<VEC, FROM_POS, P, BIAS><<<g, b, 0, s>>>(q_in, q_out, hq, k_in, k_out, hk,  \
-                                                            positions, cos_t, sin_t, T, d, inv, \
+        rope_kernel<VEC, FROM_POS, P, BIAS, NF><<<g, b, 0, s>>>(q_in, q_out, hq, k_in, k_out, hk,  \
+                                                            positions, cos_t, sin_t, T, d, sized<NF>(inv), \
                                                             bq, bk);                            \
         break;
         MI_ROPE_CASE(1)
@@ -567,6 +579,22 @@ int launch_rope_t(const half_t* q_in, half_t* q_out, int hq, const half_t* k_in,
         default: return MI_ERR_UNSUPPORTED;
     }
     return launch_status();
+}
+
+template <int VEC, bool FROM_POS, bool BIAS = false>
+int launch_rope_t(const half_t* q_in, half_t* q_out, int hq, const half_t* k_in, half_t* k_out,
+                  int hk, const int64_t* positions, const half_t* cos_t, const half_t* sin_t,
+                  int64_t T, int d, const InvFreq& inv, hipStream_t s,
+                  const half_t* bq = nullptr, const half_t* bk = nullptr) {
+    if constexpr (!FROM_POS)  // the tables hold them
+        return launch_rope_n<VEC, false, BIAS, 1>(q_in, q_out, hq, k_in, k_out, hk, positions, cos_t,
+                                                  sin_t, T, d, inv, s, bq, bk);
+    else if (d <= 128)
+        return launch_rope_n<VEC, true, BIAS, 64>(q_in, q_out, hq, k_in, k_out, hk, positions, cos_t,
+                                                  sin_t, T, d, inv, s, bq, bk);
+    else
+        return launch_rope_n<VEC, true, BIAS, kMaxHalf>(q_in, q_out, hq, k_in, k_out, hk, positions,
+                                                        cos_t, sin_t, T, d, inv, s, bq, bk);
 }
 
 int launch_rope(const half_t* q_in, half_t* q_out, int64_t Hq, const half_t* k_in, half_t* k_out,
@@ -625,7 +653,7 @@ int launch_qk_norm_rope_pipe(half_t* q, int hq, half_t* k, int hk, const half_t*
     if (grid > ngroups) grid = ngroups;
     if (grid > kMaxGridX) grid = kMaxGridX;
     qk_norm_rope_pipe_kernel<CPH, P><<<dim3(static_cast<unsigned>(grid)), dim3(256), 0, s>>>(
-        q, hq, k, hk, wq, wk, positions, T, G, eps, w_bias, inv);
+        q, hq, k, hk, wq, wk, positions, T, G, eps, w_bias, sized<CPH * 8>(inv));
     return launch_status();
 }
 
@@ -653,7 +681,7 @@ int launch_qk_norm_rope_t(half_t* q, int hq, half_t* k, int hk, const half_t* wq
 #define MI_QKN_CASE(P)                                                                          \
     case P:                                                                                     \
         qk_norm_rope_kernel<CPH, P><<<g, b, 0, s>>>(q, hq, k, hk, wq, wk, positions, T, eps,     \
-                                                    w_bias, inv);                               \
+                                                    w_bias, sized<CPH * 8>(inv));               \
         break;
         MI_QKN_CASE(1)
         MI_QKN_CASE(2)
@@ -704,8 +732,8 @@ __global__ __launch_bounds__(256) void rope_kv_scatter_kernel(RopeKv a, InvFreqN
 // `inv` is the first parameter: it sits at offset 0 of the kernel-argument
 // block, which the kernel reads directly (below).
 template <bool BIAS, bool NORM, int CPH>
-__global__ __launch_bounds__(256) void rope_token_kernel(InvFreq inv, half_t* q, half_t* k, int Hq,
-                                                         int Hkv, int hd,
+__global__ __launch_bounds__(256) void rope_token_kernel(InvFreqN<CPH ? CPH * 8 : kMaxHalf> inv,
+                                                         half_t* q, half_t* k, int Hq, int Hkv, int hd,
                                                          const int64_t* __restrict__ positions,
                                                          const half_t* __restrict__ bq,
                                                          const half_t* __restrict__ bk,
@@ -735,7 +763,7 @@ __global__ __launch_bounds__(256) void rope_token_kernel(InvFreq inv, half_t* q,
         const float* ip =
             reinterpret_cast<const float*>(
                 reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr())) +
-            (tid & (kMaxHalf - 1));  // inv.v[tid] (tid < half <= kMaxHalf uses it)
+            (tid & ((CPH ? CPH * 8 : kMaxHalf) - 1));  // inv.v[tid] (tid < half uses it)
         asm volatile("global_load_dword %0, %1, off" : "=v"(inv_l) : "v"(ip) : "memory");
         const bool act = tid < units;
         const int u = act ? tid : 0;
@@ -864,7 +892,7 @@ __device__ __forceinline__ h8 partner_vec(h8 v) {
 // kernel-argument block (explicit arguments are laid out in order from 0).
 template <bool BIAS, bool NORM, int X, int R, int TPW>
 __global__ __launch_bounds__(256) void rope_rows_kernel(
-    InvFreq inv, half_t* q, half_t* k, int Hq, int Hkv, int64_t T,
+    InvFreqN<X * 8> inv, half_t* q, half_t* k, int Hq, int Hkv, int64_t T,
     const int64_t* __restrict__ positions, const half_t* __restrict__ bq, const half_t* __restrict__ bk,
     const half_t* __restrict__ wq, const half_t* __restrict__ wk, float eps, float w_bias) {
     constexpr int HALF = X * 8;  // head_dim / 2
@@ -1035,7 +1063,7 @@ void rope_rows_go(int tpw, dim3 g, hipStream_t s, const InvFreq& inv, half_t* q,
                   int hq, int hk, int64_t T, const int64_t* positions, const half_t* bq,
                   const half_t* bk, const half_t* wq, const half_t* wk, float eps, float w_bias) {
 #define MI_RR_GO(TT)                                                                            \
-    rope_rows_kernel<BI, NO, XX, RR, TT><<<g, dim3(256), 0, s>>>(inv, q, k, hq, hk, T, positions, \
+    rope_rows_kernel<BI, NO, XX, RR, TT><<<g, dim3(256), 0, s>>>(sized<XX * 8>(inv), q, k, hq, hk, T, positions, \
                                                                  bq, bk, wq, wk, eps, w_bias)
     switch (tpw) {
         case 1: MI_RR_GO(1); break;
@@ -1152,25 +1180,25 @@ int rope_qk_one_token(half_t* q, half_t* k, const half_t* bq, const half_t* bk,
         return MI_ERR_UNSUPPORTED;
     const dim3 g(static_cast<unsigned>(T)), b(256);
     const int hq = static_cast<int>(Hq), hk = static_cast<int>(Hkv), d = static_cast<int>(head_dim);
-#define MI_RQ_ARGS inv, q, k, hq, hk, d, positions, bq, bk, wq, wk, eps, w_bias
+#define MI_RQ_ARGS(C) sized<C ? C * 8 : kMaxHalf>(inv), q, k, hq, hk, d, positions, bq, bk, wq, wk, eps, w_bias
 #define MI_RQ_CPH(BIAS)                                                                     \
     switch (head_dim / 16) {                                                                \
-        case 1: rope_token_kernel<BIAS, false, 1><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
-        case 2: rope_token_kernel<BIAS, false, 2><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
-        case 4: rope_token_kernel<BIAS, false, 4><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
-        case 8: rope_token_kernel<BIAS, false, 8><<<g, b, 0, s>>>(MI_RQ_ARGS); break;   \
-        case 16: rope_token_kernel<BIAS, false, 16><<<g, b, 0, s>>>(MI_RQ_ARGS); break; \
-        case 32: rope_token_kernel<BIAS, false, 32><<<g, b, 0, s>>>(MI_RQ_ARGS); break; \
-        default: rope_token_kernel<BIAS, false, 0><<<g, b, 0, s>>>(MI_RQ_ARGS);         \
+        case 1: rope_token_kernel<BIAS, false, 1><<<g, b, 0, s>>>(MI_RQ_ARGS(1)); break;   \
+        case 2: rope_token_kernel<BIAS, false, 2><<<g, b, 0, s>>>(MI_RQ_ARGS(2)); break;   \
+        case 4: rope_token_kernel<BIAS, false, 4><<<g, b, 0, s>>>(MI_RQ_ARGS(4)); break;   \
+        case 8: rope_token_kernel<BIAS, false, 8><<<g, b, 0, s>>>(MI_RQ_ARGS(8)); break;   \
+        case 16: rope_token_kernel<BIAS, false, 16><<<g, b, 0, s>>>(MI_RQ_ARGS(16)); break; \
+        case 32: rope_token_kernel<BIAS, false, 32><<<g, b, 0, s>>>(MI_RQ_ARGS(32)); break; \
+        default: rope_token_kernel<BIAS, false, 0><<<g, b, 0, s>>>(MI_RQ_ARGS(0));         \
     }
     if (norm) {
         switch (head_dim / 16) {
-            case 1: rope_token_kernel<false, true, 1><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
-            case 2: rope_token_kernel<false, true, 2><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
-            case 4: rope_token_kernel<false, true, 4><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
-            case 8: rope_token_kernel<false, true, 8><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
-            case 16: rope_token_kernel<false, true, 16><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
-            case 32: rope_token_kernel<false, true, 32><<<g, b, 0, s>>>(MI_RQ_ARGS); break;
+            case 1: rope_token_kernel<false, true, 1><<<g, b, 0, s>>>(MI_RQ_ARGS(1)); break;
+            case 2: rope_token_kernel<false, true, 2><<<g, b, 0, s>>>(MI_RQ_ARGS(2)); break;
+            case 4: rope_token_kernel<false, true, 4><<<g, b, 0, s>>>(MI_RQ_ARGS(4)); break;
+            case 8: rope_token_kernel<false, true, 8><<<g, b, 0, s>>>(MI_RQ_ARGS(8)); break;
+            case 16: rope_token_kernel<false, true, 16><<<g, b, 0, s>>>(MI_RQ_ARGS(16)); break;
+            case 32: rope_token_kernel<false, true, 32><<<g, b, 0, s>>>(MI_RQ_ARGS(32)); break;
             default: return MI_ERR_UNSUPPORTED;
         }
     } else if (bq) {
@@ -1225,10 +1253,16 @@ extern "C" int mi_rope_tables_f16(const float* inv_freq_host, const int64_t* pos
     if (grid > mi::kMaxGridX) return MI_ERR_UNSUPPORTED;
     const int64_t bytes = total * 2;
     if (mi::overlaps(cos_t, bytes, sin_t, bytes)) return MI_ERR_ALIASING;
-    mi::rope_table_kernel<<<dim3(static_cast<unsigned>(grid)), dim3(256), 0,
-                            mi::as_stream(stream)>>>(positions, static_cast<half_t*>(cos_t),
-                                                     static_cast<half_t*>(sin_t), N,
-                                                     static_cast<int>(half), inv);
+    const dim3 g(static_cast<unsigned>(grid)), b(256);
+    const hipStream_t s = mi::as_stream(stream);
+    auto* c = static_cast<half_t*>(cos_t);
+    auto* sn = static_cast<half_t*>(sin_t);
+    const int hf = static_cast<int>(half);
+    if (half <= 64)
+        mi::rope_table_kernel<64><<<g, b, 0, s>>>(positions, c, sn, N, hf, mi::sized<64>(inv));
+    else
+        mi::rope_table_kernel<mi::kMaxHalf>
+            <<<g, b, 0, s>>>(positions, c, sn, N, hf, mi::sized<mi::kMaxHalf>(inv));
     return mi::launch_status();
 }
 
@@ -1307,9 +1341,7 @@ namespace {
 template <bool BIAS, bool NORM, int CPH, int P, int LPT>
 int rope_kv_p(const RopeKv& a, const float* inv_host, int64_t T, hipStream_t s) {
     constexpr int NF = CPH ? CPH * 8 : kMaxHalf;
-    InvFreqN<NF> inv;
-    const int half = a.hd / 2;
-    for (int i = 0; i < NF; ++i) inv.v[i] = i < half ? inv_host[i] : 0.0f;
+    const InvFreqN<NF> inv = sized<NF>(InvFreq{inv_host, a.hd / 2});
     rope_kv_scatter_kernel<BIAS, NORM, CPH, P, NF, LPT>
         <<<dim3(static_cast<unsigned>(ceil_div(T, 256 / LPT))), dim3(256), 0, s>>>(a, inv, T);
     return launch_status();

@@ -18,13 +18,7 @@ struct KvSegs {
     const int* sp[kMaxKvSegs];
 };
 
-// Everything a launch needs but the inverse frequencies, which travel by value
-// too, as many as the head has (a kernel with 1 KB of arguments took 4.3 us to
-// launch, one with few 2.9).
-template <int NF>
-struct InvFreqN {
-    float v[NF];
-};
+// Everything a launch needs but the inverse frequencies.
 struct RopeKv {
     half_t *q, *k;
     const half_t* v;

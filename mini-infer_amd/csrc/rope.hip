@@ -204,8 +204,9 @@ __attribute__((amdgpu_waves_per_eu(TPW == 8 ? 4 : 1))) void rope_kernel(const ha
             set_elem<VEC>(y2, k, fp32_rounded(b * cv + a * sv));
         }
         if constexpr (VEC == 8) {
-            st8_out<MI_WT_ROPE>(dst, y1);
-            st8_out<MI_WT_ROPE>(dst + half, y2);
+            // (write-through: table form, T = 4096, 28 heads of 128 11.4 -> 12.4 us)
+            st8_stream(dst, y1);
+            st8_stream(dst + half, y2);
         } else {
             V::store(dst, y1);
             V::store(dst + half, y2);
@@ -322,8 +323,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(half_t* q, int Hq, ha
             y1[e] = to_half(fp32_rounded(n1 * cv - n2 * sv));
             y2[e] = to_half(fp32_rounded(n2 * cv + n1 * sv));
         }
-        st8_out<MI_WT_QKNR>(hp + c * 8, y1);
-        st8_out<MI_WT_QKNR>(hp + HALF + c * 8, y2);
+        st8_out<MI_WT_QKNR && whole_lines<CPH>()>(hp + c * 8, y1);
+        st8_out<MI_WT_QKNR && whole_lines<CPH>()>(hp + HALF + c * 8, y2);
     };
 #pragma unroll
     for (int p = 0; p < TPW; ++p) process(threadIdx.x + p * 256, x1[p], x2[p]);
@@ -338,163 +339,6 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(half_t* q, int Hq, ha
             a2 = ld8_stream(hp + HALF + c * 8);
         }
         process(u, a1, a2);
-    }
-}
-
-// Persistent, software-pipelined form of qk_norm_rope_kernel: a grid of
-// about the resident capacity walks groups of G tokens (G * units-per-token
-// <= 256 * P, G * head_dim/2 <= 256), and while it normalises and rotates
-// group g it already holds the loads of the next group in flight and builds
-// that group's cos/sin rows in the other half of a double-buffered LDS table.
-// HBM reads of the next group overlap the writes of the current one, which a
-// single round of load-everything / barrier / store-everything workgroups
-// cannot do.
-//
-// The vector-memory counter retires loads and stores in issue order, so the
-// loop is arranged so that no wait drains more than it needs to:
-//   * each step begins with one full drain -- the current group's data and
-//     the next group's positions, both issued a step earlier, and the last
-//     step's stores -- and only then issues its prefetch, so nothing inside
-//     the step waits for the loads just issued (with loads and stores both
-//     outstanding, the compiler can only wait for a load with a full drain);
-//   * the two register buffers are used ping-pong (no loop-carried copies);
-//   * each lane's table entry (token-in-group, frequency index) is the same in
-//     every group, so its inv_freq is read once.
-// One barrier per group: the table half written in a step was last read in
-// the step before, ahead of this step's barrier.
-
-template <int CPH, int P>
-__global__ __launch_bounds__(256) void qk_norm_rope_pipe_kernel(
-    half_t* q, int Hq, half_t* k, int Hkv, const half_t* __restrict__ wq,
-    const half_t* __restrict__ wk, const int64_t* __restrict__ positions, int64_t T, int G,
-    float eps, float w_bias, InvFreqN<CPH * 8> inv) {
-    constexpr int HALF = CPH * 8;
-    constexpr int HD = 2 * HALF;
-    constexpr int kTab = 256;  // cos (or sin) entries per table half: G * HALF <= kTab
-    __shared__ float cs[2][2 * kTab];
-    // (w + bias) in fp32 for Q heads (row 0) and K heads (row 1), read from
-    // LDS per unit rather than held in 32 registers across the loop; the
-    // loop's first barrier orders these writes before any read.
-    __shared__ float wt[2][HD];
-    for (int i = threadIdx.x; i < 2 * HD; i += 256) {
-        const int r = i / HD, j = i - r * HD;
-        const int hh = j >= HALF ? HALF : 0;  // quad_split within each half
-        wt[r][hh + quad_split(j - hh, HALF)] =
-            (r == 0 || Hkv > 0) ? (float)(r == 0 ? wq : wk)[j] + w_bias : 0.0f;
-    }
-    const int upt = (Hq + Hkv) * CPH;
-    const int c = threadIdx.x & (CPH - 1);
-    const int64_t ngroups = (T + G - 1) / G;
-    const int64_t stride = gridDim.x;
-
-    // A lane's slots are the same (token-in-group, head) pairs in every
-    // group; only the group's first token moves.
-    int slot_t[P];
-    int64_t slot_off[P];  // element offset of the head at token 0 of the group
-    bool slot_k[P], slot_on[P];
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-        const int u = threadIdx.x + p * 256;
-        const int t = u / upt;
-        const int h = (u - t * upt) / CPH;
-        slot_t[p] = t;
-        slot_on[p] = t < G;
-        slot_k[p] = h >= Hq;
-        slot_off[p] = slot_k[p] ? (static_cast<int64_t>(t) * Hkv + (h - Hq)) * HD + c * 8
-                                : (static_cast<int64_t>(t) * Hq + h) * HD + c * 8;
-    }
-    // This lane's table entry.
-    const bool tab_on = static_cast<int>(threadIdx.x) < G * HALF;
-    const int tab_t = threadIdx.x / HALF;
-    const float tab_f = inv.v[threadIdx.x % HALF];
-
-    auto slot_ptr = [&](int p, int64_t tok0) -> half_t* {
-        return slot_k[p] ? k + tok0 * Hkv * HD + slot_off[p] : q + tok0 * Hq * HD + slot_off[p];
-    };
-    auto load_position = [&](int64_t g) -> int64_t {
-        const int64_t tok = g * G + tab_t;
-        return (g < ngroups && tab_on && tok < T) ? positions[tok] : 0;
-    };
-    auto load_group = [&](int64_t g, h8* a1, h8* a2) {
-        const int64_t tok0 = g * G;
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            a1[p] = h8(0);
-            a2[p] = h8(0);
-            if (slot_on[p] && tok0 + slot_t[p] < T) {
-                const half_t* hp = slot_ptr(p, tok0);
-                a1[p] = ld8_stream(hp);
-                a2[p] = ld8_stream(hp + HALF);
-            }
-        }
-    };
-    auto build_table = [&](int64_t pos, float* tab) {
-        if (tab_on) {
-            half_t hc, hs;
-            cos_sin_half(static_cast<float>(pos) * tab_f, hc, hs);
-            const int li = tab_t * HALF + quad_split(threadIdx.x - tab_t * HALF, HALF);
-            tab[li] = (float)hc;
-            tab[kTab + li] = (float)hs;
-        }
-    };
-    auto process = [&](int64_t g, const float* tab, const h8* a1, const h8* a2) {
-        const int64_t tok0 = g * G;
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            float ss = pair_sumsq(a1[p], a2[p]);
-            ss = group_sum<CPH>(ss);
-            if (!slot_on[p] || tok0 + slot_t[p] >= T) continue;
-            const float rrms = rsqrtf(ss / static_cast<float>(HD) + eps);
-            // weights and table in the quad_split layout: entry e of this
-            // lane's group at c*4 + (e & 3), plus HALF/2 for e >= 4
-            const float* w = &wt[slot_k[p] ? 1 : 0][c * 4];
-            const float* cst = tab + slot_t[p] * HALF + c * 4;
-            h8 y1, y2;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int le = (e & 4) ? HALF / 2 + (e & 3) : e;
-                const float v1 = (float)to_half((float)a1[p][e] * rrms * w[le]);
-                const float v2 = (float)to_half((float)a2[p][e] * rrms * w[HALF + le]);
-                const float cv = cst[le], sv = cst[kTab + le];
-                y1[e] = to_half(fp32_rounded(v1 * cv - v2 * sv));
-                y2[e] = to_half(fp32_rounded(v2 * cv + v1 * sv));
-            }
-            half_t* hp = slot_ptr(p, tok0);
-            st8_out<MI_WT_QKNR>(hp, y1);
-            st8_out<MI_WT_QKNR>(hp + HALF, y2);
-        }
-    };
-
-    int64_t g = blockIdx.x;
-    if (g >= ngroups) return;  // whole workgroup: no barrier is skipped by part of it
-    h8 a1[P], a2[P], b1[P], b2[P];
-    int64_t pos = load_position(g);
-    load_group(g, a1, a2);
-    int64_t pos_next = load_position(g + stride);
-    build_table(pos, cs[0]);
-    // One step: prefetch group g + stride into (n1, n2) and its table into
-    // cs[nb], prefetch the positions of g + 2 * stride, then process g.
-    auto step = [&](int cb, const h8* c1, const h8* c2, h8* n1, h8* n2) -> bool {
-        // Drain here, before the next loads are issued: with stores in
-        // flight every wait on a load is a full drain, so the only wait of a
-        // step must come before its prefetch, not after it.
-        __builtin_amdgcn_s_waitcnt(kDrainVmem);
-        const int64_t gn = g + stride;
-        const bool more = gn < ngroups;
-        if (more) {
-            const int64_t pn = pos_next;
-            pos_next = load_position(gn + stride);
-            load_group(gn, n1, n2);
-            build_table(pn, cs[cb ^ 1]);
-        }
-        __syncthreads();
-        process(g, cs[cb], c1, c2);
-        g = gn;
-        return more;
-    };
-    for (;;) {
-        if (!step(0, a1, a2, b1, b2)) break;
-        if (!step(1, b1, b2, a1, a2)) break;
     }
 }
 
@@ -627,51 +471,14 @@ int launch_rope(const half_t* q_in, half_t* q_out, int64_t Hq, const half_t* k_i
                                    inv, s);
 }
 
-// MI_QKN_PIPE=0 selects the one-round kernel for every shape (measurement).
-#ifndef MI_QKN_PIPE
-#define MI_QKN_PIPE 1
-#endif
-
-// Pipelined launch: P register slots per lane (launched with P = 1, a
-// token's units in one slot), G tokens per group (as many as the slots and
-// the table hold), and a grid of the resident capacity, so every workgroup stays
-// resident and walks ngroups / grid groups.  Measured at T = 6064, Qwen2.5
-// heads: 63% of HBM peak against 56% for the one-round kernel; two tokens
-// per step (P = 2) and a grid of twice the capacity both measured lower.
-template <int CPH, int P>
-int launch_qk_norm_rope_pipe(half_t* q, int hq, half_t* k, int hk, const half_t* wq,
-                             const half_t* wk, const int64_t* positions, int64_t T, float eps,
-                             float w_bias, const InvFreq& inv, hipStream_t s) {
-    constexpr int HALF = CPH * 8;
-    const int upt = (hq + hk) * CPH;
-    int G = (256 * P) / upt;
-    if (G > 256 / HALF) G = 256 / HALF;
-    const int64_t ngroups = ceil_div(T, G);
-    const int64_t cap =
-        resident_workgroups(reinterpret_cast<const void*>(qk_norm_rope_pipe_kernel<CPH, P>), 256);
-    int64_t grid = cap > 0 ? cap : ngroups;
-    if (grid > ngroups) grid = ngroups;
-    if (grid > kMaxGridX) grid = kMaxGridX;
-    qk_norm_rope_pipe_kernel<CPH, P><<<dim3(static_cast<unsigned>(grid)), dim3(256), 0, s>>>(
-        q, hq, k, hk, wq, wk, positions, T, G, eps, w_bias, sized<CPH * 8>(inv));
-    return launch_status();
-}
-
 template <int CPH>
 int launch_qk_norm_rope_t(half_t* q, int hq, half_t* k, int hk, const half_t* wq,
                           const half_t* wk, const int64_t* positions, int64_t T, float eps,
                           float w_bias, const InvFreq& inv, hipStream_t s) {
-    // The pipelined kernel when a token's units fit one register slot per
-    // lane (<= 256 units).  With 2 or 4 slots (P = 2, 4) its register use
-    // (128 / 194 VGPRs) cost more occupancy than the pipelining gained: the
-    // one-round kernel below measured 2-11 points faster for 32|8, 32|32,
-    // 16|8 x 256 and 64|8 heads, so only P = 1 is launched.
-    if (MI_QKN_PIPE && (hq + hk) * CPH <= 256)
-        return launch_qk_norm_rope_pipe<CPH, 1>(q, hq, k, hk, wq, wk, positions, T, eps, w_bias,
-                                                inv, s);
     // (the lane-fill rule of the RoPE kernel measured 2-3 points lower here)
-    const int tpw = pick_tokens_per_wg(T, qk_norm_rope_kernel<CPH, 1>, qk_norm_rope_kernel<CPH, 2>,
-                                       qk_norm_rope_kernel<CPH, 4>, qk_norm_rope_kernel<CPH, 8>);
+    int tpw = pick_tokens_per_wg(T, qk_norm_rope_kernel<CPH, 1>, qk_norm_rope_kernel<CPH, 2>,
+                                 qk_norm_rope_kernel<CPH, 4>, qk_norm_rope_kernel<CPH, 8>);
+    while (tpw < 8 && ceil_div(T, tpw) > kMaxGridX) tpw *= 2;
     const int64_t grid = ceil_div(T, tpw);
     if (grid > kMaxGridX) return MI_ERR_UNSUPPORTED;
     if (static_cast<int64_t>(tpw) * (hq + hk) * CPH >= (int64_t{1} << 22))
@@ -831,8 +638,9 @@ __global__ __launch_bounds__(256) void rope_token_kernel(InvFreqN<CPH ? CPH * 8 
             y1[e] = to_half(fp32_rounded(a * cv - bb * sv));
             y2[e] = to_half(fp32_rounded(bb * cv + a * sv));
         }
-        st8_out<NORM ? MI_WT_QKNR : MI_WT_ROPE>(hp + c * 8, y1);
-        st8_out<NORM ? MI_WT_QKNR : MI_WT_ROPE>(hp + half + c * 8, y2);
+        constexpr bool WT = (NORM ? MI_WT_QKNR : MI_WT_ROPE) && whole_lines<CPH>();
+        st8_out<WT>(hp + c * 8, y1);
+        st8_out<WT>(hp + half + c * 8, y2);
     }
 }
 
@@ -1143,6 +951,45 @@ int rope_qk_rows(half_t* q, half_t* k, const half_t* bq, const half_t* bk,
     return launch_status();
 }
 
+template <bool BIAS, bool NORM, int CPH, int P, int LPT>
+int rope_kv_p(const RopeKv& a, const float* inv_host, int64_t T, hipStream_t s) {
+    constexpr int NF = CPH ? CPH * 8 : kMaxHalf;
+    const InvFreqN<NF> inv = sized<NF>(InvFreq{inv_host, a.hd / 2});
+    rope_kv_scatter_kernel<BIAS, NORM, CPH, P, NF, LPT>
+        <<<dim3(static_cast<unsigned>(ceil_div(T, 256 / LPT))), dim3(256), 0, s>>>(a, inv, T);
+    return launch_status();
+}
+// slots: the larger of the token's units and V vectors
+template <bool BIAS, bool NORM, int CPH>
+int rope_kv_cph(const RopeKv& a, const float* inv, int64_t T, int64_t slots, hipStream_t s) {
+    const int64_t lanes = std::max<int64_t>(slots, a.hd / 2);  // a lane per cos/sin entry too
+    if (lanes <= 64) return rope_kv_p<BIAS, NORM, CPH, 1, 64>(a, inv, T, s);
+    if (lanes <= 128) return rope_kv_p<BIAS, NORM, CPH, 1, 128>(a, inv, T, s);
+    if (slots <= 256) return rope_kv_p<BIAS, NORM, CPH, 1, 256>(a, inv, T, s);
+    if constexpr (CPH == 1 || CPH == 2) {
+        return MI_ERR_UNSUPPORTED;  // more than 128 heads of 16 or 32
+    } else {
+        if (slots <= 512) return rope_kv_p<BIAS, NORM, CPH, 2, 256>(a, inv, T, s);
+        return rope_kv_p<BIAS, NORM, CPH, 3, 256>(a, inv, T, s);
+    }
+}
+template <bool BIAS, bool NORM>
+int rope_kv_go(const RopeKv& a, const float* inv, int64_t T, int64_t slots, hipStream_t s) {
+    switch (a.hd / 16) {
+        case 1: return rope_kv_cph<BIAS, NORM, 1>(a, inv, T, slots, s);
+        case 2: return rope_kv_cph<BIAS, NORM, 2>(a, inv, T, slots, s);
+        case 4: return rope_kv_cph<BIAS, NORM, 4>(a, inv, T, slots, s);
+        case 8: return rope_kv_cph<BIAS, NORM, 8>(a, inv, T, slots, s);
+        case 16: return rope_kv_cph<BIAS, NORM, 16>(a, inv, T, slots, s);
+        case 32: return rope_kv_cph<BIAS, NORM, 32>(a, inv, T, slots, s);
+        default:
+            if constexpr (NORM)
+                return MI_ERR_UNSUPPORTED;  // head_dim not 16 * 2^k
+            else
+                return rope_kv_cph<BIAS, false, 0>(a, inv, T, slots, s);
+    }
+}
+
 // RoPE of Q and K from positions (+ the Q/K bias, or the Q/K norm) through
 // rope_token_kernel: one token per 256-lane workgroup, head_dim's lane split at
 // compile time.  Against rope_kernel at T = 6064 (plain / with the bias):
@@ -1151,15 +998,23 @@ int rope_qk_rows(half_t* q, half_t* k, const half_t* bq, const half_t* bk,
 // 13.3 -> 12.1 / 15.4 -> 13.7, 96 units 9.4 -> 9.1; below that plain RoPE is
 // faster in rope_kernel, which packs several tokens per workgroup (64 units
 // 7.3 against 7.6 us), while the bias form there is not (40 units 17.0
-// against 7.4 us).  MI_ERR_UNSUPPORTED: the caller runs rope_kernel.
-// With the Q/K norm (against qk_norm_rope_pipe_kernel, T = 6064): 256 units
-// 19.5 -> 17.9 us (T = 4096: 13.8 -> 12.8, T = 64: 4.2 -> 3.1), 192 units
-// 15.5 -> 14.1, 144 units 14.6 -> 13.0; 96 units 9.5 against 10.1 us, so the
-// norm form takes tokens of 120 units and more.
+// against 7.4 us).  MI_ERR_UNSUPPORTED: the caller runs rope_kernel, or with the
+// norm qk_norm_rope_kernel.
+//
+// Two kinds of token go through rope_kv_scatter_kernel, with no cache to write:
+//  * wide ones, of 257 to 768 units, two or three per lane, in batches of up to
+//    kWideMaxTokens: 32 + 8 heads of 128 with the bias T = 1 3.7 -> 2.7 us, T = 1000
+//    6.5 -> 5.5 (the norm 6.6 -> 5.9), but 16.8 -> 17.3 at T = 4096; heads whose
+//    halves are no whole lines in any batch (32 + 32 of 80, T = 4096: 22.3 -> 19.7);
+//  * narrow ones, of up to 128 units with the bias or the norm, two or four per
+//    workgroup, from kNarrowMinTokens on: 14 + 2 heads of 64, T = 4096 6.3 -> 4.9 us
+//    (bias), 6.1 -> 5.4 (norm), but 3.0 against 2.3 at T = 64, where one token per
+//    workgroup keeps more CUs busy.
 #ifndef MI_RKV_MIN_UNITS
 #define MI_RKV_MIN_UNITS 80
 #endif
-constexpr int64_t kRkvMinUnitsNorm = 120;
+constexpr int64_t kWideMaxTokens = 1024;
+constexpr int64_t kNarrowMinTokens = 2048;
 int rope_qk_one_token(half_t* q, half_t* k, const half_t* bq, const half_t* bk,
                       const int64_t* positions, const InvFreq& inv, int64_t T, int64_t Hq,
                       int64_t Hkv, int64_t head_dim, hipStream_t s,
@@ -1172,12 +1027,33 @@ int rope_qk_one_token(half_t* q, half_t* k, const half_t* bq, const half_t* bk,
     }
     const int64_t units = (Hq + Hkv) * (head_dim / 16);
     const bool norm = wq != nullptr;
-    const int64_t min_units = norm ? kRkvMinUnitsNorm : (bq ? 1 : MI_RKV_MIN_UNITS);
-    if (head_dim % 16 != 0 || head_dim / 2 > kMaxHalf || units > 256 || units < min_units ||
-        T > kMaxGridX || !aligned16(q) || (Hkv > 0 && !aligned16(k)) ||
-        (bq && !aligned16(bq)) || (bk && Hkv > 0 && !aligned16(bk)) ||
-        (norm && (!aligned16(wq) || (Hkv > 0 && !aligned16(wk)))))
+    const bool aligned = aligned16(q) && (Hkv == 0 || aligned16(k)) && (!bq || aligned16(bq)) &&
+                         (!bk || Hkv == 0 || aligned16(bk)) &&
+                         (!norm || (aligned16(wq) && (Hkv == 0 || aligned16(wk))));
+    if (head_dim % 16 != 0 || head_dim / 2 > kMaxHalf || T > kMaxGridX || units < 1 || !aligned)
         return MI_ERR_UNSUPPORTED;
+    const bool wide = units > 256 && units <= 768 && (T <= kWideMaxTokens || head_dim % 128 != 0);
+    const bool narrow = (bq || norm) && units <= 128 && head_dim <= 256 && T >= kNarrowMinTokens;
+    if (wide || narrow) {  // rope_kv_scatter_kernel with no segment
+        RopeKv a{};
+        a.q = q;
+        a.k = k;
+        a.Hq = static_cast<int>(Hq);
+        a.Hkv = static_cast<int>(Hkv);
+        a.hd = static_cast<int>(head_dim);
+        a.positions = positions;
+        a.bq = bq;
+        a.bk = bk;
+        a.wq = wq;
+        a.wk = wk;
+        a.eps = eps;
+        a.w_bias = w_bias;
+        a.bs = 1;
+        return norm ? rope_kv_go<false, true>(a, inv.v, T, units, s)
+               : bq ? rope_kv_go<true, false>(a, inv.v, T, units, s)
+                    : rope_kv_go<false, false>(a, inv.v, T, units, s);
+    }
+    if (units > 256 || (!bq && !norm && units < MI_RKV_MIN_UNITS)) return MI_ERR_UNSUPPORTED;
     const dim3 g(static_cast<unsigned>(T)), b(256);
     const int hq = static_cast<int>(Hq), hk = static_cast<int>(Hkv), d = static_cast<int>(head_dim);
 #define MI_RQ_ARGS(C) sized<C ? C * 8 : kMaxHalf>(inv), q, k, hq, hk, d, positions, bq, bk, wq, wk, eps, w_bias
@@ -1337,45 +1213,6 @@ extern "C" int mi_bias_rope_neox_qk_f16(void* q, void* k, const void* q_bias, co
 
 namespace mi {
 namespace {
-
-template <bool BIAS, bool NORM, int CPH, int P, int LPT>
-int rope_kv_p(const RopeKv& a, const float* inv_host, int64_t T, hipStream_t s) {
-    constexpr int NF = CPH ? CPH * 8 : kMaxHalf;
-    const InvFreqN<NF> inv = sized<NF>(InvFreq{inv_host, a.hd / 2});
-    rope_kv_scatter_kernel<BIAS, NORM, CPH, P, NF, LPT>
-        <<<dim3(static_cast<unsigned>(ceil_div(T, 256 / LPT))), dim3(256), 0, s>>>(a, inv, T);
-    return launch_status();
-}
-// slots: the larger of the token's units and V vectors
-template <bool BIAS, bool NORM, int CPH>
-int rope_kv_cph(const RopeKv& a, const float* inv, int64_t T, int64_t slots, hipStream_t s) {
-    const int64_t lanes = std::max<int64_t>(slots, a.hd / 2);  // a lane per cos/sin entry too
-    if (lanes <= 64) return rope_kv_p<BIAS, NORM, CPH, 1, 64>(a, inv, T, s);
-    if (lanes <= 128) return rope_kv_p<BIAS, NORM, CPH, 1, 128>(a, inv, T, s);
-    if (slots <= 256) return rope_kv_p<BIAS, NORM, CPH, 1, 256>(a, inv, T, s);
-    if constexpr (CPH == 1 || CPH == 2) {
-        return MI_ERR_UNSUPPORTED;  // more than 128 heads of 16 or 32
-    } else {
-        if (slots <= 512) return rope_kv_p<BIAS, NORM, CPH, 2, 256>(a, inv, T, s);
-        return rope_kv_p<BIAS, NORM, CPH, 3, 256>(a, inv, T, s);
-    }
-}
-template <bool BIAS, bool NORM>
-int rope_kv_go(const RopeKv& a, const float* inv, int64_t T, int64_t slots, hipStream_t s) {
-    switch (a.hd / 16) {
-        case 1: return rope_kv_cph<BIAS, NORM, 1>(a, inv, T, slots, s);
-        case 2: return rope_kv_cph<BIAS, NORM, 2>(a, inv, T, slots, s);
-        case 4: return rope_kv_cph<BIAS, NORM, 4>(a, inv, T, slots, s);
-        case 8: return rope_kv_cph<BIAS, NORM, 8>(a, inv, T, slots, s);
-        case 16: return rope_kv_cph<BIAS, NORM, 16>(a, inv, T, slots, s);
-        case 32: return rope_kv_cph<BIAS, NORM, 32>(a, inv, T, slots, s);
-        default:
-            if constexpr (NORM)
-                return MI_ERR_UNSUPPORTED;  // head_dim not 16 * 2^k
-            else
-                return rope_kv_cph<BIAS, false, 0>(a, inv, T, slots, s);
-    }
-}
 
 // Shared checks and arguments of rope_kv_scatter_kernel.  q_bias / k_bias / v_bias (all
 // or none) and q_weight / k_weight (NORM) exclude each other.  wide: tokens of

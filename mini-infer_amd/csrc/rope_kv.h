@@ -78,8 +78,8 @@ __device__ __forceinline__ int64_t kv_row(const RopeKv& a, int64_t tok, int64_t 
 // value is rounded to fp16 where the reference stores it, and the rotation takes
 // it from registers.  CPH at compile time (shifts for the lane -> (head, slice)
 // split: 0.3-0.4 us less than CPH = 0 at Qwen2.5's shapes, T = 6064); CPH = 0:
-// head_dim known at run time (no norm).  Cache rows are written through to
-// memory ("nt sc1"), as the scatter kernel writes them.
+// head_dim known at run time (no norm).  Rows are written through to
+// memory ("nt sc1") where their pieces are whole lines.
 // P = 2 (32 + 8 heads of 128, 320 units, T = 1048 in two segments): 13.5 us with the
 // gather before it, against 19.7 for RoPE and two scatters after it.
 // LPT: lanes per token -- 256, or 64 or 128 for tokens of so few units, so that a
@@ -92,6 +92,9 @@ __device__ __forceinline__ void rope_kv_token(const RopeKv& a, const float* inv,
     static_assert(LPT == 256 || P == 1, "several tokens per workgroup take one slot per lane");
     static_assert(!(BIAS && NORM), "no model adds a QKV bias before a Q/K norm");
     static_assert(!NORM || (CPH >= 1 && CPH <= 32), "the norm needs head_dim / 16 at compile time");
+    // written through (rope_math.h); with several units per lane the stores' wait
+    // states would queue behind one another (T = 1, 320 units: 3.2 -> 2.7 us)
+    constexpr bool WT = (NORM ? MI_WT_QKNR : MI_WT_ROPE) && whole_lines<CPH>() && P == 1;
     const int half = CPH ? CPH * 8 : a.hd >> 1;
     const int cph = CPH ? CPH : half >> 3;  // 16-byte slices per half head
     const int Hq = a.Hq, Hkv = a.Hkv;
@@ -187,12 +190,12 @@ __device__ __forceinline__ void rope_kv_token(const RopeKv& a, const float* inv,
             y1[e] = to_half(fp32_rounded(xa * cv - xb * sv));
             y2[e] = to_half(fp32_rounded(xb * cv + xa * sv));
         }
-        st8_out<NORM ? MI_WT_QKNR : MI_WT_ROPE>(hp[p] + c[p] * 8, y1);
-        st8_out<NORM ? MI_WT_QKNR : MI_WT_ROPE>(hp[p] + half + c[p] * 8, y2);
+        st8_out<WT>(hp[p] + c[p] * 8, y1);
+        st8_out<WT>(hp[p] + half + c[p] * 8, y2);
         if (h[p] >= Hq && dst_base >= 0) {
             half_t* kd = a.k_cache + dst_base + static_cast<int64_t>(h[p] - Hq) * a.bs * (2 * half);
-            st8_stream_wt(kd + c[p] * 8, y1);
-            st8_stream_wt(kd + half + c[p] * 8, y2);
+            st8_out<WT>(kd + c[p] * 8, y1);
+            st8_out<WT>(kd + half + c[p] * 8, y2);
         }
     }
 #pragma unroll
@@ -210,8 +213,7 @@ __device__ __forceinline__ void rope_kv_token(const RopeKv& a, const float* inv,
             else
                 vh = small_div(vj, 1.0f / static_cast<float>(per_head));
             const int vd = (vj - vh * per_head) * 8;
-            st8_stream_wt(a.v_cache + dst_base + static_cast<int64_t>(vh) * a.bs * (2 * half) + vd,
-                          vv[p]);
+            st8_out<WT>(a.v_cache + dst_base + static_cast<int64_t>(vh) * a.bs * (2 * half) + vd, vv[p]);
         }
     }
 }

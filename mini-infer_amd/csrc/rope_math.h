@@ -7,7 +7,11 @@
 #include "rope_sincos.h"
 
 // Stores of the in-place RoPE and fused Q/K-norm + RoPE kernels: write-through
-// ("nt sc1", st8_stream_wt) measured 1-3 points faster than plain non-temporal.
+// ("nt sc1", st8_stream_wt) measured 1-3 points faster than plain non-temporal
+// where each store instruction's pieces are whole 128-byte lines -- the halves of
+// heads of 128, 256, 512 -- and far slower where they are not, each line then being
+// written through in parts: T = 4096 in place, 32 + 32 heads of 80 33.3 -> 20.0 us
+// without it, 32 + 8 of 80 20.8 -> 12.6, 14 + 2 of 64 with a bias 6.3 -> 4.9.
 #ifndef MI_WT_ROPE
 #define MI_WT_ROPE 1
 #endif
@@ -18,6 +22,11 @@
 namespace mi {
 
 constexpr int kMaxHalf = 256;  // head_dim <= 512
+
+// Whether the halves of a head of 16 * CPH elements are whole 128-byte lines
+// (CPH = 0, any other head_dim: no).
+template <int CPH>
+constexpr bool whole_lines() { return CPH > 0 && CPH % 8 == 0; }
 
 // LDS position of element i of a half-row of n entries (n a multiple of 8),
 // for lanes that each read the 8 entries c*8 .. c*8+7 as two 16-byte LDS

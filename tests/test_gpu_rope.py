@@ -188,11 +188,10 @@ def test_position_zero_is_identity(mk, orc, dev):
 def test_qk_norm_rope(mk, orc, dev, T, Hq, Hkv, hd):
     """Fused Q/K RMSNorm + RoPE == the reference's norm-then-rope composition
     (src/layers/attention.cpp:754-780), within rtol = atol = 1e-3.  Shapes
-    cover both launch forms: the pipelined kernel (at most 256 lanes per
-    token) with token groups of 1 to 32 tokens, a ragged last group and
-    groups walked several times per workgroup (T = 20000, 6064); and the
-    one-round kernel at 48, 96 and 144 heads of 128 (384 to 1152 lanes per
-    token, one to five units per lane)."""
+    cover the launch forms: one token per workgroup (at most 256 units), several
+    (20000 of 40 units), two or three units per lane (500 of 768), and the
+    kernel of any width at 48 and 144 heads of 128 (384 units in a large
+    batch, 1152)."""
     _case(f"qk_norm_rope T={T} Hq={Hq} Hkv={Hkv} hd={hd}")
     rng = np.random.default_rng(T * 7 + hd)
     q = normal_f16(rng, (T, Hq, hd))
@@ -209,6 +208,51 @@ def test_qk_norm_rope(mk, orc, dev, T, Hq, Hkv, hd):
     if Hkv:
         ref, n16 = qk_norm_rope_ref(orc, k, wk, pos, inv)
         assert_norm_rope_close(to_host(kd), ref, n16, what="k")
+
+
+# either side of one, two and three units per lane, of two and four tokens per
+# workgroup (the last one part-filled), and of the token counts the forms change at
+@pytest.mark.parametrize("T,Hq,Hkv,hd", [(1, 32, 1, 128), (1024, 30, 3, 128), (1025, 30, 3, 128),
+                                         (3, 64, 1, 128), (2, 95, 1, 128), (2, 96, 1, 128),
+                                         (9, 40, 12, 80), (1100, 40, 12, 80), (5, 3, 50, 96),
+                                         (2047, 14, 2, 64), (2048, 14, 2, 64), (2049, 17, 0, 64),
+                                         (2051, 0, 3, 64), (2049, 14, 2, 128), (2049, 14, 3, 128),
+                                         (2050, 4, 1, 256), (2050, 2, 2, 512), (2053, 5, 2, 48)])
+@pytest.mark.parametrize("kind", ["plain", "bias", "norm"])
+def test_wide_and_narrow_tokens(mk, dev, T, Hq, Hkv, hd, kind):
+    """Every form gives a token the same bits: against the table-driven rotation
+    (after the bias add), and with the norm against the call on a few tokens at a
+    time."""
+    import torch
+    if kind == "norm" and hd & (hd - 1):
+        pytest.skip("the norm takes heads of 16 * 2^k")
+    _case(f"wide / narrow tokens T={T} {Hq}|{Hkv}x{hd} {kind}")
+    rng = np.random.default_rng(T + Hq + hd)
+    q, k = (to_dev(normal_f16(rng, (T, h, hd)), dev) for h in (Hq, Hkv))
+    pos = to_dev(rng.integers(0, 1 << 21, T).astype(np.int64), dev)
+    inv = mk.rope_inv_freq(hd)
+    if kind == "norm":
+        wq, wk = (to_dev(normal_f16(rng, (hd,), 1.0, 0.1), dev) for _ in range(2))
+        q2, k2 = q.clone(), k.clone()
+        mk.qk_norm_rope(q, k if Hkv else None, wq, wk if Hkv else None, pos, inv)
+        for t in range(0, T, max(1, T // 3)):
+            e = min(T, t + max(1, T // 3))
+            mk.qk_norm_rope(q2[t:e], k2[t:e] if Hkv else None, wq, wk if Hkv else None, pos[t:e], inv)
+    else:
+        q2, k2 = q.clone(), k.clone()
+        if kind == "bias":
+            bq, bk = (to_dev(normal_f16(rng, (h * hd,), 0, 0.5), dev) for h in (Hq, Hkv))
+            mk.bias_rope_neox_qk(q, k if Hkv else None, bq, bk if Hkv else None, pos, inv)
+            for x, b, h in ((q2, bq, Hq), (k2, bk, Hkv)):
+                if h:
+                    mk.add_bias(x, b, T, h * hd, T * h * hd)
+        else:
+            mk.rope_neox_qk(q, k if Hkv else None, pos, inv)
+        c, s = mk.rope_tables(inv, pos)
+        for x, h in ((q2, Hq), (k2, Hkv)):
+            if h:
+                mk.rope_neox(x[None], c, s, y=x[None])
+    assert torch.equal(q, q2) and torch.equal(k, k2)
 
 
 def test_qk_norm_rope_huge_positions(mk, orc, dev):

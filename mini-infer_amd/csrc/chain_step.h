@@ -62,7 +62,7 @@ struct ChainStep {
     const void* logits;
     void* probs;
     int32_t* next_tokens;
-    int64_t N, vocab;
+    int64_t N, vocab;  // N = 0: the step without its sampling
     void* workspace;
     int64_t workspace_bytes;
 };

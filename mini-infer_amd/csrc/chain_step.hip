@@ -354,7 +354,7 @@ __attribute__((amdgpu_waves_per_eu(DOUBLE ? 5 : 6))) void chain_step_kernel(
 
 template <int NF, bool DOUBLE>
 int step_go(const ChainStep& c, StepArgs<NF>& a, hipStream_t s) {
-    const int64_t R = ceil_div(c.N, kXcds) * kXcds;
+    const int64_t R = ceil_div(c.N, kXcds) * kXcds;  // 0: a step without sampling
     // every sampling chunk resident at once: at the softmax's own chunk size, or
     // the larger one
     const int64_t cap =
@@ -420,9 +420,15 @@ int chain_step(const ChainStep& c, void* stream) {
                      c.num_segments, /*wide=*/true, kv, slots) != MI_OK ||
         slots > 512)
         return MI_ERR_UNSUPPORTED;
-    StreamPlan sp;
-    if (!softmax_argmax_plan(c.logits, c.probs, c.next_tokens, c.N, c.vocab, c.workspace,
-                             c.workspace_bytes, sp))
+    // Where the launches apart are faster: without the sampling to hide, large
+    // batches (T = 764, Gemma norms 40.9 -> 38.5 us in two launches instead of four,
+    // but T = 5464 138.9 against 142.2); tokens of few units, which RoPE + cache by
+    // itself takes several of per workgroup (14 + 2 heads of 64: T = 2830 37.7 -> 34.3,
+    // but T = 5430 56.5 against 58.8).
+    if ((c.N == 0 && c.rows.T > 1024) || (slots <= 128 && c.rows.T > 4096)) return MI_ERR_UNSUPPORTED;
+    StreamPlan sp{};
+    if (c.N > 0 && !softmax_argmax_plan(c.logits, c.probs, c.next_tokens, c.N, c.vocab, c.workspace,
+                                        c.workspace_bytes, sp))
         return MI_ERR_UNSUPPORTED;
     const hipStream_t s = as_stream(stream);
     return c.head_dim == 256 ? step_plan<128>(c, rows, kv, slots, sp, s)

@@ -246,9 +246,9 @@ bool DecoderChain::rows_fused(hipStream_t s) const {
     return true;
 }
 
-// The whole step in one launch (chain_step.h).  False (nothing launched) for
-// steps it does not take.
-bool DecoderChain::step_fused(hipStream_t s) const {
+// The whole step, or all of it up to the sampling, in one launch (chain_step.h).
+// False (nothing launched) for steps it does not take.
+bool DecoderChain::step_fused(hipStream_t s, bool sample) const {
     const mi_chain_desc& d = d_;
     const bool bias = d.q_bias != nullptr, norm = d.use_qk_norm != 0;
     if ((norm && bias) || d.num_heads <= 0 || d.num_kv_heads <= 0) return false;
@@ -282,17 +282,27 @@ bool DecoderChain::step_fused(hipStream_t s) const {
     c.act_out = d.act_out;
     c.act_n = d.T * d.intermediate_size;
     c.gelu = d.act;
-    c.logits = d.logits;
-    c.probs = d.probs;
-    c.next_tokens = d.next_tokens;
-    c.N = d.logit_rows;
-    c.vocab = d.vocab;
-    c.workspace = d.sample_ws;
-    c.workspace_bytes = d.sample_ws_bytes;
+    if (sample) {
+        c.logits = d.logits;
+        c.probs = d.probs;
+        c.next_tokens = d.next_tokens;
+        c.N = d.logit_rows;
+        c.vocab = d.vocab;
+        c.workspace = d.sample_ws;
+        c.workspace_bytes = d.sample_ws_bytes;
+    }
     const int st = mi::chain_step(c, sv(s));
     if (st == MI_ERR_UNSUPPORTED) return false;
     check(st, "the step in one launch");
     return true;
+}
+
+// Softmax and greedy argmax of the logit rows in one pass.
+void DecoderChain::sample(hipStream_t s) const {
+    const mi_chain_desc& d = d_;
+    check(mi_softmax_argmax_ws_f16(d.logits, d.probs, d.next_tokens, d.logit_rows, d.vocab,
+                                   d.sample_ws, d.sample_ws_bytes, sv(s)),
+          "softmax + greedy argmax");
 }
 
 void DecoderChain::run(hipStream_t s, DecoderChainHooks* hooks) const {
@@ -318,7 +328,11 @@ void DecoderChain::run(hipStream_t s, DecoderChainHooks* hooks) const {
     // without hooks every GEMM output is there already, so stages 1-2, 5 and 7
     // need not wait for one another: one launch for all three
     const bool apart = !hooks && last_ >= MI_CHAIN_FINAL_NORM && buffers_apart();
-    if (apart && last_ == MI_CHAIN_SAMPLE && step_fused(s)) return;
+    if (apart && last_ == MI_CHAIN_SAMPLE && step_fused(s, true)) return;
+    if (apart && step_fused(s, false)) {  // sampling rows that do not fit beside it
+        if (last_ == MI_CHAIN_SAMPLE) sample(s);
+        return;
+    }
     const bool rows = apart && rows_fused(s);
     if (!rows)
         check(mi_embedding_rmsnorm_f16(d.ids, d.embed, d.hidden, d.input_norm, d.normed, T, D,
@@ -427,9 +441,7 @@ void DecoderChain::run(hipStream_t s, DecoderChainHooks* hooks) const {
     // 8. LM head, then the sampling step: softmax and greedy argmax of the
     //    logits rows in one pass
     h.lm_head(d, s);
-    check(mi_softmax_argmax_ws_f16(d.logits, d.probs, d.next_tokens, d.logit_rows, d.vocab,
-                                   d.sample_ws, d.sample_ws_bytes, sv(s)),
-          "softmax + greedy argmax");
+    sample(s);
 }
 
 }  // namespace mini_infer

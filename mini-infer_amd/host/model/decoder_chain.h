@@ -52,7 +52,8 @@ private:
     bool buffers_apart() const;
     mi::ChainRows rows_args() const;
     bool rows_fused(hipStream_t stream) const;
-    bool step_fused(hipStream_t stream) const;
+    bool step_fused(hipStream_t stream, bool sample) const;
+    void sample(hipStream_t stream) const;
 
     mi_chain_desc d_;
     int last_;

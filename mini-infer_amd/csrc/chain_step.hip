@@ -6,7 +6,7 @@
 // back between them: 11 D elements a token move (13 with the norms of the
 // blocks' outputs: those re-read what they wrote).  Held in registers it is
 // written once: 7 D (9 D).  One workgroup of 256 lanes per token, lane j on
-// 16-byte vectors j, j + 256, ...; every load of the row and of the weights is
+// 16-byte vectors j, j + lanes, ...; every load of the row and of the weights is
 // issued first.  The three sums of squares share one barrier, since the second
 // and third residual need no norm's result; with the blocks' outputs
 // normalised first (DOUBLE) those two sums join the first barrier and the two
@@ -32,6 +32,8 @@ struct RowArgs {
     const half_t *w_in, *w_post, *w_fin, *w_attn, *w_mlp;
     int64_t D, vocab;
     float scale, eps, w_bias;
+    int lanes;  // of the 256: rms_row_kernel's for rows of D, so that the norms of the
+                // blocks' outputs and of the residuals are its, bit for bit
 };
 
 // Opaque copies of x.
@@ -59,8 +61,8 @@ __device__ __forceinline__ void chain_row(const RowArgs& r, int64_t t, float* sl
     bool ok[VPT];
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
-        const int64_t c = threadIdx.x + j * 256;
-        ok[j] = c < nv;
+        const int64_t c = threadIdx.x + j * r.lanes;
+        ok[j] = c < nv && static_cast<int>(threadIdx.x) < r.lanes;
         at[j] = (ok[j] ? c : nv - 1) * 8;  // unconditional loads; idle lanes masked below
     }
 #pragma unroll
@@ -211,6 +213,8 @@ bool rows_plan(const ChainRows& c, RowArgs& r) {
     r.w_fin = static_cast<const half_t*>(c.w_final);
     r.w_attn = static_cast<const half_t*>(c.w_attn);
     r.w_mlp = static_cast<const half_t*>(c.w_mlp);
+    const int64_t chunks = c.D / 8, vpt = ceil_div(chunks, 256);
+    r.lanes = static_cast<int>(ceil_div(ceil_div(chunks, vpt), kWave) * kWave);
     r.D = c.D;
     r.vocab = c.vocab;
     r.scale = c.scale;

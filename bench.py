@@ -819,15 +819,16 @@ def cpu_kernel_table(budget_s=1.0):
 
 def chain_bytes(s, segments_tokens):
     """Algorithmic HBM bytes of one chain step (each input read once, each
-    output written once), from the workload's shapes."""
+    output written once: the residual stream stays on chip between the stages,
+    and K's rotated rows reach q / k and the cache from one read), from the
+    workload's shapes."""
     T, D, I, V, N = s["T"], s["hidden_size"], s["intermediate_size"], s["vocab"], s["logit_rows"]
     Hq, Hkv, hd = s["num_heads"], s["num_kv_heads"], s["head_dim"]
     weights = (2 * hd * 2 if s["use_qk_norm"] else 0) + \
         ((Hq + 2 * Hkv) * hd * 2 if s.get("qkv_bias") else 0)       # q/k norm weights, qkv bias
-    return ((T * 8 + 3 * T * D * 2 + D * 2)                           # gather + input norm
+    return ((T * 8 + 7 * T * D * 2 + 3 * D * 2)                       # gather, 2x add, 3x norm
             + (2 * T * (Hq + Hkv) * hd * 2 + T * 8 + weights)         # (bias,) (qk-norm,) rope
-            + (2 * 2 * segments_tokens * Hkv * hd * 2)                # K + V scatter
-            + 2 * (4 * T * D * 2 + D * 2)                             # 2x residual add + norm
+            + (3 * segments_tokens * Hkv * hd * 2)                    # V read, K and V cached
             + 3 * T * I * 2                                           # SwiGLU
             + (2 * N * V * 2 + N * 4))                                # softmax + argmax
 

@@ -11,7 +11,8 @@
 // output that is None is allocated, as the wrapper does), and otherwise None,
 // having launched nothing: an argument is not what the call needs (a tensor on
 // another device, of another type or shape, not contiguous, a subclass with its
-// own ways, one without memory of its own), or the library refused it.  The Python wrapper then makes the call itself and raises what
+// own ways, one without memory of its own, as under torch.vmap), or the library
+// refused it.  The Python wrapper then makes the call itself and raises what
 // there is to raise, so its errors and conversions stay where they were.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -106,13 +107,25 @@ struct Floats {
     const float* data() const { return static_cast<const float*>(view.buf); }
 };
 
-// The library call without the GIL (it may wait for room in the stream's queue).
-template <typename F>
-void launch(F call) {
+// Without the GIL for its lifetime, also where that ends in an exception.
+struct NoGil {
+    PyThreadState* thread = PyEval_SaveThread();
+    NoGil() = default;
+    NoGil(const NoGil&) = delete;
+    ~NoGil() { PyEval_RestoreThread(thread); }
+};
+
+// The library call f(args...) without the GIL (it may wait for room in the
+// stream's queue).  The arguments are values, so that what makes them runs with
+// the GIL held: ptr() throws for a tensor without memory of its own, and the
+// handlers below are Python calls.
+template <typename F, typename... A>
+void launch(F f, A... args) {
     int st;
-    Py_BEGIN_ALLOW_THREADS
-    st = call();
-    Py_END_ALLOW_THREADS
+    {
+        const NoGil released;
+        st = f(args...);
+    }
     need(st == 0);
 }
 
@@ -174,7 +187,7 @@ MI_FAST(rmsnorm) {
         const float eps = static_cast<float>(number(a[3]));
         const int one = truth(a[4]);
         void* s = stream_of(a[5]);
-        launch([&] { return mi_rmsnorm_f16(ptr(x), ptr(w), ptr(y), x.size(0), x.size(1), eps, one, s); });
+        launch(mi_rmsnorm_f16, ptr(x), ptr(w), ptr(y), x.size(0), x.size(1), eps, one, s);
         return out.result();
     });
 }
@@ -190,10 +203,8 @@ MI_FAST(fused_add_rmsnorm) {
         const float eps = static_cast<float>(number(a[4]));
         const int one = truth(a[5]);
         void* s = stream_of(a[6]);
-        launch([&] {
-            return mi_fused_add_rmsnorm_f16(ptr(x), ptr(r), ptr(w), ptr(y), x.size(0), x.size(1),
-                                            eps, one, s);
-        });
+        launch(mi_fused_add_rmsnorm_f16, ptr(x), ptr(r), ptr(w), ptr(y), x.size(0), x.size(1), eps,
+               one, s);
         return out.result();
     });
 }
@@ -207,7 +218,7 @@ PyObject* binary(PyObject* const* a, Py_ssize_t n, F f) {
         const Out out(a[2], x);
         need(out.t->numel() == x.numel());
         void* s = stream_of(a[3]);
-        launch([&] { return f(ptr(x), ptr(y), ptr(*out.t), x.numel(), s); });
+        launch(f, ptr(x), ptr(y), ptr(*out.t), x.numel(), s);
         return out.result();
     });
 }
@@ -231,13 +242,11 @@ MI_FAST(softmax) {
         need(y.sizes() == x.sizes());
         void* s = stream_of(a[3]);
         if (a[2] == Py_None) {
-            launch([&] { return mi_softmax_f16(ptr(x), ptr(y), x.size(0), x.size(1), s); });
+            launch(mi_softmax_f16, ptr(x), ptr(y), x.size(0), x.size(1), s);
         } else {
             const auto& w = bytes_on_gpu(a[2]);
-            launch([&] {
-                return mi_softmax_ws_f16(ptr(x), ptr(y), x.size(0), x.size(1), ptr(w),
-                                         static_cast<int64_t>(w.nbytes()), s);
-            });
+            launch(mi_softmax_ws_f16, ptr(x), ptr(y), x.size(0), x.size(1), ptr(w),
+                   static_cast<int64_t>(w.nbytes()), s);
         }
         return out.result();
     });
@@ -253,10 +262,8 @@ MI_FAST(softmax_argmax) {
         const at::Tensor &y = *probs.t, &o = *next.t;
         need(y.sizes() == x.sizes() && o.numel() == x.size(0));
         void* s = stream_of(a[4]);
-        launch([&] {
-            return mi_softmax_argmax_ws_f16(ptr(x), ptr(y), static_cast<int32_t*>(ptr(o)), x.size(0),
-                                            x.size(1), ptr(w), static_cast<int64_t>(w.nbytes()), s);
-        });
+        launch(mi_softmax_argmax_ws_f16, ptr(x), ptr(y), static_cast<int32_t*>(ptr(o)), x.size(0),
+               x.size(1), ptr(w), static_cast<int64_t>(w.nbytes()), s);
         return pair(probs.result(), next.result());
     });
 }
@@ -271,13 +278,11 @@ MI_FAST(greedy_argmax) {
         auto* out = static_cast<int32_t*>(ptr(*next.t));
         void* s = stream_of(a[3]);
         if (a[2] == Py_None) {
-            launch([&] { return mi_greedy_argmax_f16(ptr(x), x.size(0), x.size(1), out, s); });
+            launch(mi_greedy_argmax_f16, ptr(x), x.size(0), x.size(1), out, s);
         } else {
             const auto& w = bytes_on_gpu(a[2]);
-            launch([&] {
-                return mi_greedy_argmax_ws_f16(ptr(x), x.size(0), x.size(1), out, ptr(w),
-                                               static_cast<int64_t>(w.nbytes()), s);
-            });
+            launch(mi_greedy_argmax_ws_f16, ptr(x), x.size(0), x.size(1), out, ptr(w),
+                   static_cast<int64_t>(w.nbytes()), s);
         }
         return next.result();
     });
@@ -293,11 +298,8 @@ MI_FAST(top_p_sample) {
         const float p = static_cast<float>(number(a[1])), temp = static_cast<float>(number(a[2]));
         const int64_t seed = whole(a[3]);
         void* s = stream_of(a[5]);
-        launch([&] {
-            return mi_top_p_sample_batched_f16(ptr(x), x.size(0), x.size(1), p, temp,
-                                               static_cast<uint64_t>(seed),
-                                               static_cast<int32_t*>(ptr(*next.t)), s);
-        });
+        launch(mi_top_p_sample_batched_f16, ptr(x), x.size(0), x.size(1), p, temp,
+               static_cast<uint64_t>(seed), static_cast<int32_t*>(ptr(*next.t)), s);
         return next.result();
     });
 }
@@ -329,9 +331,7 @@ MI_FAST(rope_neox_qk) {
         const Floats inv(a[3]);
         need(inv.size() == r.hd / 2);
         void* s = stream_of(a[4]);
-        launch([&] {
-            return mi_rope_neox_qk_f16(ptr(r.q), r.kp(), r.pp(), inv.data(), r.T, r.Hq, r.Hkv, r.hd, s);
-        });
+        launch(mi_rope_neox_qk_f16, ptr(r.q), r.kp(), r.pp(), inv.data(), r.T, r.Hq, r.Hkv, r.hd, s);
         return PyTuple_Pack(2, a[0], a[1]);
     });
 }
@@ -346,10 +346,8 @@ MI_FAST(bias_rope_neox_qk) {
         const Floats inv(a[5]);
         need(inv.size() == r.hd / 2);
         void* s = stream_of(a[6]);
-        launch([&] {
-            return mi_bias_rope_neox_qk_f16(ptr(r.q), r.kp(), ptr(bq), bk ? ptr(*bk) : nullptr,
-                                            r.pp(), inv.data(), r.T, r.Hq, r.Hkv, r.hd, s);
-        });
+        launch(mi_bias_rope_neox_qk_f16, ptr(r.q), r.kp(), ptr(bq), bk ? ptr(*bk) : nullptr, r.pp(),
+               inv.data(), r.T, r.Hq, r.Hkv, r.hd, s);
         return PyTuple_Pack(2, a[0], a[1]);
     });
 }
@@ -366,10 +364,8 @@ MI_FAST(qk_norm_rope) {
         const float eps = static_cast<float>(number(a[6]));
         const int one = truth(a[7]);
         void* s = stream_of(a[8]);
-        launch([&] {
-            return mi_qk_norm_rope_f16(ptr(r.q), r.kp(), ptr(wq), wk ? ptr(*wk) : nullptr, r.pp(),
-                                       inv.data(), r.T, r.Hq, r.Hkv, r.hd, eps, one, s);
-        });
+        launch(mi_qk_norm_rope_f16, ptr(r.q), r.kp(), ptr(wq), wk ? ptr(*wk) : nullptr, r.pp(),
+               inv.data(), r.T, r.Hq, r.Hkv, r.hd, eps, one, s);
         return PyTuple_Pack(2, a[0], a[1]);
     });
 }
@@ -385,7 +381,7 @@ MI_FAST(rope_neox) {
         const int64_t B = x.size(0), S = x.size(1), H = x.size(2), D = x.size(3);
         need(c.numel() == B * S * (D / 2) && sn.numel() == B * S * (D / 2));
         void* s = stream_of(a[4]);
-        launch([&] { return mi_rope_neox_f16(ptr(x), ptr(c), ptr(sn), ptr(y), B, S, H, D, s); });
+        launch(mi_rope_neox_f16, ptr(x), ptr(c), ptr(sn), ptr(y), B, S, H, D, s);
         return out.result();
     });
 }
@@ -400,10 +396,8 @@ MI_FAST(rope_tables) {
         const at::Tensor &c = *oc.t, &sn = *os.t;
         need(c.numel() == N * hf && sn.numel() == N * hf);
         void* s = stream_of(a[4]);
-        launch([&] {
-            return mi_rope_tables_f16(inv.data(), static_cast<const int64_t*>(ptr(pos)), ptr(c),
-                                      ptr(sn), N, hf, s);
-        });
+        launch(mi_rope_tables_f16, inv.data(), static_cast<const int64_t*>(ptr(pos)), ptr(c),
+               ptr(sn), N, hf, s);
         return pair(oc.result(), os.result());
     });
 }
@@ -427,10 +421,8 @@ MI_FAST(embedding_gather) {
         need(o.numel() == T * H);
         const int check = truth(a[3]);
         void* s = stream_of(a[4]);
-        launch([&] {
-            return mi_embedding_gather_f16(static_cast<const int64_t*>(ptr(ids)), ptr(tb), ptr(o), T, H,
-                                           check ? V : 0, s);
-        });
+        launch(mi_embedding_gather_f16, static_cast<const int64_t*>(ptr(ids)), ptr(tb), ptr(o), T,
+               H, check ? V : 0, s);
         return out.result();
     });
 }
@@ -449,10 +441,8 @@ MI_FAST(embedding_rmsnorm) {
         const float scale = static_cast<float>(number(a[5])), eps = static_cast<float>(number(a[6]));
         const int one = truth(a[7]), check = truth(a[8]);
         void* s = stream_of(a[9]);
-        launch([&] {
-            return mi_embedding_rmsnorm_f16(static_cast<const int64_t*>(ptr(ids)), ptr(tb), ptr(h), ptr(w),
-                                            ptr(y), T, D, check ? V : 0, scale, eps, one, s);
-        });
+        launch(mi_embedding_rmsnorm_f16, static_cast<const int64_t*>(ptr(ids)), ptr(tb), ptr(h),
+               ptr(w), ptr(y), T, D, check ? V : 0, scale, eps, one, s);
         return pair(oh.result(), oy.result());
     });
 }
@@ -468,9 +458,8 @@ MI_FAST(chain_run) {
         const auto* d = reinterpret_cast<const mi_chain_desc*>(static_cast<intptr_t>(whole(a[0])));
         const int last = static_cast<int>(whole(a[1]));
         void* s = stream_of(a[2]);
-        Py_BEGIN_ALLOW_THREADS
+        const NoGil released;
         st = mi_decoder_chain_run(d, last, s);
-        Py_END_ALLOW_THREADS
     } catch (const Leave&) {
         Py_RETURN_NONE;
     } catch (const std::exception& e) {

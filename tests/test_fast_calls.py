@@ -2,10 +2,92 @@
 wrapper's result, and what they leave -- wrong types, shapes, devices, layouts,
 tensor subclasses, sequences for the inverse frequencies -- is checked, converted
 and refused by the wrapper as before."""
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import pytest
 
 from helpers import assert_bits_equal, normal_f16, to_dev, to_host
+
+PKG = Path(__file__).resolve().parent.parent / "mini-infer_amd"
+
+
+def _child(code, *args):
+    """Runs code in a process of its own (a native fault ends only that); its output."""
+    r = subprocess.run([sys.executable, "-c", code, *map(str, args)], capture_output=True, text=True,
+                       timeout=110)
+    assert r.returncode == 0, f"exit status {r.returncode}\n{r.stdout}\n{r.stderr[-2000:]}"
+    return r.stdout
+
+
+VMAP = """
+import sys
+sys.path.insert(0, sys.argv[1])
+import numpy as np
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+import mi_kernels as mk
+
+
+class Stream:
+    cuda_stream = 0
+
+
+s, n = Stream(), 0
+
+
+def refused(call, *args):
+    def body(*a):
+        t = next(x for x in a if x is not None)
+        assert type(t) is torch.Tensor and t.is_cuda and t.is_contiguous()
+        return call(*a)
+    try:
+        torch.vmap(body)(*args)
+    except RuntimeError as e:
+        assert "data pointer" in str(e), e
+        global n
+        n += 1
+    else:
+        raise AssertionError("not refused")
+
+
+def h(*shape, dtype=torch.float16):
+    return torch.empty((3, *shape), dtype=dtype, device="cuda")
+
+
+with FakeTensorMode():
+    x, w, q, k = h(4, 8), h(8), h(4, 2, 16), h(4, 1, 16)
+    hd, b, i32 = h(16), h(1024, dtype=torch.uint8), h(4, dtype=torch.int32)
+    pos, inv = h(4, dtype=torch.int64), np.ones(8, np.float32)
+    refused(lambda x, w, y: mk.rmsnorm(x, w, y=y, stream=s), x, w, x)
+    refused(lambda x, w: mk.rmsnorm(x, w, stream=s), x, w)
+    refused(lambda x, r, w: mk.fused_add_rmsnorm(x, r, w, stream=s), x, x, w)
+    refused(lambda x, y: mk.swiglu(x, y, stream=s), x, x)
+    refused(lambda x, y: mk.geglu(x, y, stream=s), x, x)
+    refused(lambda x: mk.softmax(x, stream=s), x)
+    refused(lambda x, b: mk.softmax(x, workspace=b, stream=s), x, b)
+    refused(lambda x, b, o: mk.softmax_argmax(x, b, out=o, stream=s), x, b, i32)
+    refused(lambda x, o: mk.greedy_argmax(x, out=o, stream=s), x, i32)
+    refused(lambda x, o, b: mk.greedy_argmax(x, out=o, workspace=b, stream=s), x, i32, b)
+    refused(lambda x, o: mk.top_p_sample(x, 0.9, 1.0, 7, out=o, stream=s), x, i32)
+    refused(lambda q, k, p: mk.rope_neox_qk(q, k, p, inv, stream=s), q, k, pos)
+    refused(lambda q, k, b, c, p: mk.bias_rope_neox_qk(q, k, b, c, p, inv, stream=s), q, k, h(32), hd,
+            pos)
+    refused(lambda q, k, w, p: mk.qk_norm_rope(q, k, w, w, p, inv, stream=s), q, k, hd, pos)
+    refused(lambda x, c: mk.rope_neox(x, c, c, stream=s), h(1, 4, 2, 16), h(4, 8))
+    refused(lambda p, c, d: mk.rope_tables(inv, p, c, d, stream=s), pos, h(4, 8), h(4, 8))
+    refused(lambda i, t: mk.embedding_gather(i, t, stream=s), pos, h(50, 8))
+    refused(lambda i, t, w: mk.embedding_rmsnorm(i, t, w, stream=s), pos, h(50, 8), w)
+print("refused", n)
+"""
+
+
+def test_tensors_without_memory_are_refused():
+    """torch.vmap hands in tensors of exact type and layout whose data_ptr() throws."""
+    pytest.importorskip("torch")
+    assert "refused 18" in _child(VMAP, PKG)
 
 
 def test_cpu_tensors_are_refused(monkeypatch):

@@ -11,9 +11,12 @@
 // output that is None is allocated, as the wrapper does), and otherwise None,
 // having launched nothing: an argument is not what the call needs (a tensor on
 // another device, of another type or shape, not contiguous, a subclass with its
-// own ways, one without memory of its own, as under torch.vmap), or the library
-// refused it.  The Python wrapper then makes the call itself and raises what
-// there is to raise, so its errors and conversions stay where they were.
+// own ways, one without memory of its own, as under torch.vmap).  The Python
+// wrapper then makes the call itself and raises what there is to raise, so its
+// errors and conversions stay where they were.  A library call that was made is
+// never made again: its status, if not 0, is raised here.  (A status does not say
+// that nothing ran: an error that an earlier HIP call left behind is reported by
+// the next launch, and a second call would add a residual or rotate twice.)
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -32,6 +35,12 @@ namespace {
 
 // Thrown where a call is left to the Python wrapper.
 struct Leave {};
+
+// Thrown where the library call was made and gave a status other than 0.
+struct Failed {
+    const char* what;
+    int status;
+};
 
 void need(bool ok) {
     if (!ok) throw Leave{};
@@ -120,14 +129,15 @@ struct NoGil {
 // the GIL held: ptr() throws for a tensor without memory of its own, and the
 // handlers below are Python calls.
 template <typename F, typename... A>
-void launch(F f, A... args) {
+void launch(const char* what, F f, A... args) {
     int st;
     {
         const NoGil released;
         st = f(args...);
     }
-    need(st == 0);
+    if (st != 0) throw Failed{what, st};
 }
+#define MI_CALL(f, ...) launch(#f, f, __VA_ARGS__)
 
 // An output: the caller's tensor, or where it is None a new one of x's shape or
 // of `sizes`.
@@ -157,7 +167,8 @@ PyObject* pair(PyObject* a, PyObject* b) {
     return r;
 }
 
-// Runs body(args) for exactly n arguments: its result, or None where it is left.
+// Runs body() for exactly n arguments: its result, None where it is left, or the
+// error of a library call that failed.
 template <typename F>
 PyObject* guarded(Py_ssize_t got, Py_ssize_t n, F body) {
     if (got != n) {
@@ -168,6 +179,10 @@ PyObject* guarded(Py_ssize_t got, Py_ssize_t n, F body) {
         return body();
     } catch (const Leave&) {
         Py_RETURN_NONE;
+    } catch (const Failed& e) {  // the wrapper's message
+        PyErr_Format(PyExc_RuntimeError, "%s failed: status %d (%s)", e.what, e.status,
+                     mi_status_string(e.status));
+        return nullptr;
     } catch (const std::exception&) {  // torch: a tensor without memory of its own
         PyErr_Clear();
         Py_RETURN_NONE;
@@ -187,7 +202,7 @@ MI_FAST(rmsnorm) {
         const float eps = static_cast<float>(number(a[3]));
         const int one = truth(a[4]);
         void* s = stream_of(a[5]);
-        launch(mi_rmsnorm_f16, ptr(x), ptr(w), ptr(y), x.size(0), x.size(1), eps, one, s);
+        MI_CALL(mi_rmsnorm_f16, ptr(x), ptr(w), ptr(y), x.size(0), x.size(1), eps, one, s);
         return out.result();
     });
 }
@@ -203,27 +218,27 @@ MI_FAST(fused_add_rmsnorm) {
         const float eps = static_cast<float>(number(a[4]));
         const int one = truth(a[5]);
         void* s = stream_of(a[6]);
-        launch(mi_fused_add_rmsnorm_f16, ptr(x), ptr(r), ptr(w), ptr(y), x.size(0), x.size(1), eps,
-               one, s);
+        MI_CALL(mi_fused_add_rmsnorm_f16, ptr(x), ptr(r), ptr(w), ptr(y), x.size(0), x.size(1), eps,
+                one, s);
         return out.result();
     });
 }
 
 // (a, b, out, stream)
 template <typename F>
-PyObject* binary(PyObject* const* a, Py_ssize_t n, F f) {
+PyObject* binary(PyObject* const* a, Py_ssize_t n, const char* what, F f) {
     return guarded(n, 4, [&] {
         const auto &x = half(a[0]), &y = half(a[1]);
         need(y.numel() == x.numel());
         const Out out(a[2], x);
         need(out.t->numel() == x.numel());
         void* s = stream_of(a[3]);
-        launch(f, ptr(x), ptr(y), ptr(*out.t), x.numel(), s);
+        launch(what, f, ptr(x), ptr(y), ptr(*out.t), x.numel(), s);
         return out.result();
     });
 }
-MI_FAST(swiglu) { return binary(a, n, mi_swiglu_f16); }
-MI_FAST(geglu) { return binary(a, n, mi_geglu_f16); }
+MI_FAST(swiglu) { return binary(a, n, "mi_swiglu_f16", mi_swiglu_f16); }
+MI_FAST(geglu) { return binary(a, n, "mi_geglu_f16", mi_geglu_f16); }
 
 const at::Tensor& bytes_on_gpu(PyObject* o) {  // a workspace of any type
     need(THPVariable_CheckExact(o));
@@ -242,11 +257,11 @@ MI_FAST(softmax) {
         need(y.sizes() == x.sizes());
         void* s = stream_of(a[3]);
         if (a[2] == Py_None) {
-            launch(mi_softmax_f16, ptr(x), ptr(y), x.size(0), x.size(1), s);
+            MI_CALL(mi_softmax_f16, ptr(x), ptr(y), x.size(0), x.size(1), s);
         } else {
             const auto& w = bytes_on_gpu(a[2]);
-            launch(mi_softmax_ws_f16, ptr(x), ptr(y), x.size(0), x.size(1), ptr(w),
-                   static_cast<int64_t>(w.nbytes()), s);
+            MI_CALL(mi_softmax_ws_f16, ptr(x), ptr(y), x.size(0), x.size(1), ptr(w),
+                    static_cast<int64_t>(w.nbytes()), s);
         }
         return out.result();
     });
@@ -262,8 +277,8 @@ MI_FAST(softmax_argmax) {
         const at::Tensor &y = *probs.t, &o = *next.t;
         need(y.sizes() == x.sizes() && o.numel() == x.size(0));
         void* s = stream_of(a[4]);
-        launch(mi_softmax_argmax_ws_f16, ptr(x), ptr(y), static_cast<int32_t*>(ptr(o)), x.size(0),
-               x.size(1), ptr(w), static_cast<int64_t>(w.nbytes()), s);
+        MI_CALL(mi_softmax_argmax_ws_f16, ptr(x), ptr(y), static_cast<int32_t*>(ptr(o)), x.size(0),
+                x.size(1), ptr(w), static_cast<int64_t>(w.nbytes()), s);
         return pair(probs.result(), next.result());
     });
 }
@@ -278,11 +293,11 @@ MI_FAST(greedy_argmax) {
         auto* out = static_cast<int32_t*>(ptr(*next.t));
         void* s = stream_of(a[3]);
         if (a[2] == Py_None) {
-            launch(mi_greedy_argmax_f16, ptr(x), x.size(0), x.size(1), out, s);
+            MI_CALL(mi_greedy_argmax_f16, ptr(x), x.size(0), x.size(1), out, s);
         } else {
             const auto& w = bytes_on_gpu(a[2]);
-            launch(mi_greedy_argmax_ws_f16, ptr(x), x.size(0), x.size(1), out, ptr(w),
-                   static_cast<int64_t>(w.nbytes()), s);
+            MI_CALL(mi_greedy_argmax_ws_f16, ptr(x), x.size(0), x.size(1), out, ptr(w),
+                    static_cast<int64_t>(w.nbytes()), s);
         }
         return next.result();
     });
@@ -298,8 +313,8 @@ MI_FAST(top_p_sample) {
         const float p = static_cast<float>(number(a[1])), temp = static_cast<float>(number(a[2]));
         const int64_t seed = whole(a[3]);
         void* s = stream_of(a[5]);
-        launch(mi_top_p_sample_batched_f16, ptr(x), x.size(0), x.size(1), p, temp,
-               static_cast<uint64_t>(seed), static_cast<int32_t*>(ptr(*next.t)), s);
+        MI_CALL(mi_top_p_sample_batched_f16, ptr(x), x.size(0), x.size(1), p, temp,
+                static_cast<uint64_t>(seed), static_cast<int32_t*>(ptr(*next.t)), s);
         return next.result();
     });
 }
@@ -331,7 +346,7 @@ MI_FAST(rope_neox_qk) {
         const Floats inv(a[3]);
         need(inv.size() == r.hd / 2);
         void* s = stream_of(a[4]);
-        launch(mi_rope_neox_qk_f16, ptr(r.q), r.kp(), r.pp(), inv.data(), r.T, r.Hq, r.Hkv, r.hd, s);
+        MI_CALL(mi_rope_neox_qk_f16, ptr(r.q), r.kp(), r.pp(), inv.data(), r.T, r.Hq, r.Hkv, r.hd, s);
         return PyTuple_Pack(2, a[0], a[1]);
     });
 }
@@ -346,8 +361,8 @@ MI_FAST(bias_rope_neox_qk) {
         const Floats inv(a[5]);
         need(inv.size() == r.hd / 2);
         void* s = stream_of(a[6]);
-        launch(mi_bias_rope_neox_qk_f16, ptr(r.q), r.kp(), ptr(bq), bk ? ptr(*bk) : nullptr, r.pp(),
-               inv.data(), r.T, r.Hq, r.Hkv, r.hd, s);
+        MI_CALL(mi_bias_rope_neox_qk_f16, ptr(r.q), r.kp(), ptr(bq), bk ? ptr(*bk) : nullptr, r.pp(),
+                inv.data(), r.T, r.Hq, r.Hkv, r.hd, s);
         return PyTuple_Pack(2, a[0], a[1]);
     });
 }
@@ -364,8 +379,8 @@ MI_FAST(qk_norm_rope) {
         const float eps = static_cast<float>(number(a[6]));
         const int one = truth(a[7]);
         void* s = stream_of(a[8]);
-        launch(mi_qk_norm_rope_f16, ptr(r.q), r.kp(), ptr(wq), wk ? ptr(*wk) : nullptr, r.pp(),
-               inv.data(), r.T, r.Hq, r.Hkv, r.hd, eps, one, s);
+        MI_CALL(mi_qk_norm_rope_f16, ptr(r.q), r.kp(), ptr(wq), wk ? ptr(*wk) : nullptr, r.pp(),
+                inv.data(), r.T, r.Hq, r.Hkv, r.hd, eps, one, s);
         return PyTuple_Pack(2, a[0], a[1]);
     });
 }
@@ -381,7 +396,7 @@ MI_FAST(rope_neox) {
         const int64_t B = x.size(0), S = x.size(1), H = x.size(2), D = x.size(3);
         need(c.numel() == B * S * (D / 2) && sn.numel() == B * S * (D / 2));
         void* s = stream_of(a[4]);
-        launch(mi_rope_neox_f16, ptr(x), ptr(c), ptr(sn), ptr(y), B, S, H, D, s);
+        MI_CALL(mi_rope_neox_f16, ptr(x), ptr(c), ptr(sn), ptr(y), B, S, H, D, s);
         return out.result();
     });
 }
@@ -396,8 +411,8 @@ MI_FAST(rope_tables) {
         const at::Tensor &c = *oc.t, &sn = *os.t;
         need(c.numel() == N * hf && sn.numel() == N * hf);
         void* s = stream_of(a[4]);
-        launch(mi_rope_tables_f16, inv.data(), static_cast<const int64_t*>(ptr(pos)), ptr(c),
-               ptr(sn), N, hf, s);
+        MI_CALL(mi_rope_tables_f16, inv.data(), static_cast<const int64_t*>(ptr(pos)), ptr(c),
+                ptr(sn), N, hf, s);
         return pair(oc.result(), os.result());
     });
 }
@@ -421,8 +436,8 @@ MI_FAST(embedding_gather) {
         need(o.numel() == T * H);
         const int check = truth(a[3]);
         void* s = stream_of(a[4]);
-        launch(mi_embedding_gather_f16, static_cast<const int64_t*>(ptr(ids)), ptr(tb), ptr(o), T,
-               H, check ? V : 0, s);
+        MI_CALL(mi_embedding_gather_f16, static_cast<const int64_t*>(ptr(ids)), ptr(tb), ptr(o), T,
+                H, check ? V : 0, s);
         return out.result();
     });
 }
@@ -441,8 +456,8 @@ MI_FAST(embedding_rmsnorm) {
         const float scale = static_cast<float>(number(a[5])), eps = static_cast<float>(number(a[6]));
         const int one = truth(a[7]), check = truth(a[8]);
         void* s = stream_of(a[9]);
-        launch(mi_embedding_rmsnorm_f16, static_cast<const int64_t*>(ptr(ids)), ptr(tb), ptr(h),
-               ptr(w), ptr(y), T, D, check ? V : 0, scale, eps, one, s);
+        MI_CALL(mi_embedding_rmsnorm_f16, static_cast<const int64_t*>(ptr(ids)), ptr(tb), ptr(h),
+                ptr(w), ptr(y), T, D, check ? V : 0, scale, eps, one, s);
         return pair(oh.result(), oy.result());
     });
 }

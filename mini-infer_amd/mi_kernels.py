@@ -121,7 +121,7 @@ _fast = None
 
 def _load_fast():
     """The native calls (host/python/fast_calls.cpp): each takes the wrapper's arguments
-    and returns its result, or None when it has launched nothing and the wrapper
+    and returns its result, or None when it has made no library call and the wrapper
     is to check, call and raise by itself."""
     global _fast
     load_library()

@@ -2,8 +2,11 @@
 wrapper's result, and what they leave -- wrong types, shapes, devices, layouts,
 tensor subclasses, sequences for the inverse frequencies -- is checked, converted
 and refused by the wrapper as before."""
+import importlib.util
+import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 import numpy as np
@@ -101,6 +104,95 @@ def test_cpu_tensors_are_refused(monkeypatch):
             call()
     with pytest.raises(TypeError):
         mk.softmax(np.zeros((4, 8), np.float16))
+
+
+ONCE = """
+import ctypes
+import sys
+sys.path.insert(0, sys.argv[1])
+import numpy as np
+import torch
+import mi_kernels as mk
+
+mk._need = lambda *a: None  # the wrapper too would take these tensors
+stub = ctypes.CDLL(sys.argv[1] + "/libmi_kernels.so")
+calls = ctypes.c_int.in_dll(stub, "calls")
+status = ctypes.c_int.in_dll(stub, "status")
+
+
+class Stream:
+    cuda_stream = 0
+
+
+s = Stream()
+
+
+def h(*shape, dtype=torch.float16):
+    return torch.zeros(shape, dtype=dtype)
+
+
+x, w, q, k, hd, ws = h(4, 8), h(8), h(4, 2, 16), h(4, 1, 16), h(16), h(64, dtype=torch.uint8)
+pos, inv = h(4, dtype=torch.int64), np.ones(8, np.float32)
+each = {
+    "mi_rmsnorm_f16": lambda: mk.rmsnorm(x, w, stream=s),
+    "mi_fused_add_rmsnorm_f16": lambda: mk.fused_add_rmsnorm(x, x, w, stream=s),
+    "mi_swiglu_f16": lambda: mk.swiglu(x, x, stream=s),
+    "mi_geglu_f16": lambda: mk.geglu(x, x, stream=s),
+    "mi_softmax_f16": lambda: mk.softmax(x, stream=s),
+    "mi_softmax_ws_f16": lambda: mk.softmax(x, workspace=ws, stream=s),
+    "mi_softmax_argmax_ws_f16": lambda: mk.softmax_argmax(x, ws, stream=s),
+    "mi_greedy_argmax_f16": lambda: mk.greedy_argmax(x, stream=s),
+    "mi_greedy_argmax_ws_f16": lambda: mk.greedy_argmax(x, workspace=ws, stream=s),
+    "mi_top_p_sample_batched_f16": lambda: mk.top_p_sample(x, 0.9, 1.0, 7, stream=s),
+    "mi_rope_neox_qk_f16": lambda: mk.rope_neox_qk(q, k, pos, inv, stream=s),
+    "mi_bias_rope_neox_qk_f16": lambda: mk.bias_rope_neox_qk(q, k, h(32), hd, pos, inv, stream=s),
+    "mi_qk_norm_rope_f16": lambda: mk.qk_norm_rope(q, k, hd, hd, pos, inv, stream=s),
+    "mi_rope_neox_f16": lambda: mk.rope_neox(h(1, 4, 2, 16), h(4, 8), h(4, 8), stream=s),
+    "mi_rope_tables_f16": lambda: mk.rope_tables(inv, pos, stream=s),
+    "mi_embedding_gather_f16": lambda: mk.embedding_gather(pos, x, stream=s),
+    "mi_embedding_rmsnorm_f16": lambda: mk.embedding_rmsnorm(pos, x, w, stream=s),
+}
+for name, call in each.items():
+    calls.value = status.value = 0
+    assert call() is not None and calls.value == 1, name
+    for st in (100, -1, -2):  # a HIP error, refusals
+        calls.value, status.value = 0, st
+        try:
+            call()
+        except RuntimeError as e:
+            assert str(e) == f"{name} failed: status {st} (why)", e
+        else:
+            raise AssertionError(name + ": status lost")
+        assert calls.value == 1, (name, st, calls.value)
+print("once", len(each))
+"""
+
+
+def test_a_failed_call_is_made_once(tmp_path):
+    """The binding over a library whose calls only count themselves and return a
+    status: whatever it is, there is one call, and the status is raised.  The native
+    part is built to take CPU tensors for it."""
+    torch = pytest.importorskip("torch")
+    import mi_kernels as mk
+    names = [*mk.SIGNATURES, "mi_greedy_argmax_workspace_bytes", "mi_softmax_workspace_bytes",
+             "mi_softmax_argmax_workspace_bytes", "mi_decoder_chain_run"]
+    stub = tmp_path / "stub.c"
+    stub.write_text("int calls, status;\nconst char* mi_status_string(int s) { return \"why\"; }\n" +
+                    "".join(f"int {n}() {{ ++calls; return status; }}\n" for n in names))
+    lib = tmp_path / "libmi_kernels.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", str(stub), "-o", str(lib)], check=True)
+    src = (PKG / "host/python/fast_calls.cpp").read_text()
+    assert src.count("t.is_cuda()") == 2
+    cpu = tmp_path / "fast_calls_cpu.cpp"
+    cpu.write_text(src.replace("t.is_cuda()", "t.is_cpu()"))
+    at = Path(importlib.util.find_spec("torch").submodule_search_locations[0])
+    subprocess.run(["g++", "-O0", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
+                    "-DUSE_ROCM=1", f"-I{PKG.parent / 'include'}", f"-I{sysconfig.get_paths()['include']}",
+                    "-isystem", str(at / "include"), "-isystem", "/opt/rocm/include", "-o",
+                    str(tmp_path / "_mi_fast.so"), str(cpu), str(lib), f"-L{at / 'lib'}", "-ltorch_python",
+                    "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"], check=True)
+    shutil.copy(PKG / "mi_kernels.py", tmp_path)
+    assert "once 17" in _child(ONCE, tmp_path)
 
 
 @pytest.mark.gpu

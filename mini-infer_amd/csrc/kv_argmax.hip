@@ -619,10 +619,9 @@ extern "C" int mi_greedy_argmax_f16(const void* logits, int64_t B, int64_t V, in
     // Otherwise two launches with a stream-ordered keys workspace (a fresh
     // pool allocation is not zeroed, which the two-launch form does not need).
     void* ws = nullptr;
-    hipError_t e = hipMallocAsync(&ws, static_cast<size_t>(need), s);
-    if (e != hipSuccess) return static_cast<int>(e);
+    const hipError_t e = hipMallocAsync(&ws, static_cast<size_t>(need), s);
+    if (e != hipSuccess) return mi::taken(e);
     const int st = mi::argmax(logits, B, V, out, ws, need, mi::Ws::kKeys, stream);
-    e = hipFreeAsync(ws, s);
-    if (st != MI_OK) return st;
-    return e == hipSuccess ? MI_OK : static_cast<int>(e);
+    const int released = mi::taken(hipFreeAsync(ws, s));
+    return st != MI_OK ? st : released;
 }

@@ -42,6 +42,14 @@ inline bool product_fits(std::initializer_list<int64_t> factors) {
     return true;
 }
 
+// Takes a failed runtime call's error off the thread and gives its status.  A
+// call that the library answers itself -- by returning the status, or by another
+// path -- must not leave it there: the next launch would report it.
+inline int taken(hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();
+    return static_cast<int>(e);
+}
+
 // Maps the outcome of the launches just issued to the ABI's status code.
 inline int launch_status() {
     const hipError_t e = hipGetLastError();
@@ -61,15 +69,15 @@ inline int64_t resident_workgroups(const void* kernel, int threads) {
     static std::mutex mu;
     static std::map<std::pair<const void*, int>, int64_t> cache;
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    if (taken(hipGetDevice(&dev)) != hipSuccess) return 0;
     std::lock_guard<std::mutex> lock(mu);
     const auto key = std::make_pair(kernel, dev * 4096 + threads);
     auto it = cache.find(key);
     if (it != cache.end()) return it->second;
     int per_cu = 0, cus = 0;
     int64_t cap = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) == hipSuccess &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+    if (taken(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0)) == hipSuccess &&
+        taken(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) == hipSuccess)
         cap = static_cast<int64_t>(per_cu) * cus;
     cache[key] = cap;
     return cap;
@@ -81,12 +89,12 @@ inline int device_cus() {
     static std::mutex mu;
     static std::map<int, int> cache;
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    if (taken(hipGetDevice(&dev)) != hipSuccess) return 0;
     std::lock_guard<std::mutex> lock(mu);
     auto it = cache.find(dev);
     if (it != cache.end()) return it->second;
     int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    if (taken(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess)
         cus = 0;
     cache[dev] = cus;
     return cus;
@@ -107,22 +115,15 @@ inline void* default_stream_region(int tag, int64_t bytes, hipStream_t s) {
     static std::mutex mu;
     static std::map<std::pair<int, int>, void*> regions;
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    if (taken(hipGetDevice(&dev)) != hipSuccess) return nullptr;
     std::lock_guard<std::mutex> lock(mu);
     const auto key = std::make_pair(dev, tag);
     auto it = regions.find(key);
     if (it != regions.end()) return it->second;
     void* p = nullptr;
-    if (hipMalloc(&p, static_cast<size_t>(bytes)) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (hipMemsetAsync(p, 0, static_cast<size_t>(bytes), nullptr) != hipSuccess) {
-        (void)hipGetLastError();
-        (void)hipFree(p);
+    if (taken(hipMalloc(&p, static_cast<size_t>(bytes))) != hipSuccess) return nullptr;
+    if (taken(hipMemsetAsync(p, 0, static_cast<size_t>(bytes), nullptr)) != hipSuccess) {
+        (void)taken(hipFree(p));
         return nullptr;
     }
     regions[key] = p;

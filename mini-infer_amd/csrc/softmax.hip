@@ -647,7 +647,7 @@ void* scratch_for_current_device(int* err) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) {
-        *err = static_cast<int>(e);
+        *err = taken(e);
         return nullptr;
     }
     std::lock_guard<std::mutex> lock(mu);
@@ -656,8 +656,7 @@ void* scratch_for_current_device(int* err) {
     void* ptr = nullptr;
     e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
     if (e != hipSuccess || ptr == nullptr) {
-        *err = static_cast<int>(e != hipSuccess ? e : hipErrorInvalidSymbol);
-        (void)hipGetLastError();
+        *err = taken(e != hipSuccess ? e : hipErrorInvalidSymbol);
         return nullptr;
     }
     ptrs[dev] = ptr;
@@ -780,12 +779,11 @@ extern "C" int mi_softmax_f16(const void* x, void* y, int64_t N, int64_t D, void
     // own; a fresh pool allocation is not zeroed, which the two-pass form
     // does not need).
     void* ws = nullptr;
-    hipError_t e = hipMallocAsync(&ws, static_cast<size_t>(need), s);
-    if (e != hipSuccess) return static_cast<int>(e);
+    const hipError_t e = hipMallocAsync(&ws, static_cast<size_t>(need), s);
+    if (e != hipSuccess) return mi::taken(e);
     const int st = mi::softmax_checked(x, y, N, D, ws, need, mi::Ws::kPairs, stream);
-    e = hipFreeAsync(ws, s);
-    if (st != MI_OK) return st;
-    return e == hipSuccess ? MI_OK : static_cast<int>(e);
+    const int released = mi::taken(hipFreeAsync(ws, s));
+    return st != MI_OK ? st : released;
 }
 
 extern "C" int mi_softmax_test_poll_limit(int limit) {

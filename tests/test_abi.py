@@ -6,6 +6,8 @@ touching the HIP runtime.
 """
 import ctypes
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -184,3 +186,59 @@ def test_argmax_workspace_sizes(lib):
     assert lib.mi_greedy_argmax_workspace_bytes(512, 152064) == 0           # one workgroup per row
     assert lib.mi_greedy_argmax_workspace_bytes(64, 4096) == 0
     assert 0 < lib.mi_greedy_argmax_workspace_bytes(511, 10**6) <= 512 * 2176 + 256 * 1024
+
+
+PENDING = """
+import ctypes
+import sys
+sys.path.insert(0, sys.argv[1])
+stub = ctypes.CDLL(sys.argv[2], mode=ctypes.RTLD_GLOBAL)  # before the runtime's own symbols
+import mi_kernels
+lib = mi_kernels.load_library()
+pending = ctypes.c_int.in_dll(stub, "pending")
+P = ctypes.c_void_p
+x, y, out, stream = P(0x1000000), P(0x2000000), P(0x3000000), P(0x40)
+# rows split across workgroups, on a stream of their own: a workspace per call
+calls = {"softmax": lambda: lib.mi_softmax_f16(x, y, 3, 30000, stream),
+         "argmax": lambda: lib.mi_greedy_argmax_f16(x, 3, 30000, out, stream),
+         "noalloc": lambda: lib.mi_softmax_noalloc_f16(x, y, 3, 30000, stream)}
+for failing, want in ((1, dict(softmax=0)), (2, dict(softmax=0, noalloc=101)),
+                      (3, dict(softmax=2, argmax=2)), (4, dict(softmax=3, argmax=3))):
+    ctypes.c_int.in_dll(stub, "failing").value = failing
+    for what, status in want.items():
+        got = calls[what]()
+        print(failing, what, got, pending.value, flush=True)
+        assert got == status, "not the call's own status"
+        assert pending.value == 0, "left for the next launch to report"
+"""
+
+
+def test_no_failed_hip_call_is_left_for_the_next_launch(tmp_path):
+    """A launch reports the thread's pending error, so a failed runtime call that the
+    library has answered (with its status, or by another path) must not stay there.
+    Over stand-ins for the runtime calls in question: 1 the occupancy query fails, 2
+    the device query (a launch made without their answer succeeds), 3 the
+    workspace's allocation, 4 its release."""
+    stub = tmp_path / "stub.c"
+    stub.write_text("""
+#include <stddef.h>
+int pending, failing;
+static int result(int fails, int e) { if (fails) pending = e; return fails ? e : 0; }
+int hipGetLastError(void) { int e = pending; pending = 0; return e; }
+int hipMallocAsync(void** p, size_t n, void* s) { *p = (void*)0x50000000; return result(failing == 3, 2); }
+int hipFreeAsync(void* p, void* s) { return result(failing == 4, 3); }
+int hipGetDevice(int* d) { *d = 0; return result(failing == 2, 101); }
+int hipDeviceGetAttribute(int* v, int a, int d) { *v = 256; return 0; }
+int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void* f, int t, size_t l) {
+    *n = 0;
+    return result(failing == 1, 1);
+}
+int __hipPushCallConfiguration() { return 0; }
+int __hipPopCallConfiguration() { return 0; }
+int hipLaunchKernel() { return 0; }
+""")
+    so = tmp_path / "libstub.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-w", str(stub), "-o", str(so)], check=True)
+    r = subprocess.run([sys.executable, "-c", PENDING, str(ROOT / "mini-infer_amd"), str(so)],
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr

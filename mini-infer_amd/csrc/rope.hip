@@ -1240,7 +1240,8 @@ int rope_kv_plan(void* q, void* k, const void* v, const void* q_bias, const void
     // one 256-lane workgroup per token: its Q/K slices and V's vectors one
     // per lane (both <= 256; wide: up to three per lane), 16-byte vectors, few
     // segments
-    if (head_dim % 16 != 0 || head_dim / 2 > kMaxHalf || Hq + Hkv > 1024) return MI_ERR_UNSUPPORTED;
+    if (head_dim % 16 != 0 || head_dim / 2 > kMaxHalf || (head_dim > 0 && Hq + Hkv > 1024))
+        return MI_ERR_UNSUPPORTED;
     slots = std::max((Hq + Hkv) * (head_dim / 16), Hkv * head_dim / 8);
     if (slots > (wide ? 768 : 256) || num_segments > kMaxKvSegs || T > kMaxGridX ||
         block_size > INT32_MAX)
@@ -1289,7 +1290,7 @@ int rope_kv_plan(void* q, void* k, const void* v, const void* q_bias, const void
         sg.sl[i] = g.seq_len;
         sg.sp[i] = g.start_pos;
     }
-    if (!inv_freq_host) return MI_ERR_INVALID_ARGUMENT;
+    if (!inv_freq_host || head_dim == 0) return MI_ERR_INVALID_ARGUMENT;
     a.q = static_cast<half_t*>(q);
     a.k = static_cast<half_t*>(k);
     a.v = static_cast<const half_t*>(v);

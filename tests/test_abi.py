@@ -188,6 +188,18 @@ def test_argmax_workspace_sizes(lib):
     assert 0 < lib.mi_greedy_argmax_workspace_bytes(511, 10**6) <= 512 * 2176 + 256 * 1024
 
 
+@pytest.mark.parametrize("heads", [1, 100, 2000])
+def test_attention_preprocessing_refuses_a_head_of_nothing(lib, heads):
+    """head_dim 0 (a multiple of 16) with tokens to rotate."""
+    p = [P(0x10000 * i) for i in range(1, 8)]
+    inv = (ctypes.c_float * 4)()
+    for biases in ((None,) * 3, (P(0x90000), P(0xa0000), P(0xb0000))):
+        assert lib.mi_rope_kv_scatter_f16(*p[:3], *biases, p[3], inv, 4, heads, 1, 0, *p[4:6], 0, 8,
+                                          16, None, 0, None) == -1
+    assert lib.mi_qk_norm_rope_kv_scatter_f16(*p[:5], p[5], inv, 4, heads, 1, 0, 1e-6, 0, p[6],
+                                              P(0x90000), 0, 8, 16, None, 0, None) == -1
+
+
 PENDING = """
 import ctypes
 import sys

@@ -695,14 +695,20 @@ extern "C" int mi_softmax_ws_f16(const void* x, void* y, int64_t N, int64_t D, v
 
 // Fused softmax + greedy argmax: [fused row records | softmax workspace |
 // argmax workspace]; the one-launch fused kernel when the shape takes the
-// one-launch softmax, else the two entry points in turn on their parts.
+// one-launch softmax, else the two entry points in turn on their parts, each
+// 16-byte aligned.
 namespace {
 constexpr int64_t kFusedRegion = mi::kSplitMaxRows * mi::kRowRecordBytesAM;
+static_assert(kFusedRegion % 16 == 0, "the parts are 16-byte aligned");
+// (the softmax's pairs are 8 bytes each, an odd number of them for some shapes)
+int64_t fused_argmax_offset(int64_t N, int64_t V) {
+    return kFusedRegion + mi::ceil_div(mi::workspace_bytes(N, V), 16) * 16;
 }
+}  // namespace
 
 extern "C" int64_t mi_softmax_argmax_workspace_bytes(int64_t N, int64_t V) {
     if (N <= 0 || V <= 0) return 0;
-    return kFusedRegion + mi::workspace_bytes(N, V) + mi_greedy_argmax_workspace_bytes(N, V);
+    return fused_argmax_offset(N, V) + mi_greedy_argmax_workspace_bytes(N, V);
 }
 
 namespace {
@@ -753,7 +759,7 @@ extern "C" int mi_softmax_argmax_ws_f16(const void* logits, void* probs, int32_t
                                        static_cast<mi::half_t*>(probs), ws, out, N, V, s);
     // separately: argmax first (in place, softmax would overwrite the logits)
     const int64_t sw = mi::workspace_bytes(N, V);
-    unsigned char* aw = ws + kFusedRegion + sw;
+    unsigned char* aw = ws + fused_argmax_offset(N, V);
     const int st = mi_greedy_argmax_ws_f16(logits, N, V, out, aw,
                                            mi_greedy_argmax_workspace_bytes(N, V), stream);
     if (st != MI_OK) return st;

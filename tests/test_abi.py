@@ -200,41 +200,10 @@ def test_attention_preprocessing_refuses_a_head_of_nothing(lib, heads):
                                               P(0x90000), 0, 8, 16, None, 0, None) == -1
 
 
-PENDING = """
-import ctypes
-import sys
-sys.path.insert(0, sys.argv[1])
-stub = ctypes.CDLL(sys.argv[2], mode=ctypes.RTLD_GLOBAL)  # before the runtime's own symbols
-import mi_kernels
-lib = mi_kernels.load_library()
-pending = ctypes.c_int.in_dll(stub, "pending")
-P = ctypes.c_void_p
-x, y, out, stream = P(0x1000000), P(0x2000000), P(0x3000000), P(0x40)
-# rows split across workgroups, on a stream of their own: a workspace per call
-calls = {"softmax": lambda: lib.mi_softmax_f16(x, y, 3, 30000, stream),
-         "argmax": lambda: lib.mi_greedy_argmax_f16(x, 3, 30000, out, stream),
-         "noalloc": lambda: lib.mi_softmax_noalloc_f16(x, y, 3, 30000, stream)}
-for failing, want in ((1, dict(softmax=0)), (2, dict(softmax=0, noalloc=101)),
-                      (3, dict(softmax=2, argmax=2)), (4, dict(softmax=3, argmax=3))):
-    ctypes.c_int.in_dll(stub, "failing").value = failing
-    for what, status in want.items():
-        got = calls[what]()
-        print(failing, what, got, pending.value, flush=True)
-        assert got == status, "not the call's own status"
-        assert pending.value == 0, "left for the next launch to report"
-"""
-
-
-def test_no_failed_hip_call_is_left_for_the_next_launch(tmp_path):
-    """A launch reports the thread's pending error, so a failed runtime call that the
-    library has answered (with its status, or by another path) must not stay there.
-    Over stand-ins for the runtime calls in question: 1 the occupancy query fails, 2
-    the device query (a launch made without their answer succeeds), 3 the
-    workspace's allocation, 4 its release."""
-    stub = tmp_path / "stub.c"
-    stub.write_text("""
+# Stand-ins for the runtime's calls: nothing is launched, and one of them can fail.
+RUNTIME = """
 #include <stddef.h>
-int pending, failing;
+int pending, failing, launches;
 static int result(int fails, int e) { if (fails) pending = e; return fails ? e : 0; }
 int hipGetLastError(void) { int e = pending; pending = 0; return e; }
 int hipMallocAsync(void** p, size_t n, void* s) { *p = (void*)0x50000000; return result(failing == 3, 2); }
@@ -247,10 +216,72 @@ int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void* f, int t, s
 }
 int __hipPushCallConfiguration() { return 0; }
 int __hipPopCallConfiguration() { return 0; }
-int hipLaunchKernel() { return 0; }
-""")
+int hipLaunchKernel() { ++launches; return 0; }
+"""
+CHILD = """
+import ctypes
+import sys
+sys.path.insert(0, sys.argv[1])
+stub = ctypes.CDLL(sys.argv[2], mode=ctypes.RTLD_GLOBAL)  # before the runtime's own symbols
+import mi_kernels
+lib = mi_kernels.load_library()
+pending, failing, launches = (ctypes.c_int.in_dll(stub, n) for n in ("pending", "failing", "launches"))
+P = ctypes.c_void_p
+x, y, out, stream = P(0x100000000), P(0x200000000), P(0x300000000), P(0x40)
+"""
+
+
+def _without_the_runtime(tmp_path, code):
+    """Runs code after CHILD in a process of its own, where no call reaches a GPU."""
+    stub = tmp_path / "stub.c"
+    stub.write_text(RUNTIME)
     so = tmp_path / "libstub.so"
     subprocess.run(["gcc", "-shared", "-fPIC", "-w", str(stub), "-o", str(so)], check=True)
-    r = subprocess.run([sys.executable, "-c", PENDING, str(ROOT / "mini-infer_amd"), str(so)],
+    r = subprocess.run([sys.executable, "-c", CHILD + code, str(ROOT / "mini-infer_amd"), str(so)],
                        capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+PENDING = """
+# rows split across workgroups, on a stream of their own: a workspace per call
+calls = {"softmax": lambda: lib.mi_softmax_f16(x, y, 3, 30000, stream),
+         "argmax": lambda: lib.mi_greedy_argmax_f16(x, 3, 30000, out, stream),
+         "noalloc": lambda: lib.mi_softmax_noalloc_f16(x, y, 3, 30000, stream)}
+for fails, want in ((1, dict(softmax=0)), (2, dict(softmax=0, noalloc=101)),
+                    (3, dict(softmax=2, argmax=2)), (4, dict(softmax=3, argmax=3))):
+    failing.value = fails
+    for what, status in want.items():
+        got = calls[what]()
+        print(fails, what, got, pending.value, flush=True)
+        assert got == status, "not the call's own status"
+        assert pending.value == 0, "left for the next launch to report"
+"""
+
+
+def test_no_failed_hip_call_is_left_for_the_next_launch(tmp_path):
+    """A launch reports the thread's pending error, so a failed runtime call that the
+    library has answered (with its status, or by another path) must not stay there.
+    Where 1 the occupancy query fails, 2 the device query (a launch made without
+    their answer succeeds), 3 the workspace's allocation, 4 its release."""
+    _without_the_runtime(tmp_path, PENDING)
+
+
+FUSED_APART = """
+import itertools
+ws = P(0x400000000)
+for N, V, in_place in itertools.product((1, 3, 5, 6, 7, 41, 255), (8192, 8193, 30000, 50257, 151643, 152064,
+                                                                   600000), (True, False)):
+    # in place, or at another offset from a 16-byte boundary: no one-launch form
+    probs = x if in_place else P(0x200000006)
+    need = lib.mi_softmax_argmax_workspace_bytes(N, V)
+    launches.value = 0
+    got = lib.mi_softmax_argmax_ws_f16(x, probs, out, N, V, ws, need, None)
+    assert got == 0 and launches.value > 1, (N, V, in_place, got)
+    assert lib.mi_softmax_argmax_ws_f16(x, probs, out, N, V, ws, need - 1, None) == -1
+"""
+
+
+def test_softmax_and_argmax_apart_take_any_rows(tmp_path):
+    """softmax + argmax as two entry points: the argmax's part of the workspace is
+    16-byte aligned also after an odd number of softmax chunks (N * splits)."""
+    _without_the_runtime(tmp_path, FUSED_APART)

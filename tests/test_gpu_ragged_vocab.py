@@ -96,3 +96,26 @@ def test_ragged_vocab(mk, orc, dev, N, V, off):
     mk.softmax(xd, y=xd, workspace=ws)  # in place
     _close(to_host(xd), x)
     assert _guards_intact(xb, off, N, V)
+
+
+# an odd number of softmax chunks (N * splits): the argmax's part of the workspace
+# comes after them
+@pytest.mark.parametrize("N,V", [(1, 8193), (5, 50257), (1, 151643), (7, 262138)])
+@pytest.mark.parametrize("in_place", [True, False])
+def test_softmax_and_argmax_apart(mk, orc, dev, N, V, in_place):
+    """The fused entry point where its one-launch form does not apply: probs on the
+    logits, or at another offset from a 16-byte boundary."""
+    import torch
+    print(f"[case] softmax + argmax apart [{N},{V}] in place={in_place}", flush=True)
+    x = np.rint(normal_f16(np.random.default_rng(N + V), (N, V), 0, 4))
+    xb, xd = _buffer(dev, 0, N, V)
+    yb, y = (xb, xd) if in_place else _buffer(dev, 3, N, V)
+    ws = torch.zeros(mk.softmax_argmax_workspace_bytes(N, V), dtype=torch.uint8, device=dev)
+    for _ in range(2):
+        xd.copy_(to_dev(x, dev))
+        out = torch.full((N,), -7, dtype=torch.int32, device=dev)
+        mk.softmax_argmax(xd, ws, probs=y, out=out)
+        torch.cuda.synchronize()
+        _close(to_host(y), x)
+        np.testing.assert_array_equal(to_host(out), orc.greedy_argmax(x))
+        assert _guards_intact(yb, 0 if in_place else 3, N, V)

@@ -249,9 +249,8 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(const half_t* __res
     uint64_t best;
     if constexpr (RAGGED) {
         const RowWindow win(x + row * V, V);
-        const int64_t len = static_cast<int64_t>(win.nv) * 8;
-        best = chunk_best_window<U>(x + row * V - win.shift, b, split + 1 == splits ? len : b + chunk,
-                                    win, slots);
+        best = chunk_best_window<U>(x + row * V - win.shift, b,
+                                    split + 1 == splits ? win.len() : b + chunk, win, slots);
     } else {
         best = chunk_best<VEC, U>(x + row * V, b, e, slots);
     }

@@ -225,7 +225,9 @@ __device__ __forceinline__ float block_max(float v, float* slots) {
 // page; they are masked to -inf after the load and never stored.  Two tensors
 // at the same offset from a 16-byte boundary (same_window) have the same shift
 // in every row, so a vector is stored where it was loaded; rows 8 apart have
-// the same shift too (8 D elements are 16 D bytes).
+// the same shift too (8 D elements are 16 D bytes).  Vectors are counted in 32
+// bits (the launchers keep D at or below kMaxWindowRow, mi_host.h), elements of
+// rows that may be longer than 2^31 in 64 (len).
 struct RowWindow {
     int shift;  // elements of the window before the row
     int nv;     // vectors of the window
@@ -237,6 +239,7 @@ struct RowWindow {
     __device__ __forceinline__ bool partial(int v) const {
         return (v == 0 && shift > 0) || (v == nv - 1 && last < 8);
     }
+    __device__ __forceinline__ int64_t len() const { return static_cast<int64_t>(nv) * 8; }
     // the elements of vector v that are not the row's become -inf
     __device__ __forceinline__ void mask(int v, h8& a) const {
         if (v == 0) {

@@ -23,6 +23,9 @@ inline bool same_window(const void* x, const void* y) {
     return (a & 1) == 0 && ((a ^ b) & 15) == 0;
 }
 
+// The longest row walked through its window: its vectors fit 32 bits.
+constexpr int64_t kMaxWindowRow = int64_t{1} << 33;
+
 // True when [a, a+abytes) and [b, b+bbytes) share at least one byte.
 inline bool overlaps(const void* a, int64_t abytes, const void* b, int64_t bbytes) {
     const uintptr_t a0 = reinterpret_cast<uintptr_t>(a), b0 = reinterpret_cast<uintptr_t>(b);

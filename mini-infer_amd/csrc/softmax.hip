@@ -290,7 +290,7 @@ __global__ __launch_bounds__(256) void softmax_partial_kernel(const half_t* x, f
     float m = -INFINITY, s = 0.0f;
     if constexpr (RAGGED) {
         const RowWindow win(x + row * D, D);
-        tile_stats<U, true>(x + row * D - win.shift, b, split + 1 == splits ? win.nv * 8 : b + chunk,
+        tile_stats<U, true>(x + row * D - win.shift, b, split + 1 == splits ? win.len() : b + chunk,
                             m, s, &win);
     } else if constexpr (VEC == 8)
         tile_stats<U>(x + row * D, b, e, m, s);
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256) void softmax_finish_kernel(const half_t* x, ha
     if constexpr (RAGGED) {
         const RowWindow win(x + row * D, D);
         const int64_t off = row * D - win.shift;
-        write_range<VEC, true>(x + off, y + off, b, split + 1 == splits ? win.nv * 8 : b + chunk, M,
+        write_range<VEC, true>(x + off, y + off, b, split + 1 == splits ? win.len() : b + chunk, M,
                                1.0f / S, &win);
     } else {
         write_range<VEC>(x + row * D, y + row * D, b, e, M, 1.0f / S);
@@ -598,7 +598,7 @@ int softmax_checked(const void* x, void* y, int64_t N, int64_t D, void* ws, int6
         else
             softmax_partial_kernel<8, 1><<<g, dim3(256), 0, s>>>(xh, part, D, chunk);
         softmax_finish_kernel<8><<<g, dim3(256), 0, s>>>(xh, yh, part, D, chunk);
-    } else if (same_window(x, y)) {
+    } else if (same_window(x, y) && D <= kMaxWindowRow) {
         if (split_tile(N, D) == 4096)
             softmax_partial_kernel<8, 2, true><<<g, dim3(256), 0, s>>>(xh, part, D, chunk);
         else

@@ -102,6 +102,32 @@ def test_large_softmax(mk, orc, dev):
     del x, y
 
 
+@pytest.mark.parametrize("D,off", [(BIG - 15, 0), (BIG - 7, 0), (BIG, 5), (BIG + 1, 0)])
+def test_large_ragged_softmax_row(mk, dev, D, off):
+    """One row of no whole number of 16-byte vectors, or off a 16-byte boundary,
+    around 2^31 elements: zeros but for a few elements at both ends, so every
+    probability has a closed form.  Sums of up to 8192 terms per lane in fp32, each
+    rounding relative 2^-24, then one fp16 rounding: |y - ref| <= 2^-10 ref."""
+    import torch
+    _case(f"softmax of one row of {D} elements, offset {off}")
+    side = torch.cuda.Stream()  # no records there: the two-launch form
+    x = torch.zeros(off + D, dtype=torch.float16, device=dev)[off:].view(1, D)
+    y = torch.full((off + D + 8,), 7.0, dtype=torch.float16, device=dev)
+    spots = {0: 20.0, 5: 21.0, D // 2: 19.0, D - 9: 20.5, D - 2: 21.0, D - 1: 20.0}
+    for i, v in spots.items():
+        x[0, i] = v
+    torch.cuda.synchronize()
+    mk.softmax(x, y=y[off:off + D].view(1, D), stream=side)
+    side.synchronize()
+    S = sum(np.exp(v) for v in spots.values()) + (D - len(spots))
+    for i, v in spots.items():
+        assert abs(y[off + i].item() - np.exp(v) / S) <= 2.0 ** -10 * np.exp(v) / S, i
+    assert (y[:off] == 7).all() and (y[off + D:] == 7).all()
+    # every other element: e^-21 and less of the largest, 0 in fp16
+    assert int(torch.count_nonzero(y[off:off + D])) == len(spots)
+    del x, y
+
+
 def test_large_argmax(mk, orc, dev):
     import torch
     B, V = 16384, 152064

@@ -17,6 +17,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import warnings
 from pathlib import Path
 
 _HERE = Path(__file__).resolve().parent
@@ -119,6 +120,18 @@ def _torch():
 _fast = None
 
 
+class _WrappersOnly:
+    """Where the native calls are not built, or for another torch: every call is left
+    to its wrapper, which makes it through ctypes."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+    @staticmethod
+    def current_stream():
+        return _torch().cuda.current_stream().cuda_stream
+
+
 def _load_fast():
     """The native calls (host/python/fast_calls.cpp): each takes the wrapper's arguments
     and returns its result, or None when it has made no library call and the wrapper
@@ -127,12 +140,15 @@ def _load_fast():
     load_library()
     _torch()  # the module is built on torch's libraries
     p = _HERE / "_mi_fast.so"
-    if not p.exists():
-        raise RuntimeError(f"{p} is not built; run __graft_entry__.build() (or `make -C mini-infer_amd`)")
-    loader = importlib.machinery.ExtensionFileLoader("_mi_fast", str(p))
-    spec = importlib.util.spec_from_file_location("_mi_fast", str(p), loader=loader)
-    mod = importlib.util.module_from_spec(spec)
-    loader.exec_module(mod)
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_mi_fast", str(p))
+        spec = importlib.util.spec_from_file_location("_mi_fast", str(p), loader=loader)
+        mod = importlib.util.module_from_spec(spec)
+        loader.exec_module(mod)
+    except ImportError as e:
+        warnings.warn(f"mi_kernels: calls go through ctypes, 5 us slower each ({e}); "
+                      "`make -C mini-infer_amd` builds the native ones", RuntimeWarning, stacklevel=3)
+        mod = _WrappersOnly()
     _fast = mod
     return mod
 

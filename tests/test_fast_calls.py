@@ -152,6 +152,8 @@ each = {
     "mi_embedding_gather_f16": lambda: mk.embedding_gather(pos, x, stream=s),
     "mi_embedding_rmsnorm_f16": lambda: mk.embedding_rmsnorm(pos, x, w, stream=s),
 }
+if sys.argv[2] != "built":
+    del each["mi_softmax_ws_f16"]  # its wrapper has a check of the workspace's device
 for name, call in each.items():
     calls.value = status.value = 0
     assert call() is not None and calls.value == 1, name
@@ -168,11 +170,13 @@ print("once", len(each))
 """
 
 
-def test_a_failed_call_is_made_once(tmp_path):
+@pytest.mark.parametrize("native", ["built", "missing", "unloadable"])
+def test_a_failed_call_is_made_once(tmp_path, native):
     """The binding over a library whose calls only count themselves and return a
     status: whatever it is, there is one call, and the status is raised.  The native
-    part is built to take CPU tensors for it."""
-    torch = pytest.importorskip("torch")
+    part is built to take CPU tensors for it; without one that loads, the wrappers
+    make the calls."""
+    pytest.importorskip("torch")
     import mi_kernels as mk
     names = [*mk.SIGNATURES, "mi_greedy_argmax_workspace_bytes", "mi_softmax_workspace_bytes",
              "mi_softmax_argmax_workspace_bytes", "mi_decoder_chain_run"]
@@ -181,6 +185,12 @@ def test_a_failed_call_is_made_once(tmp_path):
                     "".join(f"int {n}() {{ ++calls; return status; }}\n" for n in names))
     lib = tmp_path / "libmi_kernels.so"
     subprocess.run(["gcc", "-shared", "-fPIC", str(stub), "-o", str(lib)], check=True)
+    shutil.copy(PKG / "mi_kernels.py", tmp_path)
+    if native == "unloadable":
+        (tmp_path / "_mi_fast.so").write_bytes(b"")
+    if native != "built":
+        assert "once 16" in _child(ONCE, tmp_path, native)
+        return
     src = (PKG / "host/python/fast_calls.cpp").read_text()
     assert src.count("t.is_cuda()") == 2
     cpu = tmp_path / "fast_calls_cpu.cpp"
@@ -191,8 +201,14 @@ def test_a_failed_call_is_made_once(tmp_path):
                     "-isystem", str(at / "include"), "-isystem", "/opt/rocm/include", "-o",
                     str(tmp_path / "_mi_fast.so"), str(cpu), str(lib), f"-L{at / 'lib'}", "-ltorch_python",
                     "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"], check=True)
-    shutil.copy(PKG / "mi_kernels.py", tmp_path)
-    assert "once 17" in _child(ONCE, tmp_path)
+    assert "once 17" in _child(ONCE, tmp_path, native)
+
+
+def test_all_is_built_without_torch():
+    for without in ("TORCH=", "PYINC="):
+        out = subprocess.run(["make", "-n", "-B", "-C", str(PKG), "all", without], check=True,
+                             capture_output=True, text=True).stdout
+        assert "libmini_infer.so" in out and "_mi_fast.so" not in out
 
 
 @pytest.mark.gpu

@@ -79,7 +79,9 @@ def _check_kv(orc, w, k_src, what):
 
 def _check_chain(chain_mod, orc, w, what):
     """Runs the chain three times (to the embedding, to the post-attention
-    norm, to the end) and checks every intermediate against the oracle."""
+    norm, to the end) and checks every intermediate against the oracle; what
+    the second run leaves once more after the third, which may take the stages
+    in one launch."""
     S = chain_mod.Stage
     h, s = w.host, w.shapes
     eps, add1 = s["rms_eps"], bool(s["norm_add_one"])
@@ -130,7 +132,15 @@ def _check_chain(chain_mod, orc, w, what):
     w.reload("q", "k")
     if s["double_norm"]:
         w.reload("attn_out", "mlp_out")
+    for n in ("normed", "post_normed", "k_cache", "v_cache"):
+        w.t[n].zero_()
     w.run(S.SAMPLE)
+    assert_bits_equal(to_host(w.t["q"]), q_out, what=f"{what}: q of the whole step")
+    assert_bits_equal(to_host(w.t["k"]), k_out, what=f"{what}: k of the whole step")
+    _check_kv(orc, w, k_out, f"{what}, whole step")
+    assert_close(to_host(w.t["normed"]), orc.rmsnorm(hid0, h["input_norm"], eps, add1, nthreads=8),
+                 what=f"{what}: input norm of the whole step")
+    assert_close(to_host(w.t["post_normed"]), pn, what=f"{what}: post-attention norm of the whole step")
     act = orc.geglu(h["gate"], h["up"], nthreads=8) if s["act"] else \
         orc.swiglu(h["gate"], h["up"], nthreads=8)
     assert_close(to_host(w.t["act_out"]), act, what=f"{what}: activation")

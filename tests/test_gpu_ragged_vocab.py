@@ -119,3 +119,62 @@ def test_softmax_and_argmax_apart(mk, orc, dev, N, V, in_place):
         _close(to_host(y), x)
         np.testing.assert_array_equal(to_host(out), orc.greedy_argmax(x))
         assert _guards_intact(yb, 0 if in_place else 3, N, V)
+
+
+# rows in registers, in one launch in one round and in rounds, as many short rows
+@pytest.mark.parametrize("N,V", [(64, 1203), (12, 8193), (9, 16391), (48, 50257), (600, 40001)])
+@pytest.mark.parametrize("off", [0, 5])
+def test_ragged_special_values(mk, orc, dev, N, V, off):
+    """NaN and infinities at the ends of a row share 16-byte granules with its
+    neighbours' elements; inside it they reach the element-by-element tie search."""
+    import torch
+    print(f"[case] ragged special values [{N},{V}] offset {off}", flush=True)
+    x = normal_f16(np.random.default_rng(N + V + off), (N, V), 0, 4)
+    bits = x.view(np.uint16)
+    x[1, 0], x[1, -1] = np.inf, np.nan
+    x[3, V // 2] = np.nan                       # never chosen
+    x[4, [7, V // 3, V - 1]] = np.inf           # ties, in the reference's order
+    bits[6, :] = 0x7e00                         # only NaN: -1
+    bits[7, :] = 0x7e00
+    x[7, V - 2] = -65504.0                      # the one finite value
+    bits[8, ::2] = 0x7d01                       # signalling NaNs
+    want = orc.greedy_argmax(x)
+    assert want[1] == 0 and want[6] == -1 and want[7] == V - 2
+    plain = [r for r in range(N) if r not in (1, 3, 4, 6, 7, 8)]
+    xb, xd = _buffer(dev, off, N, V)
+    xd.copy_(to_dev(x, dev))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    ws = torch.zeros(max(16, mk.softmax_workspace_bytes(N, V)), dtype=torch.uint8, device=dev)
+    aw = torch.zeros(max(16, mk.greedy_argmax_workspace_bytes(N, V)), dtype=torch.uint8, device=dev)
+    fw = torch.zeros(mk.softmax_argmax_workspace_bytes(N, V), dtype=torch.uint8, device=dev)
+
+    def check(what, fn):
+        yb, y = _buffer(dev, off, N, V)
+        out = torch.full((N,), -7, dtype=torch.int32, device=dev)
+        fn(y, out)
+        torch.cuda.synchronize()
+        h = to_host(y)
+        _close(h[plain], x[plain])
+        assert np.isnan(h[[1, 3, 4]]).all(), what  # the sum is NaN
+        assert _guards_intact(yb, off, N, V), what
+        np.testing.assert_array_equal(to_host(out), want, err_msg=what)
+
+    def apart(y, o):
+        mk.softmax(xd, y=y, workspace=ws)
+        mk.greedy_argmax(xd, out=o, workspace=aw)
+
+    def on_side(y, o):
+        mk.softmax(xd, y=y, stream=side)
+        mk.greedy_argmax(xd, out=o, stream=side)
+
+    check("fused", lambda y, o: mk.softmax_argmax(xd, fw, probs=y, out=o))
+    check("apart", apart)
+    check("two launches", on_side)
+    prev = mk.softmax_test_poll_limit(0), mk.greedy_argmax_test_poll_limit(0)
+    try:
+        check("fused, no polls", lambda y, o: mk.softmax_argmax(xd, fw, probs=y, out=o))
+        check("apart, no polls", apart)
+    finally:
+        mk.softmax_test_poll_limit(prev[0])
+        mk.greedy_argmax_test_poll_limit(prev[1])

@@ -125,7 +125,10 @@ enum {
 
 /* (A run to MI_CHAIN_FINAL_NORM or beyond, whose buffers do not overlap, may
  * issue the stages in another order or several in one launch: every output
- * is as after the stages in their order.)
+ * is as after the stages in their order, bit for bit but for `normed` where
+ * rows hold several vectors per lane of fewer than 256 lanes, and `probs` where
+ * the sampling shares the launch.  Those may differ in the order of an fp32 sum:
+ * by one fp16 ulp at most.)
  * Validates `d` against every stage up to last_stage (MI_ERR_* of
  * mi_kernels.h when a pointer or size is missing or out of range; nothing is
  * launched then), then enqueues the stages on `stream` (hipStream_t; NULL =

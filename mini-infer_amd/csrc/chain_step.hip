@@ -33,7 +33,10 @@ struct RowArgs {
     int64_t D, vocab;
     float scale, eps, w_bias;
     int lanes;  // of the 256: rms_row_kernel's for rows of D, so that the norms of the
-                // blocks' outputs and of the residuals are its, bit for bit
+                // blocks' outputs and of the residuals have its bits, and
+                // rms_small_kernel's (D <= 512: one vector per lane in both).  The
+                // gather + norm kernel has 256: where these are fewer and hold several
+                // vectors each, the input norm may be an fp16 ulp from its
 };
 
 // Opaque copies of x.
@@ -232,9 +235,13 @@ bool rows_plan(const ChainRows& c, RowArgs& r) {
 // kernel body: first the sampling chunks (they wait for one another, so all must
 // be resident), then a workgroup per token for RoPE + cache and one for the rows,
 // then the activation's tiles.  No stage reads what another writes.
+// Only for a caller that has every stage's input before the call: in a model that
+// runs, a GEMM between the stages makes each from the one before, and its layer
+// calls the stages one by one.
 // Measured as called, against rows, RoPE + cache, activation and sampling as four
-// launches: T = 1 17.7 -> 8.2 us, T = 24 (Gemma norms) 25.6 -> 9.9, T = 1048 44.0 ->
-// 36.3, T = 6064 196.8 -> 181.9 (6.3 TB/s of what the step has to move).
+// launches: T = 1 17.7 -> 8.2 us (5.9 since the Python call is native), T = 24 (Gemma
+// norms) 25.6 -> 9.9 (9.2), T = 1048 44.0 -> 36.3 (36.1), T = 6064 196.8 -> 181.9
+// (181.4, 6.3 TB/s of what the step has to move).
 // ---------------------------------------------------------------------------
 struct ActArgs {
     const half_t *gate, *up;

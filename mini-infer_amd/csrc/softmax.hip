@@ -133,7 +133,7 @@ __global__ __launch_bounds__(G > 64 ? G : 256) void softmax_reg_kernel(const hal
     for (int j = 0; j < VPT; ++j) {
         const int64_t v = gl + j * G;
         const char* base = reinterpret_cast<const char*>(xr + static_cast<int64_t>(j) * G * 8);
-                a[j] = live && v < nv ? ld8_stream(reinterpret_cast<const half_t*>(base + lo))
+        a[j] = live && v < nv ? ld8_stream(reinterpret_cast<const half_t*>(base + lo))
                               : h8(-__builtin_huge_valf16());
     }
     if constexpr (RAGGED) {

@@ -20,11 +20,12 @@
 // R (a multiple of 8) apart, so one window shape serves all its rounds.
 // Against the 2-byte two-launch forms: [64, 151643] 32.1 -> 9.9 us (softmax),
 // 37.1 -> 11.0 (with the argmax); aligned [64, 152064] 9.0 / 10.2.
-// ONE (ragged rows only): every row in one round, so no next row's registers
-// and no conditions kept across rounds -- 44-68 VGPRs against 73-96 and, with
-// AM, spills: [64, 151643] softmax + argmax 14.2 -> 11.0 us, [200, 32001]
-// softmax 10.2 -> 8.2.  (For aligned rows, which have no such conditions, it
-// measured slower: [64, 152064] 9.0 -> 9.6 and 10.2 -> 11.1 us.)
+// ONE: every row in one round, so no next row's registers and no conditions
+// kept across rounds.  softmax_stream_kernel takes it for ragged rows, 44-68
+// VGPRs against 73-96 and, with AM, spills: [64, 151643] softmax + argmax 14.2 ->
+// 11.0 us, [200, 32001] softmax 10.2 -> 8.2; aligned rows, which have no such
+// conditions, measured slower with it there ([64, 152064] 9.0 -> 9.6 and 10.2 ->
+// 11.1 us).  The one-launch step, whose chunks are all resident, takes no other.
     constexpr int64_t kChunk = 2048 * U;
     constexpr int SW = AM ? 4 : 2;
     __shared__ float slots[256 / kWave];
